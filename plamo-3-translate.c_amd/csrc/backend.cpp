@@ -59,6 +59,11 @@ struct RopeTable {
     float *freq_dev = nullptr;
     float *table = nullptr;   // [rows][dim]: cos | sin
     uint64_t rows = 0;
+    // The same with FP64 angles, for rows past a sliding window (grown on
+    // demand): keys and queries of a prompt that overflows its window are
+    // rotated at their virtual rows, up to capacity + kMaxPrompt.
+    float *exact = nullptr;
+    uint64_t exact_rows = 0;
 };
 
 struct Layer {
@@ -147,7 +152,7 @@ struct plamo_metal {
     // Prompt / candidate workspace (grown on demand).
     uint64_t prompt_rows = 0;
     Buffer p_state, p_norm, p_qkv, p_q, p_attn, p_branch, p_gu, p_act, p_side_k, p_side_v,
-        p_ids, p_window, p_logits, p_attn_split;
+        p_ids, p_window, p_logits, p_attn_split, p_virtual;
     uint32_t *ids_host = nullptr;
     // Candidate results kept for commit.
     float *v_state = nullptr, *v_norm = nullptr, *v_logits = nullptr, *v_prop = nullptr;
@@ -401,6 +406,7 @@ void release_model(plamo_metal *m) {
     for (RopeTable &r : m->ropes) {
         dev_free(m, r.freq_dev);
         dev_free(m, r.table);
+        dev_free(m, r.exact);
     }
     m->layers.clear();
     m->ropes.clear();
@@ -433,6 +439,21 @@ int ensure_rope_rows(plamo_metal *m, RopeTable &r, uint64_t rows) {
     r.table = table;
     r.rows = target;
     ++m->epoch;
+    return 1;
+}
+
+int ensure_exact_rows(plamo_metal *m, RopeTable &r, uint64_t rows) {
+    if (rows <= r.exact_rows) return 1;
+    const uint64_t target = (rows + 1023) / 1024 * 1024;
+    float *table = dev_alloc<float>(m, target * r.dim);
+    if (!table) return 0;
+    float scale;
+    memcpy(&scale, &r.scale_bits, 4);
+    HIP_TRY(m, launch_rope_table(m->stream, r.freq_dev, scale, r.dim / 2, 0, target, table, true));
+    HIP_TRY(m, hipStreamSynchronize(m->stream));
+    dev_free(m, r.exact);
+    r.exact = table;
+    r.exact_rows = target;
     return 1;
 }
 
@@ -1438,17 +1459,25 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         m, T, std::max({h, m->max_attention, m->max_inter, gemm_swiglu_cols(h, m->max_inter)}));
     if (!ws) return -1;
     if (verify && !m->v_state && !alloc_verify(m, L, h, V)) return -1;
-    std::vector<char> overflow(L, 0);
-    uint64_t split_floats = 0;
+    // wide[i]: the rows overflow a sliding window and the matrix-core
+    // attention takes the layer, over keys rotated at their virtual rows.
+    std::vector<char> overflow(L, 0), wide(L, 0);
+    uint64_t split_floats = 0, virtual_floats = 0;
     for (uint64_t i = 0; i < L; ++i) {
         const Layer &d = m->layers[i];
         const struct cache *c = model->layers[i]->mixer->cache;
         const uint32_t window = c->count + T > c->capacity ? (uint32_t)c->capacity : 0;
+        wide[i] = window && prompt_attention_matrix(d.dim, d.qh, d.kh);
+        if (wide[i]) {
+            if (!ensure_exact_rows(m, m->ropes[d.rope], c->count + T)) return -1;
+            virtual_floats = std::max(virtual_floats, (c->count + T) * d.width);
+        }
         split_floats = std::max(split_floats,
                                 prompt_attention_scratch((uint32_t)c->count, (uint32_t)T, d.qh,
-                                                         d.kh, d.dim, window));
+                                                         d.kh, d.dim, window, wide[i]));
     }
     if (split_floats && !ensure(m, m->p_attn_split, split_floats * 4)) return -1;
+    if (virtual_floats && !ensure(m, m->p_virtual, virtual_floats * 4)) return -1;
     for (uint64_t i = 0; i < L; ++i) {
         Layer &d = m->layers[i];
         const struct cache *c = model->layers[i]->mixer->cache;
@@ -1555,6 +1584,12 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             qp.rows_from_count = 1;
             qp.rotate_k = 1;
         }
+        if (wide[i]) {
+            qp.virtual_table = rope.exact;
+            qp.k_virtual = as<float>(m->p_virtual);
+            HIP_FAIL(m, launch_rerotate(s, d.k, qp.k_virtual, rope.exact, c->count, d.kh, d.dim));
+            ++n;
+        }
         HIP_FAIL(m, launch_qkv_post(s, qp));
         ++n;
         // With states == NULL only the final row feeds the logits; the last
@@ -1574,8 +1609,8 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         // The O projection over every row reads the attention output as BF16
         // planes, written by the attention itself.
         const uint32_t o_tp =
-            !last_row_only && !overflow[i] &&
-                    prompt_attention_writes_planes(d.dim, d.qh, d.kh, 0)
+            !last_row_only && (!overflow[i] || wide[i]) &&
+                    prompt_attention_matrix(d.dim, d.qh, d.kh)
                 ? gemm_planes_rows(T, aw, ws)
                 : 0;
         pa.planes = o_tp ? planes : nullptr;
@@ -1586,6 +1621,11 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             pa.k_new = verify ? prop_k : as<float>(m->p_side_k);
             pa.v_new = verify ? prop_v : as<float>(m->p_side_v);
             pa.window = (uint32_t)d.capacity;
+            if (wide[i]) {
+                pa.rotated = 1;
+                pa.k_cache = as<float>(m->p_virtual);
+                pa.k_new = pa.k_cache + c->count * d.width;
+            }
         } else {
             pa.k_cache = d.rot;
             pa.v_cache = d.v;

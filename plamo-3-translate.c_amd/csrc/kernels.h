@@ -47,8 +47,11 @@ struct Prologue {
     uint32_t *status_out;
 };
 
+// Rows [first_row, first_row + rows) of a rotation table: cos | sin of
+// frequency times row, the product rounded to FP32 as the reference's
+// (src/rope_table.s:5-30), or kept in FP64 with `exact`.
 hipError_t launch_rope_table(hipStream_t, const float *freq, float scale, uint32_t half,
-                             uint64_t first_row, uint64_t rows, float *table);
+                             uint64_t first_row, uint64_t rows, float *table, bool exact = false);
 // Row gather widened from BF16: token t reads ids[t], or params->token when
 // ids is null. With `publish`, block 0 also copies *params (a pinned host
 // block, read over the bus) to *publish for the later kernels of the step.
@@ -168,6 +171,11 @@ struct QkvPost {
     int rows_from_count;
     int rotate_k;            // 0: leave k_rot alone (sliding overflow)
     float *stage;            // optional [3][width] copy of the last row (decode mirror)
+    // Optional: Q is rotated at its virtual row (count + t, past the window's
+    // capacity too) by this table instead, and the keys, rotated likewise, go
+    // to k_virtual[(count + t) * width].
+    const float *virtual_table;
+    float *k_virtual;
 };
 hipError_t launch_qkv_post(hipStream_t, const QkvPost &);
 
@@ -228,7 +236,9 @@ uint32_t decode_attention_splits(uint64_t rows);
 // General causal attention for `tokens` query rows. Key j of query t is the
 // virtual row j of [cache rows 0..prefix) ++ [new rows 0..tokens). With
 // window > 0 query t sees only the last `window` virtual rows ending at its
-// own row and keys are rotated on the fly at their window-local position.
+// own row; its keys are raw and rotated on the fly at their window-local
+// position, or `rotated` (keys and Q at their virtual rows) where
+// prompt_attention_matrix holds.
 struct PromptAttention {
     const float *q;          // [tokens, qh*dim] rotated Q
     const float *k_cache, *v_cache;  // rotated (or raw when window) cache rows
@@ -236,6 +246,7 @@ struct PromptAttention {
     const float *table;
     float *out;              // [tokens, qh*dim]
     uint32_t prefix, tokens, qh, kh, dim, window;
+    int rotated;
     // Optional scratch for key splits (prompt_attention_scratch floats): few
     // query tiles then spread their keys over several blocks and a merge.
     float *partial;
@@ -243,16 +254,17 @@ struct PromptAttention {
     // `padded`) instead of FP32 rows in `out`, so the O projection's GEMM
     // reads them with planes_ready. Rows past `tokens` are not written (each
     // GEMM output row depends on its own input row only, and rows past the
-    // token count are never stored). Only where
-    // prompt_attention_writes_planes holds.
+    // token count are never stored). Only where prompt_attention_matrix holds
+    // (and, with a window, the keys are rotated).
     uint16_t *planes;
     uint32_t padded;
 };
 hipError_t launch_prompt_attention(hipStream_t, const PromptAttention &);
-bool prompt_attention_writes_planes(uint32_t dim, uint32_t qh, uint32_t kh, uint32_t window);
+// Head dims and group sizes of the matrix-core form.
+bool prompt_attention_matrix(uint32_t dim, uint32_t qh, uint32_t kh);
 // Floats of split scratch launch_prompt_attention uses for this shape (0: none).
 uint64_t prompt_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t qh, uint32_t kh,
-                                  uint32_t dim, uint32_t window);
+                                  uint32_t dim, uint32_t window, int rotated);
 
 // Rotates cache rows [0, rows) of raw K into rotated K at their row position.
 hipError_t launch_rerotate(hipStream_t, const float *k_raw, float *k_rot, const float *table,

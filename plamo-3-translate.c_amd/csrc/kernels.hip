@@ -230,10 +230,12 @@ __device__ float block_inverse_from_partial(float s, uint32_t n, float *red) {
 // the cosine and sine of frequency j at `position`, times `scale`. The table
 // kernel and the decode attention (which rotates at the step's position
 // without a table lookup) share it, so both give the same bits.
+// EXACT: the angle is the FP64 product, not its FP32 rounding.
+template <bool EXACT = false>
 __device__ __forceinline__ void rope_cos_sin(float freq, float scale, float position, float &cs,
                                              float &sn) {
     float angle = freq * position;
-    double a = (double)angle;
+    double a = EXACT ? (double)freq * (double)position : (double)angle;
     const double two_pi = 6.283185307179586;
     double n = __builtin_rint(a / two_pi);
     double r = __builtin_fma(-n, two_pi, a);
@@ -262,6 +264,7 @@ __device__ __forceinline__ void rope_cos_sin(float freq, float scale, float posi
     sn = s * scale;
 }
 
+template <bool EXACT>
 __global__ __launch_bounds__(kThreads) void rope_table_kernel(const float *freq, float scale,
                                                               uint32_t half, uint64_t first_row,
                                                               uint64_t rows, float *table) {
@@ -270,15 +273,20 @@ __global__ __launch_bounds__(kThreads) void rope_table_kernel(const float *freq,
     uint64_t row = first_row + e / half;
     uint32_t j = (uint32_t)(e % half);
     float *out = table + row * 2 * half;
-    rope_cos_sin(freq[j], scale, (float)row, out[j], out[half + j]);
+    rope_cos_sin<EXACT>(freq[j], scale, (float)row, out[j], out[half + j]);
 }
 
 hipError_t launch_rope_table(hipStream_t stream, const float *freq, float scale, uint32_t half,
-                             uint64_t first_row, uint64_t rows, float *table) {
+                             uint64_t first_row, uint64_t rows, float *table, bool exact) {
     uint64_t n = rows * half;
     if (!n) return hipSuccess;
-    rope_table_kernel<<<(unsigned)((n + kThreads - 1) / kThreads), kThreads, 0, stream>>>(
-        freq, scale, half, first_row, rows, table);
+    const unsigned blocks = (unsigned)((n + kThreads - 1) / kThreads);
+    if (exact)
+        rope_table_kernel<true><<<blocks, kThreads, 0, stream>>>(freq, scale, half, first_row, rows,
+                                                                 table);
+    else
+        rope_table_kernel<false><<<blocks, kThreads, 0, stream>>>(freq, scale, half, first_row,
+                                                                  rows, table);
     return hipGetLastError();
 }
 
@@ -2524,7 +2532,8 @@ __global__ __launch_bounds__(64) void qkv_post_kernel(QkvPost a) {
     const uint32_t stride = (a.qh + 2 * a.kh) * dim;
     const float *x = a.qkv + (uint64_t)t * stride + (uint64_t)h * dim;
     const uint32_t count0 = a.params ? a.params->count[a.layer] : 0;
-    uint32_t position = count0 + t;
+    const uint32_t virtual_row = count0 + t;
+    uint32_t position = virtual_row;
     if (position > a.capacity - 1) position = a.capacity - 1;
     float s = 0.0f;
     for (uint32_t i = lane; i < dim; i += 64) {
@@ -2537,6 +2546,8 @@ __global__ __launch_bounds__(64) void qkv_post_kernel(QkvPost a) {
     float inv = 1.0f / __builtin_sqrtf(ms);
     const uint16_t *nw = h < a.qh ? a.qn : a.kn;
     const float *cs = a.table + (uint64_t)position * dim;
+    const float *vs = a.k_virtual ? a.virtual_table + (uint64_t)virtual_row * dim : nullptr;
+    if (vs && h < a.qh) cs = vs;
     const bool last = t + 1 == a.tokens;
     for (uint32_t j = lane; j < half; j += 64) {
         float sa = bf16f(nw[j]) + 1.0f, sb = bf16f(nw[j + half]) + 1.0f;
@@ -2564,6 +2575,13 @@ __global__ __launch_bounds__(64) void qkv_post_kernel(QkvPost a) {
             if (a.rotate_k) {
                 a.k_rot[o + j] = ra;
                 a.k_rot[o + j + half] = rb;
+            }
+            if (vs) {
+                const float vc = vs[j], vn = vs[half + j];
+                const float u0 = va * vc, u1 = vb * vn, u2 = vb * vc, u3 = va * vn;
+                float *kv_row = a.k_virtual + (uint64_t)virtual_row * width + (uint64_t)kv * dim;
+                kv_row[j] = u0 - u1;
+                kv_row[j + half] = u2 + u3;
             }
             if (a.stage && last) {
                 float *st = a.stage + (uint64_t)kv * dim;
@@ -3305,10 +3323,11 @@ hipError_t launch_decode_attention(hipStream_t stream, const DecodeAttention &a)
 
 // ---------------------------------------------------------------- prompt attention
 // Causal attention for a block of up to 16 queries of one head, online softmax
-// over key tiles of 32 rows. Without a window the keys are the materialized
-// rotated rows; with a window (sliding cache overflow) each key is rotated at
-// its position inside the query's window, as the CPU path does after every
-// shift (src/cache_rope.s:15-27 rotates all rows at local positions).
+// over key tiles of 32 rows, for head dims and group sizes the matrix-core
+// form does not take. Without a window the keys are the materialized rotated
+// rows; with a window (sliding cache overflow) each key is rotated at its
+// position inside the query's window, as the CPU path does after every shift
+// (src/cache_rope.s:15-27 rotates all rows at local positions).
 constexpr int kQT = 16, kKT = 32;
 __global__ __launch_bounds__(kThreads) void prompt_attention_kernel(PromptAttention a,
                                                                     uint32_t split_rows) {
@@ -3557,11 +3576,15 @@ static uint32_t prompt_attention_splits(uint32_t prefix, uint32_t tokens, uint32
 
 
 // ---------------------------------------------------------------- prompt attention on matrix cores
-// The same causal attention without a sliding window, with Q K^T and P V on
-// the FP32 matrix cores (v_mfma_f32_16x16x4_f32: FP32 operands, products and
-// sums in FP32; only the summation order differs from the scalar form, as
-// it already does there). Block: KV head blockIdx.x, query tokens
-// [16 * blockIdx.y, + 16), key split blockIdx.z; wave g is query head
+// The same causal attention, with Q K^T and P V on the FP32 matrix cores
+// (v_mfma_f32_16x16x4_f32: FP32 operands, products and sums in FP32; only the
+// summation order differs from the scalar form, as it already does there).
+// With a window the keys must be rotated at their virtual rows (and Q at its
+// own): a score depends on the distance of the two positions alone, so one
+// rotation per key serves every query, where rotating each key at its place
+// in each query's window costs more than the products (3500 tokens of 16
+// heads over a 2049-row window: 11.9 ms per layer in the scalar form). Block:
+// KV head blockIdx.x, 16 query tokens, key split blockIdx.z; wave g is query head
 // kvh * G + g, so the G heads of a group share every staged key and value
 // tile. Per tile of 32 keys a wave forms S = Q K^T for its 16 tokens (Q held
 // in registers as the A operand, K read from LDS as B), masks what the token
@@ -3590,7 +3613,8 @@ __global__ __launch_bounds__(64 * G) void prompt_attention_mfma_kernel(PromptAtt
     float *ps = vs + kMK * VS + wave * kMQ * PS;  // [kMQ][PS] of this wave
     const uint32_t kvh = blockIdx.x, h = kvh * G + wave;
     const uint32_t width = a.kh * DIM;
-    const uint32_t t0 = blockIdx.y * kMQ;
+    // The last query tiles see the most keys: they are dispatched first.
+    const uint32_t t0 = (gridDim.y - 1 - blockIdx.y) * kMQ;
     const uint32_t nq = a.tokens - t0 < (uint32_t)kMQ ? a.tokens - t0 : kMQ;
     const uint32_t col = lane & 15, grp = lane >> 4;
     // A operand of Q K^T: q[k4] = Q[token t0 + col][4 * k4 + grp] (token rows
@@ -3603,9 +3627,10 @@ __global__ __launch_bounds__(64 * G) void prompt_attention_mfma_kernel(PromptAtt
         for (int k4 = 0; k4 < DIM / 4; ++k4) q[k4] = qrow[4 * k4];
     }
     uint32_t hi_max = a.prefix + t0 + nq, lo_min = 0;
+    if (a.window && a.prefix + t0 + 1 > a.window) lo_min = a.prefix + t0 + 1 - a.window;
     if (split_rows) {
-        lo_min = blockIdx.z * split_rows;
-        hi_max = hi_max < lo_min + split_rows ? hi_max : lo_min + split_rows;
+        lo_min = max(lo_min, blockIdx.z * split_rows);
+        hi_max = min(hi_max, (blockIdx.z + 1) * split_rows);
     }
     const float scale = 1.0f / __builtin_sqrtf((float)DIM);
     const float ninf = -__builtin_inff();
@@ -3667,11 +3692,15 @@ __global__ __launch_bounds__(64 * G) void prompt_attention_mfma_kernel(PromptAtt
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const uint32_t row = 4 * grp + v;
-            const uint32_t visible = a.prefix + t0 + row + 1;  // keys of token t0 + row
+            // Keys of token t0 + row: [first, visible).
+            const uint32_t visible = a.prefix + t0 + row + 1;
+            const uint32_t first = a.window && visible > a.window ? visible - a.window : 0;
             const uint32_t r0 = k0 + col, r1 = k0 + 16 + col;
             const bool live = row < nq;
-            const float x0 = live && col < nk && r0 < visible ? s0[v] * scale : ninf;
-            const float x1 = live && 16 + col < nk && r1 < visible ? s1[v] * scale : ninf;
+            const float x0 =
+                live && col < nk && r0 < visible && r0 >= first ? s0[v] * scale : ninf;
+            const float x1 =
+                live && 16 + col < nk && r1 < visible && r1 >= first ? s1[v] * scale : ninf;
             const float m_new = fmaxf(m_run[v], row_max16(fmaxf(x0, x1)));
             const float p0 = m_new == ninf || x0 == ninf ? 0.0f : plamo_exp(x0 - m_new);
             const float p1 = m_new == ninf || x1 == ninf ? 0.0f : plamo_exp(x1 - m_new);
@@ -3732,8 +3761,8 @@ __global__ __launch_bounds__(64 * G) void prompt_attention_mfma_kernel(PromptAtt
     }
 }
 
-static bool prompt_mfma_supported(uint32_t dim, uint32_t qh, uint32_t kh, uint32_t window) {
-    if (window || !kh || qh % kh || (dim != 64 && dim != 128)) return false;
+bool prompt_attention_matrix(uint32_t dim, uint32_t qh, uint32_t kh) {
+    if (!kh || qh % kh || (dim != 64 && dim != 128)) return false;
     const uint32_t g = qh / kh;
     return g == 1 || g == 2 || g == 4 || g == 6 || g == 8 || g == 16;
 }
@@ -3782,29 +3811,31 @@ static hipError_t prompt_mfma_dim(hipStream_t stream, const PromptAttention &a, 
     }
 }
 
+// A window takes the matrix-core form when its keys are already rotated.
+static bool prompt_mfma_takes(uint32_t dim, uint32_t qh, uint32_t kh, uint32_t window,
+                              int rotated) {
+    return (!window || rotated) && prompt_attention_matrix(dim, qh, kh);
+}
+
 uint64_t prompt_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t qh, uint32_t kh,
-                                  uint32_t dim, uint32_t window) {
+                                  uint32_t dim, uint32_t window, int rotated) {
     uint32_t rows;
-    const uint32_t splits = prompt_mfma_supported(dim, qh, kh, window)
+    const uint32_t splits = prompt_mfma_takes(dim, qh, kh, window, rotated)
                                 ? prompt_mfma_splits(prefix, tokens, qh, kh, dim, &rows)
                                 : prompt_attention_splits(prefix, tokens, qh, dim, &rows);
     return splits > 1 ? (uint64_t)splits * tokens * qh * (dim + 2) : 0;
-}
-
-bool prompt_attention_writes_planes(uint32_t dim, uint32_t qh, uint32_t kh, uint32_t window) {
-    return prompt_mfma_supported(dim, qh, kh, window);
 }
 
 hipError_t launch_prompt_attention(hipStream_t stream, const PromptAttention &a) {
     if (!a.tokens) return hipSuccess;
     // Planes come from the matrix-core form only; the scalar form refuses
     // them rather than leave them unwritten.
-    if (a.planes && (!prompt_mfma_supported(a.dim, a.qh, a.kh, a.window) || a.padded < a.tokens ||
-                     (a.qh * a.dim) % (2 * kSplitBK)))
+    const bool matrix = prompt_mfma_takes(a.dim, a.qh, a.kh, a.window, a.rotated);
+    if (a.planes && (!matrix || a.padded < a.tokens || (a.qh * a.dim) % (2 * kSplitBK)))
         return hipErrorInvalidValue;
     uint32_t rows = 0, splits = 1;
     hipError_t e;
-    if (prompt_mfma_supported(a.dim, a.qh, a.kh, a.window)) {
+    if (matrix) {
         if (a.partial) splits = prompt_mfma_splits(a.prefix, a.tokens, a.qh, a.kh, a.dim, &rows);
         e = a.dim == 64 ? prompt_mfma_dim<64>(stream, a, splits, rows)
                         : prompt_mfma_dim<128>(stream, a, splits, rows);

@@ -322,3 +322,64 @@ def test_eager_decode_matches_graph(monkeypatch):
             assert np.array_equal(x, y)
     for x, y in zip(graph_kv, eager_kv):
         assert np.array_equal(x, y)
+
+
+# Prompts, decode steps and candidates past a sliding window at the head dims
+# and groups of the matrix-core prompt attention and the fused decode
+# attention: windows of less and more than a key tile (32) and an attention
+# block (64), prompts that start before, at and past the window's end, and a
+# window of which no prompt row sees the prefix.
+@pytest.mark.parametrize("qh,kh,dim,window,prefix,tokens", [
+    (8, 2, 128, 40, 0, 100), (8, 2, 128, 40, 12, 45), (4, 4, 64, 17, 18, 33),
+    (12, 2, 128, 32, 33, 2), (16, 1, 64, 300, 3, 700), (8, 4, 128, 64, 50, 17),
+    (16, 2, 64, 5, 6, 300),
+])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_past_the_window(qh, kh, dim, window, prefix, tokens, pinned):
+    say(f"past the window {qh}/{kh}x{dim} window={window} prefix={prefix} tokens={tokens}")
+    syn = plamo_hip.Synthetic(512, 2, qh, kh, dim, 768, 300, window=window, global_capacity=1200,
+                              pattern=2, embedding_std=1.0, seed=909)
+    gpu, cpu = syn.instance(pinned=pinned), syn.instance()
+    be = plamo_hip.Backend(syn)
+    try:
+        ids = [(j * 13 + 5) % 300 for j in range(prefix + tokens)]
+        for part in (ids[:prefix], ids[prefix:]):
+            if not part:
+                continue
+            actual = np.zeros((len(part), 512), np.float32)
+            expected = np.zeros((len(part), 512), np.float32)
+            assert be.prefill(gpu, part, actual) == 1
+            assert oracle_lib.prefill(cpu, part, expected)
+            gate(actual, expected, "all prompt states")
+            compare(gpu, cpu)
+        for token in (7, 11, 2, 290):
+            assert be.forward(gpu, token) == 1
+            assert oracle_lib.forward(cpu, token)
+            compare(gpu, cpu)
+        candidates = [9, 4, 250, 31, 8, 77, 6]
+        assert be.verify(gpu, candidates)[0] == 1
+        for i, token in enumerate(candidates[:5]):
+            assert oracle_lib.forward(cpu, token)
+            assert be.commit(gpu, i) == 1
+            compare(gpu, cpu)
+        # Past the slack rows a full window moves through (128 steps).
+        for step in range(135):
+            assert be.forward(gpu, step) == 1
+            assert oracle_lib.forward(cpu, step)
+        compare(gpu, cpu)
+        # A new request on the moved buffers.
+        gpu.reset()
+        cpu.reset()
+        assert be.prefill(gpu, ids[:9]) == 1
+        assert oracle_lib.prefill(cpu, ids[:9])
+        for token in (3, 5):
+            assert be.forward(gpu, token) == 1
+            assert oracle_lib.forward(cpu, token)
+            compare(gpu, cpu)
+        info = be.info()
+        assert info.errors == 0 and info.cpu_fallbacks == 0, info.note.decode()
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
