@@ -44,6 +44,9 @@ constexpr float kMlpOffset = 0.08944271909999159f;        // src/model.s:111
 // current row count still pass through the CU slots ahead of the
 // O-projection blocks of the same launch.
 constexpr uint64_t kInitialRows = 256;
+// Steps a full sliding window takes between two moves of its rows to the start
+// of their allocation (two copies of the window, once per kWindowSlack steps).
+constexpr uint64_t kWindowSlack = 128;
 constexpr uint64_t kMaxPrompt = 4096;                     // runtime/metal_model.m:540
 
 struct Range {
@@ -78,6 +81,12 @@ struct Layer {
     float *k = nullptr, *v = nullptr, *rot = nullptr;
     float *host_k = nullptr, *host_v = nullptr, *host_rot = nullptr;  // device views of pinned host rows
     uint64_t rows = 0;          // device rows allocated
+    // A full sliding window's K and V move on by one row per decode step:
+    // they are allocated with kWindowSlack rows more, k and v step through
+    // them (`moved` rows past the allocations) and return to the start once
+    // the slack is used up, so that a step copies no cached row.
+    float *k_base = nullptr, *v_base = nullptr;
+    uint64_t moved = 0;
     // Shadow of the host bookkeeping after this backend's last return: the
     // counters and a sample of the last K and V rows ([K sample | V sample]).
     bool synced = false;
@@ -399,8 +408,8 @@ void release_model(plamo_metal *m) {
         }
     for (Layer &l : m->layers) {
         dev_free(m, l.norms);
-        dev_free(m, l.k);
-        dev_free(m, l.v);
+        dev_free(m, l.k_base);
+        dev_free(m, l.v_base);
         dev_free(m, l.rot);
     }
     for (RopeTable &r : m->ropes) {
@@ -462,9 +471,16 @@ int ensure_kv_rows(plamo_metal *m, Layer &l, uint64_t rows) {
     uint64_t target = l.rows ? l.rows : kInitialRows;
     while (target < rows) target *= 2;
     if (target > l.capacity) target = l.capacity;
-    float *k = dev_alloc<float>(m, target * l.width), *v = dev_alloc<float>(m, target * l.width),
+    const uint64_t slack = l.sliding && target == l.capacity ? kWindowSlack : 0;
+    float *k = dev_alloc<float>(m, (target + slack) * l.width),
+          *v = dev_alloc<float>(m, (target + slack) * l.width),
           *rot = dev_alloc<float>(m, target * l.width);
-    if (!k || !v || !rot) return 0;
+    if (!k || !v || !rot) {
+        dev_free(m, k);
+        dev_free(m, v);
+        dev_free(m, rot);
+        return 0;
+    }
     if (l.rows) {
         // A pending prefix upload may still be writing the old rows.
         if (m->upload_pending) HIP_TRY(m, hipStreamWaitEvent(m->stream, m->upload_event, 0));
@@ -474,11 +490,12 @@ int ensure_kv_rows(plamo_metal *m, Layer &l, uint64_t rows) {
         HIP_TRY(m, hipMemcpyAsync(rot, l.rot, bytes, hipMemcpyDeviceToDevice, m->stream));
         HIP_TRY(m, hipStreamSynchronize(m->stream));
     }
-    dev_free(m, l.k);
-    dev_free(m, l.v);
+    dev_free(m, l.k_base);
+    dev_free(m, l.v_base);
     dev_free(m, l.rot);
-    l.k = k;
-    l.v = v;
+    l.k = l.k_base = k;
+    l.v = l.v_base = v;
+    l.moved = 0;
     l.rot = rot;
     l.rows = target;
     ++m->epoch;
@@ -873,6 +890,32 @@ struct DecodePlan {
     uint32_t row_cap = 0;
 };
 
+// Enqueues the move of a full sliding window to its next row: row r + 1 of the
+// old window is row r of the new one and its key is rotated at position r
+// (src/cache.s:8 with src/cache_rope.s:15-27), so that the step then appends
+// at row capacity - 1 as any other step appends at its count.
+int advance_window(plamo_metal *m, Layer &d, const RopeTable &rope) {
+    const uint64_t kept = d.capacity - 1;
+    if (d.moved < kWindowSlack) {
+        d.k += d.width;
+        d.v += d.width;
+        ++d.moved;
+    } else {
+        float *scratch = as<float>(m->p_window);
+        const uint64_t bytes = kept * d.width * 4;
+        for (auto [rows, base] : {std::pair{&d.k, d.k_base}, std::pair{&d.v, d.v_base}}) {
+            HIP_TRY(m, hipMemcpyAsync(scratch, *rows + d.width, bytes, hipMemcpyDeviceToDevice,
+                                      m->stream));
+            HIP_TRY(m, hipMemcpyAsync(base, scratch, bytes, hipMemcpyDeviceToDevice, m->stream));
+            *rows = base;
+        }
+        d.moved = 0;
+    }
+    ++m->epoch;  // captured graphs hold the old addresses
+    HIP_TRY(m, launch_rerotate(m->stream, d.k, d.rot, rope.table, kept, d.kh, d.dim));
+    return 1;
+}
+
 // Enqueues one decode step: embedding, every layer, final norm + head, and the
 // copy of logits/state/normalized/new KV rows to the pinned outbox.
 int encode_decode(plamo_metal *m, struct model *model, const DecodePlan &plan, int *dispatches) {
@@ -906,7 +949,11 @@ int encode_decode(plamo_metal *m, struct model *model, const DecodePlan &plan, i
         uint64_t qkv_rows = (uint64_t)(d.qh + 2 * d.kh) * d.dim;
         const bool shift = plan.shift[i], stale = plan.stale[i];
         float *layer_stage = stage + i * 3 * m->max_width;
-        // Attention over the materialized rotated rows (no sliding shift).
+        if (shift && d.fused) {
+            if (!advance_window(m, d, rope)) return 0;
+            ++n;
+        }
+        // Attention over the materialized rotated rows.
         auto attention_args = [&]() {
             DecodeAttention da{};
             da.qkv = m->qkv;
@@ -944,7 +991,7 @@ int encode_decode(plamo_metal *m, struct model *model, const DecodePlan &plan, i
             ++n;
         }
         bool fused_o = false;
-        if (!shift && d.fused) {
+        if (d.fused) {
             DecodeAttention da = attention_args();
             if (attention_o_supported(d.dim, d.qh / d.kh, (uint64_t)d.qh * d.dim) &&
                 !((uintptr_t)d.o & 15)) {
@@ -966,7 +1013,8 @@ int encode_decode(plamo_metal *m, struct model *model, const DecodePlan &plan, i
             }
             ++n;
         } else {
-            // General path (eager only: its arguments depend on the row count).
+            // General path (head dims and groups the fused attention does not
+            // cover; eager only: its arguments depend on the row count).
             const uint32_t count = m->params_host->count[i];
             QkvPost qp{};
             qp.qkv = m->qkv;
@@ -1334,7 +1382,8 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
         if (plan.shift[i] || plan.stale[i] || !d.fused) plan.special = true;
         uint64_t rows = std::min<uint64_t>(c->count + 1, c->capacity);
         if (!ensure_kv_rows(m, d, rows) || !ensure_rope_rows(m, m->ropes[d.rope], rows)) return -1;
-        m->params_host->count[i] = (uint32_t)c->count;
+        // A full window's step appends at its last row (advance_window).
+        m->params_host->count[i] = (uint32_t)(plan.shift[i] && d.fused ? c->count - 1 : c->count);
     }
     if (plan.special && (!ensure_prompt(m, model, 1) || !ensure_window_scratch(m, model))) return -1;
     m->params_host->token = (uint32_t)token;
