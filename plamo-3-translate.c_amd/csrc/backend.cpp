@@ -73,6 +73,10 @@ struct Layer {
     const uint16_t *qkv = nullptr, *o = nullptr, *gu = nullptr, *down = nullptr;
     uint16_t *norms = nullptr;  // device: pre | post | mlp_pre | mlp_post | qn | kn
     const uint16_t *pre, *post, *mlp_pre, *mlp_post, *qn, *kn;
+    // The projections as fp16 fragments (pair_ready), and the largest 2-norms
+    // of the gate and of the up rows.
+    PairWeight p_qkv{}, p_o{}, p_gu{}, p_down{};
+    uint32_t *gu_norms = nullptr;
     uint32_t qh = 0, kh = 0, dim = 0, hidden = 0, inter = 0, width = 0;
     uint64_t capacity = 0;
     bool sliding = false;
@@ -176,6 +180,13 @@ struct plamo_metal {
 
     Buffer lin_in, lin_out, mlp_state, mlp_norm, mlp_gu, mlp_act, mlp_branch, mlp_norms;
     GemmWorkspace gemm{};  // split-K partial tiles and arrival counters
+    // Fragments of every layer's projections for the prompt GEMM, one block
+    // laid out once per model, and the exponents of its input and activation
+    // rows. pair_tried: laid out, or the shapes or the memory do not allow it
+    // (prompts then take the BF16 weights).
+    char *pair_block = nullptr;
+    bool pair_ready = false, pair_tried = false;
+    int32_t *pair_exps = nullptr;
 
     hipGraphExec_t graph = nullptr;
     uint64_t epoch = 1, graph_epoch = 0;
@@ -419,6 +430,9 @@ void release_model(plamo_metal *m) {
     }
     m->layers.clear();
     m->ropes.clear();
+    dev_free(m, m->pair_block);
+    m->pair_block = nullptr;
+    m->pair_ready = m->pair_tried = false;
     dev_free(m, m->final_norm);
     m->final_norm = nullptr;
     m->model = nullptr;
@@ -734,7 +748,10 @@ int prepare(plamo_metal *m, struct model *model) {
     return 1;
 }
 
+int ensure_pair(plamo_metal *m, struct model *model);
+
 // Projections must already be resident (preloaded or mapped); a miss declines.
+// Once they are, the first call lays out their fp16 fragments.
 bool resolve_layers(plamo_metal *m, struct model *model) {
     uint64_t h = model->hidden;
     for (uint64_t i = 0; i < model->count; ++i) {
@@ -752,7 +769,78 @@ bool resolve_layers(plamo_metal *m, struct model *model) {
         }
     }
     if (!m->head) m->head = (const uint16_t *)resolve(m, model->head, model->vocab * h * 2);
-    return m->head != nullptr;
+    if (!m->head) return false;
+    (void)ensure_pair(m, model);
+    return true;
+}
+
+// Tokens from which a prompt or a candidate batch takes the fp16-pair GEMM (up
+// to five, the token GEMV streams the BF16 weights).
+constexpr uint64_t kPairTokens = 6;
+
+// Lays out the fp16 fragments of every layer (about as much memory as the
+// projections themselves, one pass over them). Without the memory, or with
+// shapes the fragments do not cover, prompts keep the BF16 weights.
+int ensure_pair(plamo_metal *m, struct model *model) {
+    if (m->pair_tried) return 1;
+    m->pair_tried = true;
+    const uint64_t h = model->hidden;
+    uint64_t bytes = 0;
+    auto take = [&](uint64_t n) {
+        const uint64_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
+    };
+    struct Place {
+        PairWeight *p;
+        const uint16_t *w;
+        uint64_t rows, cols, frag, exps;
+        bool gate_up;
+    };
+    std::vector<Place> places;
+    std::vector<uint64_t> norms;
+    for (Layer &d : m->layers) {
+        const uint64_t aw = (uint64_t)d.qh * d.dim;
+        // Norm rows and attention rows become planes in one launch each, of
+        // at most 8192 columns; gate and up rows pair up in groups of 32.
+        if (h % kPairK || h > 8192 || aw % kPairK || aw > 8192 || d.inter % kPairK) return 1;
+        places.push_back({&d.p_qkv, d.qkv, (uint64_t)(d.qh + 2 * d.kh) * d.dim, h, 0, 0, false});
+        places.push_back({&d.p_o, d.o, h, aw, 0, 0, false});
+        places.push_back({&d.p_gu, d.gu, 2 * (uint64_t)d.inter, h, 0, 0, true});
+        places.push_back({&d.p_down, d.down, h, d.inter, 0, 0, false});
+        norms.push_back(take(8));
+    }
+    for (Place &q : places) {
+        if (!pair_supported(q.rows, q.cols) || ((uintptr_t)q.w & 15)) return 1;
+        q.frag = take(pair_frag_elems(q.rows, q.cols) * 2);
+        q.exps = take(pair_exp_count(q.rows) * 4);
+    }
+    const uint64_t exps = take(2 * (kMaxPrompt + 128) * 4);
+    // Room for the KV caches and prompt buffers that grow later.
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || free_bytes < bytes + total / 16 ||
+        hipMalloc((void **)&m->pair_block, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        m->pair_block = nullptr;
+        return 1;
+    }
+    m->allocations.push_back(m->pair_block);
+    m->info.allocated_bytes += bytes;
+    m->pair_exps = (int32_t *)(m->pair_block + exps);
+    for (size_t i = 0; i < m->layers.size(); ++i) {
+        m->layers[i].gu_norms = (uint32_t *)(m->pair_block + norms[i]);
+        HIP_TRY(m, launch_fill(m->stream, m->layers[i].gu_norms, 2, 0));
+    }
+    for (size_t i = 0; i < places.size(); ++i) {
+        const Place &q = places[i];
+        *q.p = PairWeight{(uint16_t *)(m->pair_block + q.frag), (int32_t *)(m->pair_block + q.exps),
+                          (uint32_t)q.rows, (uint32_t)q.cols};
+        HIP_TRY(m, launch_pair_weights(m->stream, q.w, *q.p,
+                                       q.gate_up ? m->layers[i / 4].gu_norms : nullptr,
+                                       q.rows / 2));
+    }
+    m->pair_ready = true;
+    return 1;
 }
 
 // ---------------------------------------------------------------- host <-> device KV
@@ -1356,7 +1444,10 @@ int plamo_metal_warm_cache(struct plamo_metal *m) {
 
 int plamo_metal_prepare_model(struct plamo_metal *m, struct model *model) {
     if (m->config.memory == PLAMO_METAL_STREAM) return 1;
-    return prepare(m, model);
+    if (!prepare(m, model)) return 0;
+    // Weights preloaded later are laid out by the first call that finds them.
+    (void)resolve_layers(m, model);
+    return 1;
 }
 
 int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t token) {
@@ -1502,10 +1593,11 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     std::vector<char> stale;
     if (!sync_from_host(m, model, stale, !verify)) return -1;
     if (!ensure_prompt(m, model, T) || !ensure_window_scratch(m, model)) return -1;
-    // Planes room for the widest projection input, and for the gate/up
-    // GEMM's input and activation planes side by side.
+    const bool pair = T >= kPairTokens && m->pair_ready;
+    // Planes room for the widest projection input, and for the fp16 planes of
+    // the gate/up GEMM's input and output side by side.
     const GemmWorkspace *ws = gemm_workspace(
-        m, T, std::max({h, m->max_attention, m->max_inter, gemm_swiglu_cols(h, m->max_inter)}));
+        m, T, std::max({h, m->max_attention, m->max_inter, pair ? h + m->max_inter : 0}));
     if (!ws) return -1;
     if (verify && !m->v_state && !alloc_verify(m, L, h, V)) return -1;
     // wide[i]: the rows overflow a sliding window and the matrix-core
@@ -1554,12 +1646,15 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     // `normed` says the next layer's input norm is already in `norm`.
     const bool fuse_rows = h <= 8192;
     bool normed = false, final_normed = false;
-    // Prompts past 16 tokens take the matrix-core GEMM, which reads X as
-    // three BF16 planes: the norms that feed QKV and gate/up write them as
-    // they write their rows, so those projections skip their own split.
-    // qkv_planes: the planes of the next QKV input are already written.
-    uint16_t *const planes = ws->planes;
-    bool qkv_planes = false;
+    // With `pair` the norms that feed QKV and gate/up write the GEMM's input
+    // planes instead of FP32 rows, and gate/up writes down's.
+    PairRows in{};
+    if (pair) {
+        in.planes = ws->planes;
+        in.exps = m->pair_exps;
+        in.padded = pair_padded(T);
+    }
+    const PairRows *norm_pair = pair ? &in : nullptr;
     // Host-mirror copies of finished layers' cache rows not yet enqueued.
     struct MirrorRows {
         float *host;
@@ -1577,15 +1672,14 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         const RopeTable &rope = m->ropes[d.rope];
         const uint64_t qkv_w = (uint64_t)(d.qh + 2 * d.kh) * d.dim, aw = (uint64_t)d.qh * d.dim;
         if (!normed) {
-            const uint32_t tp = gemm_planes_rows(T, h, ws);
-            HIP_FAIL(m, launch_norm_rows(s, state, h, pre, 1.0f, norm, h, h, T, tp ? planes : nullptr,
-                                         tp));
-            qkv_planes = tp != 0;
+            HIP_FAIL(m, launch_norm_rows(s, state, h, pre, 1.0f, norm, h, h, T, norm_pair));
             ++n;
         }
         normed = false;
-        HIP_FAIL(m, launch_gemm(s, norm, h, d.qkv, qkv_w, h, T, qkv, qkv_w, ws, qkv_planes));
-        qkv_planes = false;
+        if (pair)
+            HIP_FAIL(m, launch_gemm_pair(s, in, d.p_qkv, T, qkv, qkv_w, *ws));
+        else
+            HIP_FAIL(m, launch_gemm(s, norm, h, d.qkv, qkv_w, h, T, qkv, qkv_w, ws));
         ++n;
         if (m->upload_pending) {  // cached rows are read from here on
             HIP_FAIL(m, hipStreamWaitEvent(s, m->upload_event, 0));
@@ -1655,15 +1749,6 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         pa.qh = d.qh;
         pa.kh = d.kh;
         pa.dim = d.dim;
-        // The O projection over every row reads the attention output as BF16
-        // planes, written by the attention itself.
-        const uint32_t o_tp =
-            !last_row_only && (!overflow[i] || wide[i]) &&
-                    prompt_attention_matrix(d.dim, d.qh, d.kh)
-                ? gemm_planes_rows(T, aw, ws)
-                : 0;
-        pa.planes = o_tp ? planes : nullptr;
-        pa.padded = o_tp;
         if (overflow[i]) {
             pa.k_cache = d.k;
             pa.v_cache = d.v;
@@ -1743,41 +1828,42 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             HIP_FAIL(m, launch_residual_rows(s, st, branch, mpost, kMlpOffset, h, 1));
             n += 5;
         } else {
-            HIP_FAIL(m, launch_gemm(s, attn + first * aw, aw, d.o, h, aw, rows, branch, h, ws,
-                                    o_tp != 0));
-            bool gu_planes = false;
-            if (fuse_rows) {
-                const uint32_t tp = gemm_planes_rows(rows, h, ws);
+            if (pair) {
+                // rows == T: `in` is sized for them. The attention rows become
+                // planes in a launch of their own (their scale is not known
+                // while the heads are computed); the rows' activation goes
+                // past the input planes, which gate/up's blocks still read.
+                PairRows act{};
+                act.planes = ws->planes + 2 * (uint64_t)in.padded * h;
+                act.exps = m->pair_exps + kMaxPrompt + 128;
+                act.padded = in.padded;
+                PairRows gu_in = in;
+                gu_in.norms = d.gu_norms;
+                gu_in.act_exps = act.exps;
+                HIP_FAIL(m, launch_norm_rows(s, attn, aw, nullptr, 0.0f, attn, aw, aw, T, &in));
+                HIP_FAIL(m, launch_gemm_pair(s, in, d.p_o, T, branch, h, *ws));
                 HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, post, kAttentionOffset, mpre,
-                                                     1.0f, norm, h, h, rows, tp ? planes : nullptr,
-                                                     tp));
-                gu_planes = tp != 0;
+                                                     1.0f, norm, h, h, T, &gu_in));
+                HIP_FAIL(m, launch_gemm_pair_swiglu(s, gu_in, d.p_gu, T, act, *ws));
+                HIP_FAIL(m, launch_gemm_pair(s, act, d.p_down, T, branch, h, *ws));
             } else {
-                HIP_FAIL(m, launch_residual_rows(s, st, branch, post, kAttentionOffset, h, rows));
-                HIP_FAIL(m, launch_norm_rows(s, st, h, mpre, 1.0f, norm, h, h, rows));
-                ++n;
+                HIP_FAIL(m, launch_gemm(s, attn + first * aw, aw, d.o, h, aw, rows, branch, h, ws));
+                if (fuse_rows) {
+                    HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, post, kAttentionOffset,
+                                                         mpre, 1.0f, norm, h, h, rows));
+                } else {
+                    HIP_FAIL(m, launch_residual_rows(s, st, branch, post, kAttentionOffset, h, rows));
+                    HIP_FAIL(m, launch_norm_rows(s, st, h, mpre, 1.0f, norm, h, h, rows));
+                    ++n;
+                }
+                HIP_FAIL(m, launch_gemm_swiglu(s, norm, h, d.gu, d.inter, h, rows, act, gu, ws));
+                HIP_FAIL(m, launch_gemm(s, act, d.inter, d.down, h, d.inter, rows, branch, h, ws));
             }
-            // The activation goes to down's GEMM as BF16 planes only, when
-            // that GEMM takes the matrix-core route.
-            const uint32_t act_planes = gemm_planes_rows(rows, d.inter, ws);
-            uint16_t *act_at = nullptr;
-            HIP_FAIL(m, launch_gemm_swiglu(s, norm, h, d.gu, d.inter, h, rows, act, gu, ws,
-                                          gu_planes, act_planes, &act_at));
-            // Down reads the activation planes where the gate/up launch put them.
-            GemmWorkspace down_ws = *ws;
-            if (act_planes) {
-                down_ws.planes = act_at;
-                down_ws.plane_elems = ws->plane_elems - (uint64_t)(act_at - ws->planes);
-            }
-            HIP_FAIL(m, launch_gemm(s, act, d.inter, d.down, h, d.inter, rows, branch, h,
-                                    &down_ws, act_planes != 0));
             if (fuse_rows && i + 1 < L) {
-                const uint32_t tp = gemm_planes_rows(rows, h, ws);
                 HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, mpost, kMlpOffset,
                                                      m->layers[i + 1].norms, 1.0f, norm, h, h,
-                                                     rows, tp ? planes : nullptr, tp));
+                                                     rows, norm_pair));
                 normed = true;
-                qkv_planes = tp != 0;
             } else if (fuse_rows && verify) {
                 HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, mpost, kMlpOffset,
                                                      m->final_norm, 1.0f, m->v_norm, h, h, rows));
@@ -1785,7 +1871,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             } else {
                 HIP_FAIL(m, launch_residual_rows(s, st, branch, mpost, kMlpOffset, h, rows));
             }
-            n += act_planes && act_at != ws->planes ? 5 : 6;  // the SwiGLU in gate/up's epilogue
+            n += 6;
         }
     }
     if (verify) {

@@ -85,13 +85,6 @@ struct GemmSplit {
     uint32_t *counters;
     uint16_t *planes;
     uint32_t xcd_group;  // nonzero: the M tiles of a weight tile share an XCD (see the kernel)
-    // Nonzero (the intermediate size I): the rows are a gate/up pair [2I]
-    // and each tile takes gate and up rows of the same intermediate columns;
-    // the epilogue writes silu(gate) * up as the BF16 planes `act` (rows
-    // padded to act_tp) instead of y.
-    uint32_t swiglu;
-    uint16_t *act;
-    uint32_t act_tp;
 };
 constexpr uint64_t kGemmPartialFloats = 16ull << 20;  // 64 MiB
 constexpr uint32_t kGemmCounters = 8192;
@@ -102,60 +95,73 @@ uint64_t gemm_plane_elems(uint64_t tokens, uint64_t cols);
 // the decode GEMV. Otherwise, with a workspace, more than one token and K a
 // multiple of 64: BF16 matrix cores on the exact three-term split of X; else
 // FP32 MFMA with BF16 weights widened in LDS.
-// planes_ready: the BF16 planes of X for the matrix-core path are already in
-// ws->planes (written by launch_norm_rows / launch_residual_norm_rows /
-// launch_swiglu_rows / launch_prompt_attention with gemm_planes_rows(tokens,
-// cols, ws) rows), and x is not read; other paths read x as usual.
 hipError_t launch_gemm(hipStream_t, const float *x, uint64_t x_stride, const uint16_t *w,
                        uint64_t rows, uint64_t cols, uint64_t tokens, float *y,
-                       uint64_t y_stride, const GemmWorkspace *ws, bool planes_ready = false);
-// The padded rows of the BF16 planes launch_gemm's matrix-core path reads for
-// `tokens` rows of `cols` columns, or 0 when another path takes the call.
-uint32_t gemm_planes_rows(uint64_t tokens, uint64_t cols, const GemmWorkspace *ws);
+                       uint64_t y_stride, const GemmWorkspace *ws);
+
+// A projection's weights as scaled fp16 fragments for launch_gemm_pair, and
+// each row's exponent (value = fragment * 2^-exps[row]); rows padded to 32.
+struct PairWeight {
+    uint16_t *frag;
+    int32_t *exps;
+    uint32_t rows, cols;
+};
+// Rows of X as scaled pairs of fp16 terms: [cols / 32][hi, lo][padded][32],
+// value = (hi + lo) * 2^-exps[row]. With act_exps (and norms, the largest
+// 2-norms of the gate and of the up rows as float bits), a norm also writes
+// the exponents of the rows' SwiGLU activation.
+constexpr uint32_t kPairK = 32;
+struct PairRows {
+    uint16_t *planes;
+    int32_t *exps;
+    uint32_t padded;
+    const uint32_t *norms;
+    int32_t *act_exps;
+};
+bool pair_supported(uint64_t rows, uint64_t cols);
+uint64_t pair_frag_elems(uint64_t rows, uint64_t cols);
+uint64_t pair_exp_count(uint64_t rows);
+// Rows of the planes for `tokens` rows (the consumer's tiles are whole).
+uint32_t pair_padded(uint64_t tokens);
+// Fills p.frag and p.exps from p.rows x p.cols BF16 weights (16-byte aligned);
+// norms (optional, zero before): the largest 2-norm of the rows below `half`
+// and of the others.
+hipError_t launch_pair_weights(hipStream_t, const uint16_t *w, const PairWeight &p,
+                               uint32_t *norms, uint64_t half);
+// y[t, r] = X W^T on the fp16 matrix cores, FP32 sums.
+hipError_t launch_gemm_pair(hipStream_t, const PairRows &x, const PairWeight &w, uint64_t tokens,
+                            float *y, uint64_t y_stride, const GemmWorkspace &ws);
+// silu(gate) * up of a gate | up projection into act.planes, scaled by
+// act.exps (written by the norm that formed x); w.rows / 2 a multiple of 32.
+hipError_t launch_gemm_pair_swiglu(hipStream_t, const PairRows &x, const PairWeight &w,
+                                   uint64_t tokens, const PairRows &act, const GemmWorkspace &ws);
 // Multi-row RMSNorm; with branch: state += rms(branch) * (bf16(w) + offset).
-// With planes, the normalized rows also go into the BF16 planes of
-// launch_gemm's matrix-core path, `padded` rows (gemm_planes_rows of the
-// consuming projection; rows past `rows` zero), so that projection can take
-// planes_ready.
+// With pair, the normalized rows go there instead of y, `pair->padded` rows
+// (those past `rows` zero; 16-byte-aligned rows of whole 32-column stages, at
+// most 8192 wide, hipErrorInvalidValue otherwise). Without w the rows are taken
+// as they are (pair only).
 hipError_t launch_norm_rows(hipStream_t, const float *x, uint64_t x_stride, const uint16_t *w,
                             float offset, float *y, uint64_t y_stride, uint64_t width,
-                            uint64_t rows, uint16_t *planes = nullptr, uint32_t padded = 0);
+                            uint64_t rows, const PairRows *pair = nullptr);
 // launch_residual_rows followed by launch_norm_rows of the updated rows into
-// norm, in one launch (width <= 8192; hipErrorInvalidValue otherwise), planes
-// as launch_norm_rows (16-byte-aligned rows only; hipErrorInvalidValue else).
+// norm, in one launch (width <= 8192; hipErrorInvalidValue otherwise), pair as
+// launch_norm_rows.
 hipError_t launch_residual_norm_rows(hipStream_t, float *state, const float *branch,
                                      const uint16_t *wr, float off_r, const uint16_t *wn,
                                      float off_n, float *norm, uint64_t norm_stride,
-                                     uint64_t width, uint64_t rows, uint16_t *planes = nullptr,
-                                     uint32_t padded = 0);
+                                     uint64_t width, uint64_t rows,
+                                     const PairRows *pair = nullptr);
 hipError_t launch_residual_rows(hipStream_t, float *state, const float *branch,
                                 const uint16_t *w, float offset, uint64_t width, uint64_t rows);
-// With planes, writes the activation as the BF16 planes of a following
-// launch_gemm over `padded` rows (gemm_planes_rows of the activation) instead
-// of `out`.
 hipError_t launch_swiglu_rows(hipStream_t, const float *gate_up, float *out,
-                              uint64_t intermediate, uint64_t rows, uint16_t *planes = nullptr,
-                              uint32_t padded = 0);
+                              uint64_t intermediate, uint64_t rows);
 // act[t, i] = silu(g) * u of the gate/up projection (rows i and
 // intermediate + i of w): the token GEMV writes act directly; other shapes
 // go through launch_gemm into gate_up ([tokens][2 * intermediate]) and
-// launch_swiglu_rows. act_planes (gemm_planes_rows(tokens, intermediate, ws),
-// nonzero) writes the activation only as BF16 planes, for a launch_gemm of
-// act with planes_ready over `ws` with its planes at *act_at: when the
-// workspace holds the input's planes and the activation's side by side, the
-// gate/up GEMM forms them in its epilogue (*act_at past the input's);
-// otherwise a separate SwiGLU launch writes them at ws->planes. Shapes
-// without either route fail.
+// launch_swiglu_rows.
 hipError_t launch_gemm_swiglu(hipStream_t, const float *x, uint64_t x_stride, const uint16_t *w,
                               uint64_t intermediate, uint64_t cols, uint64_t tokens, float *act,
-                              float *gate_up, const GemmWorkspace *ws, bool planes_ready = false,
-                              uint32_t act_planes = 0, uint16_t **act_at = nullptr);
-// The workspace columns a launch_gemm_swiglu over `cols` input columns needs
-// for its epilogue to write the activation planes (input and activation
-// planes side by side).
-inline uint64_t gemm_swiglu_cols(uint64_t cols, uint64_t intermediate) {
-    return cols + intermediate;
-}
+                              float *gate_up, const GemmWorkspace *ws);
 
 // Q/K head RMSNorm + RoPE + cache append for `tokens` rows of one layer.
 struct QkvPost {
@@ -250,14 +256,6 @@ struct PromptAttention {
     // Optional scratch for key splits (prompt_attention_scratch floats): few
     // query tiles then spread their keys over several blocks and a merge.
     float *partial;
-    // Optional: the output rows as launch_gemm's BF16 planes (rows padded to
-    // `padded`) instead of FP32 rows in `out`, so the O projection's GEMM
-    // reads them with planes_ready. Rows past `tokens` are not written (each
-    // GEMM output row depends on its own input row only, and rows past the
-    // token count are never stored). Only where prompt_attention_matrix holds
-    // (and, with a window, the keys are rotated).
-    uint16_t *planes;
-    uint32_t padded;
 };
 hipError_t launch_prompt_attention(hipStream_t, const PromptAttention &);
 // Head dims and group sizes of the matrix-core form.

@@ -1083,39 +1083,6 @@ __device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) {
 __device__ __forceinline__ uint32_t swizzle(uint32_t r, uint32_t q) {
     return q ^ ((r ^ (r >> 2)) & 3);
 }
-// Columns c .. c + 3 of row `row` into the BF16 planes of launch_gemm's
-// matrix-core path (the layout split_planes_kernel writes: [c / 32][plane]
-// [padded row][c % 32], the exact three-term split).
-__device__ __forceinline__ void write_planes4(uint16_t *planes, uint32_t padded, uint32_t row,
-                                              uint32_t c, f32x4 v) {
-    uint32_t h[4], md[4], lo[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        h[e] = __float_as_uint(v[e]) & 0xffff0000u;
-        const float r = v[e] - __uint_as_float(h[e]);
-        md[e] = __float_as_uint(r) & 0xffff0000u;
-        lo[e] = __float_as_uint(r - __uint_as_float(md[e]));
-    }
-    const uint64_t at = ((uint64_t)(c / kSplitBK) * 3 * padded + row) * kSplitBK + c % kSplitBK;
-    const uint64_t pl = (uint64_t)padded * kSplitBK;
-    *(u32x2 *)(planes + at) = u32x2{pack_hi16(h[0], h[1]), pack_hi16(h[2], h[3])};
-    *(u32x2 *)(planes + at + pl) = u32x2{pack_hi16(md[0], md[1]), pack_hi16(md[2], md[3])};
-    *(u32x2 *)(planes + at + 2 * pl) = u32x2{pack_hi16(lo[0], lo[1]), pack_hi16(lo[2], lo[3])};
-}
-// One column's value: the same three terms as write_planes4.
-__device__ __forceinline__ void write_planes1(uint16_t *planes, uint32_t padded, uint32_t row,
-                                              uint32_t c, float v) {
-    const uint32_t h = __float_as_uint(v) & 0xffff0000u;
-    const float r = v - __uint_as_float(h);
-    const uint32_t md = __float_as_uint(r) & 0xffff0000u;
-    const uint32_t lo = __float_as_uint(r - __uint_as_float(md));
-    const uint64_t at = ((uint64_t)(c / kSplitBK) * 3 * padded + row) * kSplitBK + c % kSplitBK;
-    const uint64_t pl = (uint64_t)padded * kSplitBK;
-    planes[at] = (uint16_t)(h >> 16);
-    planes[at + pl] = (uint16_t)(md >> 16);
-    planes[at + 2 * pl] = (uint16_t)(lo >> 16);
-}
-
 __global__ __launch_bounds__(256) void split_planes_kernel(const float *x, uint64_t ldx,
                                                            uint32_t rows, uint32_t padded,
                                                            uint32_t k, uint16_t *planes) {
@@ -1189,21 +1156,12 @@ __global__ __launch_bounds__(64 * GM * GN, (WN > 2 || GM * GN > 4) ? 1 : 2) void
         asrc[i] = g.planes + ((uint64_t)p * g.tp + m0 + r) * kSplitBK + 8 * q;
         adst[i] = R * 4 + swizzle(R, q);
     }
-    // With swiglu, tile row r of wave column wn and 32-row group j takes the
-    // gate (j even) or up (j odd) row of intermediate column
-    // bn BN/2 + wn 16 WN + (j / 2) 32 + r % 32: a lane's accumulators j and
-    // j + 1 then hold the gate and up sums of one column.
     const uint16_t *wsrc[WPT];
     uint32_t wdst[WPT];
 #pragma unroll
     for (int i = 0; i < WPT; ++i) {
         const uint32_t G = threadIdx.x + NT * i, r = G / 4, q = G % 4;
-        uint32_t row = min(n0 + r, g.n - 1);
-        if (g.swiglu) {
-            const uint32_t j = r / 32 % WN;
-            const uint32_t col = bn * (BN / 2) + r / (32 * WN) * (16 * WN) + j / 2 * 32 + r % 32;
-            row = (j & 1) ? g.swiglu + col : col;
-        }
+        const uint32_t row = min(n0 + r, g.n - 1);
         wsrc[i] = g.w + (uint64_t)row * g.k + 8 * q;
         wdst[i] = AG + r * 4 + swizzle(r, q);
     }
@@ -1378,25 +1336,6 @@ __global__ __launch_bounds__(64 * GM * GN, (WN > 2 || GM * GN > 4) ? 1 : 2) void
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[i][j][v] = sum[i][j][v];
     }
-    if (g.swiglu) {
-        // silu(gate) * up as in swiglu_planes_kernel (tests/activation_reference.s:99-126),
-        // written as the activation's BF16 planes; padding rows are not written.
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int j = 0; j < WN; j += 2) {
-                const uint32_t col = bn * (BN / 2) + wn * 16 * WN + j / 2 * 32 + (lane & 31);
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const uint32_t row =
-                        m0 + wm * 32 * WM + 32 * i + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
-                    const float gate = acc[i][j][v], up = acc[i][j + 1][v];
-                    const float d = plamo_exp(-gate) + 1.0f;
-                    if (row < g.t) write_planes1(g.act, g.act_tp, row, col, (gate / d) * up);
-                }
-            }
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -1412,10 +1351,9 @@ __global__ __launch_bounds__(64 * GM * GN, (WN > 2 || GM * GN > 4) ? 1 : 2) void
 }
 
 template <int WM, int WN, int GM = 2, int GN = 2, int PD = 3>
-static hipError_t gemm_split_variant(hipStream_t stream, GemmSplit g, const GemmWorkspace &ws,
-                                     bool planes_ready = false) {
+static hipError_t gemm_split_variant(hipStream_t stream, GemmSplit g, const GemmWorkspace &ws) {
     constexpr uint32_t BM = 32 * WM * GM, BN = 32 * WN * GN;
-    static_assert(BM == kSplitBM, "gemm_planes_rows pads the planes to kSplitBM rows");
+    static_assert(BM == kSplitBM, "gemm_split_192 counts tiles of kSplitBM rows");
     const uint32_t nt = (g.n + BN - 1) / BN, mt = (g.t + BM - 1) / BM;
     const uint32_t tiles = nt * mt, stages = g.k / kSplitBK;
     g.tp = mt * BM;
@@ -1440,9 +1378,8 @@ static hipError_t gemm_split_variant(hipStream_t stream, GemmSplit g, const Gemm
     // Grouping needs whole turns of the 8 XCDs: (weight tiles x splits) % 8 == 0.
     g.xcd_group = mt > 1 && (nt * splits) % 8 == 0;
     const uint64_t elems = (uint64_t)g.tp * g.k;
-    if (!planes_ready)
-        split_planes_kernel<<<(unsigned)((elems / 8 + 255) / 256), 256, 0, stream>>>(
-            g.x, g.ldx, g.t, g.tp, g.k, ws.planes);
+    split_planes_kernel<<<(unsigned)((elems / 8 + 255) / 256), 256, 0, stream>>>(
+        g.x, g.ldx, g.t, g.tp, g.k, ws.planes);
     const size_t lds = 3 * (size_t)(3 * BM * 4 + BN * 4) * sizeof(u32x4);
     static bool attr = false;
     if (!attr) {
@@ -2037,16 +1974,6 @@ uint64_t gemm_plane_elems(uint64_t tokens, uint64_t cols) {
     return 3 * ((tokens + 127) / 128 * 128) * cols;
 }
 
-uint32_t gemm_planes_rows(uint64_t tokens, uint64_t cols, const GemmWorkspace *ws) {
-    if (tokens <= kSkinnyTokens || tokens >= (1u << 31) || cols % (2 * kSplitBK) ||
-        cols > (1u << 30) || !ws || !ws->planes)
-        return 0;
-    const uint64_t tp = (tokens + kSplitBM - 1) / kSplitBM * kSplitBM;
-    return 3 * tp * cols <= ws->plane_elems && gemm_plane_elems(tokens, cols) <= ws->plane_elems
-               ? (uint32_t)tp
-               : 0;
-}
-
 // Wide tiles (256 weight rows per block, each wave 32 tokens x 128 rows)
 // except for short prompts' projections with few row tiles and K below 8192,
 // which take 128-row tiles (each wave 32 x 64) and get more blocks. Measured
@@ -2057,9 +1984,7 @@ uint32_t gemm_planes_rows(uint64_t tokens, uint64_t cols, const GemmWorkspace *w
 static bool gemm_split_wide(uint64_t rows, uint64_t cols, uint64_t tokens) {
     return tokens > 128 || cols >= 8192 || (rows + 255) / 256 >= 64;
 }
-// The matrix-core GEMM's tiling for g.n rows, g.t tokens (both tilings have
-// an even number of 32-row groups per wave, as a swiglu launch needs). Three
-// K stages in registers ahead of the LDS stages (2 and 4 measured within
+// Three K stages in registers ahead of the LDS stages (2 and 4 measured within
 // 1-4 % of it, either way, with three LDS buffers).
 // The weights are read with ordinary loads: each 64-byte stage of a row is
 // half a 128-byte cache line whose other half the next stage reads, and
@@ -2068,36 +1993,26 @@ static bool gemm_split_wide(uint64_t rows, uint64_t cols, uint64_t tokens) {
 // down 200.0 -> 187.5; at 116: QKV 40.6 -> 36.9, gate/up equal within the
 // spread between boxes).
 // Past 128 tokens, a projection whose 256-row tiles leave CUs idle takes
-// 192-row tiles when their count still fits one round of 256 blocks (not for
-// SwiGLU, whose gate/up pairing needs an even number of 32-row groups per
-// wave): C4 QKV at 443 tokens, 7 x 24 = 168 against 7 x 32 = 224 blocks,
-// 87.4-89.3 -> 81.7-85.7 us with planes ready.
+// 192-row tiles when their count still fits one round of 256 blocks: C4 QKV at
+// 443 tokens, 7 x 24 = 168 against 7 x 32 = 224 blocks, 87.4-89.3 -> 81.7-85.7 us
+// without the split launch.
 static bool gemm_split_192(const GemmSplit &g) {
-    if (g.swiglu || g.t <= 128 || g.n % 192) return false;
+    if (g.t <= 128 || g.n % 192) return false;
     const uint64_t mt = (g.t + kSplitBM - 1) / kSplitBM;
     const uint64_t b256 = mt * ((g.n + 255) / 256), b192 = mt * (g.n / 192);
     return b256 < 256 && b192 <= 256 && b192 > b256;
 }
-static hipError_t gemm_split_route(hipStream_t stream, const GemmSplit &g, const GemmWorkspace &ws,
-                                   bool planes_ready) {
-    if (gemm_split_192(g)) return gemm_split_variant<1, 3, 2, 2, 3>(stream, g, ws, planes_ready);
-    return gemm_split_wide(g.n, g.k, g.t)
-               ? gemm_split_variant<1, 4, 2, 2, 3>(stream, g, ws, planes_ready)
-               : gemm_split_variant<1, 2, 2, 2, 3>(stream, g, ws, planes_ready);
-}
-// Rows of one tile of the route above (the swiglu pairing needs the
-// intermediate size to be whole half tiles).
-static uint32_t gemm_split_tile_rows(uint64_t rows, uint64_t cols, uint64_t tokens) {
-    return gemm_split_wide(rows, cols, tokens) ? 256 : 128;
+static hipError_t gemm_split_route(hipStream_t stream, const GemmSplit &g,
+                                   const GemmWorkspace &ws) {
+    if (gemm_split_192(g)) return gemm_split_variant<1, 3, 2, 2, 3>(stream, g, ws);
+    return gemm_split_wide(g.n, g.k, g.t) ? gemm_split_variant<1, 4, 2, 2, 3>(stream, g, ws)
+                                          : gemm_split_variant<1, 2, 2, 2, 3>(stream, g, ws);
 }
 
 hipError_t launch_gemm(hipStream_t stream, const float *x, uint64_t x_stride, const uint16_t *w,
                        uint64_t rows, uint64_t cols, uint64_t tokens, float *y,
-                       uint64_t y_stride, const GemmWorkspace *ws, bool planes_ready) {
+                       uint64_t y_stride, const GemmWorkspace *ws) {
     if (!tokens || !rows) return hipSuccess;
-    // planes_ready callers may not have written x: only the matrix-core route
-    // below may take them.
-    if (planes_ready && tokens <= kSkinnyTokens) return hipErrorInvalidValue;
     {
         hipError_t e = launch_token_gemv(stream, x, x_stride, w, rows, cols, tokens, 0, y,
                                          y_stride, ws);
@@ -2129,9 +2044,8 @@ hipError_t launch_gemm(hipStream_t stream, const float *x, uint64_t x_stride, co
         g.t = (uint32_t)tokens;
         g.y = y;
         g.ldy = y_stride;
-        return gemm_split_route(stream, g, *ws, planes_ready);
+        return gemm_split_route(stream, g, *ws);
     }
-    if (planes_ready) return hipErrorInvalidValue;
     if (tokens <= 16) return gemm_variant<16, 64>(stream, x, x_stride, w, rows, cols, tokens, y, y_stride);
     return gemm_variant<64, 64>(stream, x, x_stride, w, rows, cols, tokens, y, y_stride);
 }
@@ -2139,50 +2053,545 @@ hipError_t launch_gemm(hipStream_t stream, const float *x, uint64_t x_stride, co
 hipError_t launch_gemm_swiglu(hipStream_t stream, const float *x, uint64_t x_stride,
                               const uint16_t *w, uint64_t intermediate, uint64_t cols,
                               uint64_t tokens, float *act, float *gate_up,
-                              const GemmWorkspace *ws, bool planes_ready, uint32_t act_planes,
-                              uint16_t **act_at) {
-    if (act_at) *act_at = ws ? ws->planes : nullptr;
+                              const GemmWorkspace *ws) {
     if (!tokens || !intermediate) return hipSuccess;
-    // Checked before anything is launched: a failure leaves the stream as it was.
-    if (act_planes && (!ws || !ws->planes || 3ull * act_planes * intermediate > ws->plane_elems ||
-                       act_planes < tokens || intermediate % (2 * kSplitBK) ||
-                       intermediate >= (1u << 30) || ((uintptr_t)gate_up & 15)))
-        return hipErrorInvalidValue;
-    // The gate/up GEMM writes the activation planes from its epilogue, past
-    // the input's planes (which its running blocks still read), when the
-    // workspace holds both: one launch less and no FP32 gate/up rows.
-    if (act_planes && act_at && tokens > kSkinnyTokens && tokens < (1u << 31) &&
-        2 * intermediate < (1u << 31) && gemm_split_supported(x, x_stride, w, cols) &&
-        intermediate % (gemm_split_tile_rows(2 * intermediate, cols, tokens) / 2) == 0 &&
-        gemm_planes_rows(tokens, cols, ws) == act_planes) {
-        const uint64_t in_elems = 3ull * act_planes * cols;
-        if (in_elems + 3ull * act_planes * intermediate <= ws->plane_elems) {
-            GemmSplit g{};
-            g.x = x;
-            g.ldx = x_stride;
-            g.w = w;
-            g.n = (uint32_t)(2 * intermediate);
-            g.k = (uint32_t)cols;
-            g.t = (uint32_t)tokens;
-            g.swiglu = (uint32_t)intermediate;
-            g.act = ws->planes + in_elems;
-            g.act_tp = act_planes;
-            *act_at = g.act;
-            return gemm_split_route(stream, g, *ws, planes_ready);
+    hipError_t e = launch_token_gemv(stream, x, x_stride, w, 2 * intermediate, cols, tokens,
+                                     intermediate, act, intermediate, ws);
+    if (e != hipErrorNotSupported) return e;
+    e = launch_gemm(stream, x, x_stride, w, 2 * intermediate, cols, tokens, gate_up,
+                    2 * intermediate, ws);
+    if (e != hipSuccess) return e;
+    return launch_swiglu_rows(stream, gate_up, act, intermediate, tokens);
+}
+
+// ---------------------------------------------------------------- fp16-pair MFMA GEMM
+// Prompt projections C[t, r] = sum_k X[t, k] * W[r, k] over resident weights
+// that have a copy in fp16 fragments (PairWeight). Each FP32 row of X is
+// scaled by a power of two (so that its largest value lies in [2^14, 2^15)) and
+// split into two fp16 terms, hi + lo, both rounded to nearest: 23 significant
+// bits, the smallest 2^-40 of the row's largest value. Each weight row is
+// scaled alike; its BF16 values are then exact in fp16 down to 2^-31 of the
+// row's largest and within 2^-40 of it below. The products are exact and
+// accumulate in FP32; the powers of two are taken out of the sums at the end.
+// Two products per weight instead of the three of the BF16 split: a third
+// fewer matrix-core instructions and FP32 additions. Measured against 64-bit
+// sums over the C4 projections (normal X, relative 2-norm): 1.8e-7 / 3.0e-7 /
+// 5.9e-7 for QKV at 116, 443 and 1900 tokens against 4.8e-7 / 7.0e-7 / 6.9e-7.
+//
+// What bounds it: the matrix cores at their power-limited clock (a library
+// product of 8192^3 random BF16 values sustains 1.2 PFLOP/s here; gate/up at
+// 1900 tokens issues 1.1), and the weight stream at short prompts. So the
+// loop moves as little as it can: X planes and weight fragments go straight
+// from global memory to LDS (no registers, no LDS writes), every fragment
+// read feeds 2 to 8 MFMAs, and the step's fragment reads, loads and MFMAs are
+// interleaved with one barrier per step.
+//
+// C4, us per launch, BF16 split -> this kernel (planes ready on both sides):
+//   tokens     QKV            O              gate/up          down
+//   37      17.5 -> 18.5   16.5 -> 17.1    62.5 -> 45.0     44.7 -> 33.3
+//   116     25.5 -> 25.6   21.4 -> 19.8   104.8 -> 71.7     58.3 -> 46.7
+//   443     66.4 -> 57.1   48.3 -> 38.9   375.5 -> 261.1   167.8 -> 118.6
+//   1900   285.1 -> 196.2 198.1 -> 118.2 1402.0 -> 946.7   691.8 -> 468.9
+//
+// Layouts. Planes: [K / 32][hi, lo][padded rows][32]; the loads permute the
+// 16-byte granules of a row (swizzle), so that a fragment's 32 rows spread
+// over the LDS banks. Weights: [K / 32][rows / 32][2][64 lanes][8], a fragment
+// of v_mfma_f32_32x32x16_f16 being 1 KB in lane order.
+// Block: GM x GN waves of WM x WN tiles of 32 x 32; S stages of 32 columns in
+// a ring of LDS buffers, S - 1 loaded ahead. Step j computes stage j, reads
+// its second half's fragments and the first half's of stage j + 1, and
+// issues the loads of stage j + S - 1 into the buffer that step j - 1 read.
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+// The power of two that brings values up to `bits` (a float's magnitude) into
+// [2^14, 2^15); rows of zeros and non-finite rows get the extreme exponents.
+__device__ __forceinline__ int pair_exponent(uint32_t bits) {
+    const int e = (int)(bits >> 23 & 255u);
+    return min(14 - ((e < 1 ? 1 : e > 254 ? 254 : e) - 127), 126);
+}
+__device__ __forceinline__ float power_of_two(int e) { return __int_as_float((e + 127) << 23); }
+// hi + lo of x * scale: hi the product rounded to fp16, lo the rest (exact in
+// the fused multiply-add) rounded to fp16.
+__device__ __forceinline__ void pair_split(float x, float scale, _Float16 &hi, _Float16 &lo) {
+    hi = (_Float16)(x * scale);
+    lo = (_Float16)__builtin_fmaf(x, scale, -(float)hi);
+}
+__device__ __forceinline__ uint64_t pair_at(uint32_t padded, uint32_t row, uint32_t c) {
+    return ((uint64_t)(c / kPairK) * 2 * padded + row) * kPairK + c % kPairK;
+}
+
+// Padding rows of the planes, for a 256-thread block.
+__device__ __forceinline__ void pair_zero_row(const PairRows &p, uint32_t row, uint32_t width) {
+    for (uint32_t c = threadIdx.x * 4; c < width; c += 4 * kThreads) {
+        const uint64_t at = pair_at(p.padded, row, c);
+        *(u32x2 *)(p.planes + at) = u32x2{0u, 0u};
+        *(u32x2 *)(p.planes + at + (uint64_t)p.padded * kPairK) = u32x2{0u, 0u};
+    }
+    if (threadIdx.x == 0) {
+        p.exps[row] = 0;
+        if (p.act_exps) p.act_exps[row] = 0;
+    }
+}
+
+// One row held by a 256-thread block (thread i: elements 4 (i + 256 j) .. + 3,
+// zero past the row) into the planes. With act_exps also the exponent of the
+// row's SwiGLU activation, from |silu(g) u| <= |g| |u| and Cauchy-Schwarz:
+// the row's 2-norm squared times the largest 2-norms of the gate and the up
+// rows (norms) is an upper bound that needs no pass over the activation. It
+// exceeds the typical value by about the row's length; the pair still
+// resolves 2^-40 of it.
+template <int NV>
+__device__ __forceinline__ void pair_row(const PairRows &p, uint32_t row, uint32_t groups,
+                                         const f32x4 (&v)[NV], float *red) {
+    float mx = 0.0f, ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            mx = fmaxf(mx, __builtin_fabsf(v[j][e]));
+            ss = __builtin_fmaf(v[j][e], v[j][e], ss);
+        }
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    __syncthreads();
+    const int ex = pair_exponent(__float_as_uint(mx));
+    const float scale = power_of_two(ex);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const uint32_t i = threadIdx.x + kThreads * j;
+        if (i >= groups) continue;
+        f16x4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            _Float16 h, l;
+            pair_split(v[j][e], scale, h, l);
+            hi[e] = h;
+            lo[e] = l;
+        }
+        const uint64_t at = pair_at(p.padded, row, 4 * i);
+        *(u32x2 *)(p.planes + at) = __builtin_bit_cast(u32x2, hi);
+        *(u32x2 *)(p.planes + at + (uint64_t)p.padded * kPairK) = __builtin_bit_cast(u32x2, lo);
+    }
+    if (p.act_exps) {
+        ss = wave_sum(ss);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        ss = (red[0] + red[1]) + (red[2] + red[3]);
+    }
+    if (threadIdx.x == 0) {
+        p.exps[row] = ex;
+        if (p.act_exps) {
+            const float bound = __uint_as_float(p.norms[0]) * __uint_as_float(p.norms[1]) * ss;
+            p.act_exps[row] = pair_exponent(__float_as_uint(bound));
         }
     }
-    // The token GEMV reads x and writes act as FP32 only: it takes neither
-    // input planes in place of x nor planes for the output.
-    if (!planes_ready && !act_planes) {
-        hipError_t e = launch_token_gemv(stream, x, x_stride, w, 2 * intermediate, cols, tokens,
-                                         intermediate, act, intermediate, ws);
-        if (e != hipErrorNotSupported) return e;
+}
+
+// Block: 32 weight rows. Rows past `rows` (the last group's padding) are zero.
+// norms[0] (rows below `half`) and norms[1]: the largest 2-norm of a row, as
+// float bits.
+__global__ __launch_bounds__(kThreads) void pair_weights_kernel(const uint16_t *w, uint32_t rows,
+                                                                uint32_t cols, uint16_t *frag,
+                                                                int32_t *exps, uint32_t *norms,
+                                                                uint32_t half) {
+    __shared__ float scales[32];
+    const uint32_t r0 = blockIdx.x * 32, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (uint32_t r = wave; r < 32; r += 4) {
+        const uint32_t row = r0 + r;
+        float mx = 0.0f, ss = 0.0f;
+        if (row < rows)
+            for (uint32_t c = lane * 8; c < cols; c += 512) {
+                const u32x4 q = *(const u32x4 *)(w + (uint64_t)row * cols + c);
+                const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float a = bf16f(u[e] & 0xffffu), b = __uint_as_float(u[e] & 0xffff0000u);
+                    mx = fmaxf(mx, fmaxf(__builtin_fabsf(a), __builtin_fabsf(b)));
+                    ss = __builtin_fmaf(a, a, __builtin_fmaf(b, b, ss));
+                }
+            }
+        mx = wave_max(mx);
+        ss = wave_sum(ss);
+        if (lane == 0) {
+            const int ex = pair_exponent(__float_as_uint(mx));
+            exps[r0 + r] = ex;
+            scales[r] = power_of_two(ex);
+            if (norms && row < rows)
+                (void)__hip_atomic_fetch_max(norms + (row < half ? 0 : 1),
+                                             __float_as_uint(__builtin_sqrtf(ss)),
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
-    hipError_t e = launch_gemm(stream, x, x_stride, w, 2 * intermediate, cols, tokens, gate_up,
-                               2 * intermediate, ws, planes_ready);
-    if (e != hipSuccess) return e;
-    return launch_swiglu_rows(stream, gate_up, act, intermediate, tokens,
-                              act_planes ? ws->planes : nullptr, act_planes);
+    __syncthreads();
+    const uint32_t row = r0 + (lane & 31);
+    const float scale = scales[lane & 31];
+    for (uint32_t f = wave; f < cols / 16; f += 4) {
+        u32x4 q = {0u, 0u, 0u, 0u};
+        if (row < rows) q = *(const u32x4 *)(w + (uint64_t)row * cols + 16 * f + 8 * (lane >> 5));
+        const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+        f16x8 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[2 * e] = (_Float16)(bf16f(u[e] & 0xffffu) * scale);
+            o[2 * e + 1] = (_Float16)(__uint_as_float(u[e] & 0xffff0000u) * scale);
+        }
+        const uint64_t at = (((uint64_t)(f / 2) * gridDim.x + blockIdx.x) * 2 + f % 2) * 512;
+        *(f16x8 *)(frag + at + lane * 8) = o;
+    }
+}
+
+bool pair_supported(uint64_t rows, uint64_t cols) {
+    return rows && cols && cols % kPairK == 0 && rows < (1u << 30) && cols < (1u << 30);
+}
+uint64_t pair_frag_elems(uint64_t rows, uint64_t cols) { return (rows + 31) / 32 * 32 * cols; }
+uint64_t pair_exp_count(uint64_t rows) { return (rows + 31) / 32 * 32; }
+
+hipError_t launch_pair_weights(hipStream_t stream, const uint16_t *w, const PairWeight &p,
+                               uint32_t *norms, uint64_t half) {
+    if (!pair_supported(p.rows, p.cols) || ((uintptr_t)w & 15)) return hipErrorInvalidValue;
+    pair_weights_kernel<<<(p.rows + 31) / 32, kThreads, 0, stream>>>(w, p.rows, p.cols, p.frag,
+                                                                     p.exps, norms, (uint32_t)half);
+    return hipGetLastError();
+}
+
+// Waits until all but the wave's YOUNGER youngest loads have landed, then for
+// every wave of the block (__syncthreads would wait for all loads to LDS).
+template <int YOUNGER>
+__device__ __forceinline__ void loads_landed() {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(YOUNGER) : "memory");
+}
+
+struct GemmPair {
+    const uint16_t *planes;
+    const int32_t *row_exps;
+    uint32_t padded;
+    PairWeight w;
+    uint32_t t, splits, xcd_group;
+    float *y;
+    uint64_t ldy;
+    float *partial;
+    uint32_t *counters;
+    // Nonzero (the intermediate size I, whole groups of 32): the weight rows
+    // are gate | up, a wave's even tiles take gate rows and its odd tiles the
+    // up rows of the same columns, and silu(gate) * up goes to `act` as planes
+    // scaled by act_exps.
+    uint32_t swiglu;
+    uint16_t *act;
+    const int32_t *act_exps;
+};
+
+// SUMS accumulators per tile (1, or 4: hi and lo terms and the two halves of a
+// stage apart, which shortens each FP32 chain by four).
+template <int WM, int WN, int GM, int GN, int S, int OCC, int SUMS>
+__global__ __launch_bounds__(64 * GM * GN, OCC) void gemm_pair_kernel(GemmPair g) {
+    constexpr int NW = GM * GN, BM = 32 * WM * GM, BN = 32 * WN * GN;
+    // 1 KB loads per stage: X (two planes of BM rows of 64 bytes), then W.
+    constexpr int AI = BM / 8, WI = BN / 16, PW = (AI + WI) / NW;
+    static_assert((AI + WI) % NW == 0 && S >= 3, "whole loads per wave; two stages visible");
+    constexpr uint32_t SG = (AI + WI) * 64;  // 16-byte granules per stage
+    extern __shared__ u32x4 lds[];           // [S][SG]
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wm = wave / GN, wn = wave % GN;
+    // The M tiles of one (weight tile, K split) take consecutive turns on one
+    // XCD, as in gemm_split_kernel.
+    uint32_t bn = blockIdx.x, bm = blockIdx.y, bz = blockIdx.z;
+    if (g.xcd_group) {
+        const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        const uint32_t slot = lin / 8, group = slot / gridDim.y * 8 + lin % 8;
+        bm = slot % gridDim.y;
+        bn = group % gridDim.x;
+        bz = group / gridDim.x;
+    }
+    const uint32_t m0 = bm * BM;
+    const uint32_t nst = g.w.cols / kPairK / g.splits, s0 = bz * nst;
+    const uint32_t groups = (g.w.rows + 31) / 32, half = g.swiglu / 32;
+    // Weight row group of tile j of wave column c.
+    auto row_group = [&](uint32_t c, uint32_t j) -> uint32_t {
+        if (g.swiglu)
+            return (j & 1 ? half : 0) + min(bn * (BN / 64) + c * (WN / 2) + j / 2, half - 1);
+        return min(bn * (BN / 32) + c * WN + j, groups - 1);
+    };
+    const char *src[PW];
+    uint32_t advance[PW];  // bytes per stage
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+        const uint32_t L = wave + NW * i;
+        if (L < AI) {
+            const uint32_t p = L / (BM / 16), r = L % (BM / 16) * 16 + lane / 4;
+            src[i] = (const char *)(g.planes + ((uint64_t)(2 * s0 + p) * g.padded + m0 + r) * kPairK +
+                                    8 * swizzle(r, lane & 3));
+            advance[i] = 4 * kPairK * g.padded;
+        } else {
+            const uint32_t f = L - AI;
+            src[i] = (const char *)(g.w.frag + ((uint64_t)s0 * groups + row_group(f / 2 / WN, f / 2 % WN)) * 1024 +
+                                    (f & 1) * 512 + lane * 8);
+            advance[i] = groups * 2048;
+        }
+    }
+    // Loads past the last stage repeat it into buffers no later step reads.
+    auto load = [&](uint32_t stage, uint32_t buf) {
+        const uint32_t st = min(stage, nst - 1);
+#pragma unroll
+        for (int i = 0; i < PW; ++i)
+            __builtin_amdgcn_global_load_lds(
+                (const void *)(src[i] + (uint64_t)st * advance[i]),
+                (__attribute__((address_space(3))) void *)(lds + buf * SG + (wave + NW * i) * 64),
+                16, 0, 0);
+    };
+    auto frag = [&](uint32_t buf, int ks, f16x8 (&a)[2][WM], f16x8 (&b)[WN]) {
+        const u32x4 *st = lds + buf * SG;
+        const uint32_t q = 2 * ks + (lane >> 5);
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const uint32_t r = (wm * WM + i) * 32 + (lane & 31);
+                a[p][i] = __builtin_bit_cast(f16x8, st[p * BM * 4 + r * 4 + swizzle(r, q)]);
+            }
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+            b[j] = __builtin_bit_cast(f16x8, st[AI * 64 + ((wn * WN + j) * 2 + ks) * 64 + lane]);
+    };
+    f32x16 sums[SUMS][WM][WN];
+#pragma unroll
+    for (int n = 0; n < SUMS; ++n)
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sums[n][i][j][v] = 0.0f;
+    auto mfma = [&](int ks, const f16x8 (&a)[2][WM], const f16x8 (&b)[WN]) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) {
+                    f32x16 &c = sums[SUMS == 4 ? 2 * p + ks : 0][i][j];
+                    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[p][i], b[j], c, 0, 0, 0);
+                }
+    };
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) load(s, s);
+    loads_landed<PW * (S - 3)>();
+    f16x8 a0[2][WM], a1[2][WM], b0[WN], b1[WN];
+    frag(0, 0, a0, b0);
+    uint32_t cur = 0, fill = S - 1;
+    for (uint32_t j = 0; j < nst; ++j) {
+        const uint32_t nxt = cur + 1 == S ? 0 : cur + 1;
+        frag(cur, 1, a1, b1);
+        load(j + S - 1, fill);
+        mfma(0, a0, b0);
+        frag(nxt, 0, a0, b0);
+        mfma(1, a1, b1);
+        // Issue order: an MFMA before each fragment read and each load.
+        constexpr int NF = 2 * WM + WN, NM = 4 * WM * WN;
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+        }
+#pragma unroll
+        for (int i = 0; i < PW; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // load
+        }
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        if constexpr (NM > 2 * NF + PW)
+            __builtin_amdgcn_sched_group_barrier(0x008, NM - 2 * NF - PW, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        loads_landed<PW * (S - 3)>();
+        __builtin_amdgcn_sched_barrier(0);
+        cur = nxt;
+        fill = fill + 1 == S ? 0 : fill + 1;
+    }
+    // No load may still write LDS when it is reused or the block ends.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    f32x16 (&acc)[WM][WN] = sums[0];
+    if constexpr (SUMS == 4)
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    acc[i][j][v] = (sums[2][i][j][v] + sums[3][i][j][v]) +
+                                   (sums[0][i][j][v] + sums[1][i][j][v]);
+
+    if (g.splits > 1) {
+        // Partial tiles as in gemm_split_kernel, summed in split order.
+        const uint32_t tile = bm * gridDim.x + bn, tiles = gridDim.x * gridDim.y;
+        float *part = g.partial + ((uint64_t)bz * tiles + tile) * (BM * BN);
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    store_through(part + (((wave * WM + i) * WN + j) * 16 + v) * 64 + lane,
+                                  acc[i][j][v]);
+        if (!arrive_last(&g.counters[tile], g.splits, (int *)lds)) return;
+        const float *base = g.partial + (uint64_t)tile * (BM * BN) + wave * WM * WN * 1024 + lane;
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    acc[i][j][v] = load_through(base + ((i * WN + j) * 16 + v) * 64);
+        for (uint32_t sp = 1; sp < g.splits; ++sp) {
+            const float *ps = base + (uint64_t)sp * tiles * (BM * BN);
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v)
+                        acc[i][j][v] = acc[i][j][v] + load_through(ps + ((i * WN + j) * 16 + v) * 64);
+        }
+    }
+    // D layout of v_mfma_f32_32x32x16: value v of lane l is row
+    // 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32 of the 32 x 32 tile.
+    int we[WN];
+#pragma unroll
+    for (int j = 0; j < WN; ++j) we[j] = g.w.exps[row_group(wn, j) * 32 + (lane & 31)];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const uint32_t row = m0 + (wm * WM + i) * 32 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
+            if (row >= g.padded) continue;
+            const int xe = g.row_exps[row];
+            if (WN % 2 == 0 && g.swiglu) {
+                const float scale = power_of_two(g.act_exps[row]);
+#pragma unroll
+                for (int j = 0; j + 1 < WN; j += 2) {
+                    const uint32_t c = bn * (BN / 64) + wn * (WN / 2) + j / 2;
+                    if (c >= half) continue;
+                    // silu(gate) * up (tests/activation_reference.s:99-126).
+                    const float gate = __builtin_ldexpf(acc[i][j][v], -(xe + we[j]));
+                    const float up = __builtin_ldexpf(acc[i][j + 1][v], -(xe + we[j + 1]));
+                    const float d = plamo_exp(-gate) + 1.0f;
+                    _Float16 hi, lo;
+                    pair_split((gate / d) * up, scale, hi, lo);
+                    const uint64_t at = pair_at(g.padded, row, c * 32 + (lane & 31));
+                    g.act[at] = __builtin_bit_cast(uint16_t, hi);
+                    g.act[at + (uint64_t)g.padded * kPairK] = __builtin_bit_cast(uint16_t, lo);
+                }
+            } else if (row < g.t) {
+#pragma unroll
+                for (int j = 0; j < WN; ++j) {
+                    const uint32_t col = (bn * (BN / 32) + wn * WN + j) * 32 + (lane & 31);
+                    if (col < g.w.rows)
+                        g.y[(uint64_t)row * g.ldy + col] =
+                            __builtin_ldexpf(acc[i][j][v], -(xe + we[j]));
+                }
+            }
+        }
+}
+
+// K splits double while the blocks stay within `most` and a split keeps four
+// stages, within the workspace.
+template <int WM, int WN, int GM, int GN, int S, int OCC, int SUMS = 1>
+static hipError_t gemm_pair_variant(hipStream_t stream, GemmPair g, const GemmWorkspace &ws,
+                                    uint32_t most) {
+    constexpr uint32_t BM = 32 * WM * GM, BN = 32 * WN * GN;
+    const uint32_t nt = (g.w.rows + BN - 1) / BN, mt = (g.t + BM - 1) / BM;
+    const uint32_t tiles = nt * mt, stages = g.w.cols / kPairK;
+    if (mt * BM > g.padded || mt > 65535) return hipErrorInvalidValue;
+    uint32_t splits = 1;
+    while (tiles * splits * 2 <= most && stages % (2 * splits) == 0 &&
+           stages / (2 * splits) >= 4 && splits < 8 && tiles <= ws.counters &&
+           2ull * splits * tiles * BM * BN <= ws.partial_floats)
+        splits *= 2;
+    g.splits = splits;
+    g.partial = ws.partial;
+    g.counters = ws.counter_base;
+    g.xcd_group = mt > 1 && (nt * splits) % 8 == 0;
+    constexpr size_t lds = (size_t)S * (BM / 8 + BN / 16) * 1024;
+    static bool attr = false;
+    if (!attr) {
+        hipError_t e = hipFuncSetAttribute((const void *)gemm_pair_kernel<WM, WN, GM, GN, S, OCC, SUMS>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    gemm_pair_kernel<WM, WN, GM, GN, S, OCC, SUMS>
+        <<<dim3(nt, mt, splits), 64 * GM * GN, lds, stream>>>(g);
+    return hipGetLastError();
+}
+
+uint32_t pair_padded(uint64_t tokens) {
+    const uint64_t unit = tokens <= 32 ? 32 : tokens <= 64 ? 64 : 128;
+    return (uint32_t)((tokens + unit - 1) / unit * unit);
+}
+
+// Tiles by the blocks they give, the largest that fill the chip (160 of 256
+// CUs): 128 tokens x 512 weight rows and 128 x 256 re-read the least (C4
+// gate/up at 443 tokens 261 us against 306 for 64 x 256; O at 1900 118 us on
+// 128 x 256 against 130 on half-filled 128 x 512), then 64 x 256. Shapes with
+// fewer blocks split K over 64 x 256 tiles, or over 64 x 128 tiles for up to
+// 128 tokens and K below 8192 (C4 O at 116 tokens 19.8 against 23.3 us, QKV
+// 25.6 against 25.4; down, K 16384, 46.7 in both). Up to 64 tokens the weights
+// are the bound and 64 x 128 tiles keep the most loads in flight, up to 32
+// tokens 32 x 128 (C4 at 12 tokens, against the skinny GEMM: gate/up 70.8 ->
+// 40.8 us = 6.6 TB/s, down 40.2 -> 28.8), with four sums per tile: the skinny
+// GEMM's K slices kept its chains short.
+static hipError_t gemm_pair_route(hipStream_t stream, const GemmPair &g, const GemmWorkspace &ws) {
+    // A SwiGLU wave holds gate and up tiles: an even number of tiles per wave.
+    auto blocks = [&](uint32_t bm, uint32_t bn) {
+        return (uint64_t)((g.t + bm - 1) / bm) * ((g.w.rows + bn - 1) / bn);
+    };
+    if (g.t <= 32 && !g.swiglu) return gemm_pair_variant<1, 1, 1, 4, 6, 2, 4>(stream, g, ws, 256);
+    if (g.t <= 32) return gemm_pair_variant<1, 2, 1, 2, 6, 2, 4>(stream, g, ws, 256);
+    if (g.t <= 64) return gemm_pair_variant<1, 2, 2, 2, 5, 2>(stream, g, ws, 384);
+    if (g.t > 128 && blocks(128, 512) >= 160)
+        return gemm_pair_variant<2, 4, 2, 4, 3, 1>(stream, g, ws, 0);
+    if (g.t > 128 && blocks(128, 256) >= 160)
+        return gemm_pair_variant<2, 2, 2, 4, 4, 1>(stream, g, ws, 0);
+    if (blocks(64, 256) >= 160 || g.t > 128 || g.w.cols >= 8192)
+        return gemm_pair_variant<1, 2, 2, 4, 6, 1>(stream, g, ws, 256);
+    return gemm_pair_variant<1, 2, 2, 2, 5, 2>(stream, g, ws, 384);
+}
+
+hipError_t launch_gemm_pair(hipStream_t stream, const PairRows &x, const PairWeight &w,
+                            uint64_t tokens, float *y, uint64_t y_stride, const GemmWorkspace &ws) {
+    if (!tokens || tokens > x.padded || !pair_supported(w.rows, w.cols)) return hipErrorInvalidValue;
+    GemmPair g{};
+    g.planes = x.planes;
+    g.row_exps = x.exps;
+    g.padded = x.padded;
+    g.w = w;
+    g.t = (uint32_t)tokens;
+    g.y = y;
+    g.ldy = y_stride;
+    return gemm_pair_route(stream, g, ws);
+}
+
+hipError_t launch_gemm_pair_swiglu(hipStream_t stream, const PairRows &x, const PairWeight &w,
+                                   uint64_t tokens, const PairRows &act, const GemmWorkspace &ws) {
+    if (!tokens || tokens > x.padded || act.padded != x.padded || !pair_supported(w.rows, w.cols) ||
+        w.rows % 64)
+        return hipErrorInvalidValue;
+    GemmPair g{};
+    g.planes = x.planes;
+    g.row_exps = x.exps;
+    g.padded = x.padded;
+    g.w = w;
+    g.t = (uint32_t)tokens;
+    g.swiglu = w.rows / 2;
+    g.act = act.planes;
+    g.act_exps = act.exps;
+    return gemm_pair_route(stream, g, ws);
 }
 
 // ---------------------------------------------------------------- row norms
@@ -2204,18 +2613,19 @@ __global__ __launch_bounds__(kThreads) void norm_rows_kernel(const float *x, uin
 // norm_rows_kernel with the row held in registers, 16-byte accesses (width a
 // multiple of 4, at most 8192): every load goes out before the sum, where the
 // strided loop above waits on each in turn (C5 verify's first norm 15 us).
-// With planes, blocks past `rows` (up to `padded`) write zero planes only.
+// With pair.planes the normalized row goes there as a scaled pair of fp16 terms
+// instead of y; blocks past `rows` (up to pair.padded) write zeros. Without w
+// the row is taken as it is.
 template <int NV>
 __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, uint64_t x_stride,
                                                               const uint16_t *w, float offset,
                                                               float *y, uint64_t y_stride,
-                                                              uint32_t width, uint16_t *planes,
-                                                              uint32_t padded, uint32_t rows) {
+                                                              uint32_t width, PairRows pair,
+                                                              uint32_t rows) {
     __shared__ float red[4];
     const uint32_t groups = width / 4;
     if (blockIdx.x >= rows) {
-        for (uint32_t i = threadIdx.x; i < groups; i += kThreads)
-            write_planes4(planes, padded, blockIdx.x, 4 * i, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+        pair_zero_row(pair, blockIdx.x, width);
         return;
     }
     const float *xr = x + blockIdx.x * x_stride;
@@ -2227,7 +2637,7 @@ __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, ui
         const uint32_t i = threadIdx.x + kThreads * j;
         const uint32_t c = (i < groups ? i : groups - 1) * 4;
         const f32x4 xv = *(const f32x4 *)(xr + c);
-        const u32x2 wv = *(const u32x2 *)(w + c);
+        const u32x2 wv = w ? *(const u32x2 *)(w + c) : u32x2{0u, 0u};
         v[j] = i < groups ? xv : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         g[j] = wv;
     }
@@ -2239,48 +2649,43 @@ __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, ui
             const float t = v[j][e] * v[j][e];
             ss = ss + t;
         }
-    const float inv = block_inverse_from_partial(ss, width, red);
+    const float inv = w ? block_inverse_from_partial(ss, width, red) : 1.0f;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const uint32_t i = threadIdx.x + kThreads * j;
         const uint32_t wb[4] = {g[j].x & 0xffffu, g[j].x >> 16, g[j].y & 0xffffu, g[j].y >> 16};
-        f32x4 o;
+        if (w)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (v[j][e] * inv) * (bf16f(wb[e]) + offset);
-        if (i < groups) {
-            *(f32x4 *)(yr + 4 * i) = o;
-            if (planes) write_planes4(planes, padded, blockIdx.x, 4 * i, o);
-        }
+            for (int e = 0; e < 4; ++e) v[j][e] = (v[j][e] * inv) * (bf16f(wb[e]) + offset);
+        if (!pair.planes && i < groups) *(f32x4 *)(yr + 4 * i) = v[j];
     }
+    if (pair.planes) pair_row<NV>(pair, blockIdx.x, groups, v, red);
 }
 
 hipError_t launch_norm_rows(hipStream_t stream, const float *x, uint64_t x_stride,
                             const uint16_t *w, float offset, float *y, uint64_t y_stride,
-                            uint64_t width, uint64_t rows, uint16_t *planes, uint32_t padded) {
+                            uint64_t width, uint64_t rows, const PairRows *pair) {
     if (!rows) return hipSuccess;
-    if (planes && (padded < rows || width % (2 * kSplitBK))) return hipErrorInvalidValue;
     if (width % 4 == 0 && width <= 8192 && x_stride % 4 == 0 && y_stride % 4 == 0 &&
         !((uintptr_t)x & 15) && !((uintptr_t)y & 15) && !((uintptr_t)w & 7)) {
+        if (pair && (pair->padded < rows || width % kPairK)) return hipErrorInvalidValue;
         const uint32_t wd = (uint32_t)width, n = (uint32_t)rows;
-        const unsigned grid = planes ? padded : n;
+        const unsigned grid = pair ? pair->padded : n;
+        const PairRows pr = pair ? *pair : PairRows{};
         if (width <= 2048)
             norm_rows4_kernel<2><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, planes, padded, n);
+                                                                y_stride, wd, pr, n);
         else if (width <= 4096)
             norm_rows4_kernel<4><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, planes, padded, n);
+                                                                y_stride, wd, pr, n);
         else
             norm_rows4_kernel<8><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, planes, padded, n);
+                                                                y_stride, wd, pr, n);
         return hipGetLastError();
     }
+    if (pair || !w) return hipErrorInvalidValue;
     norm_rows_kernel<<<(unsigned)rows, kThreads, 0, stream>>>(x, x_stride, w, offset, y, y_stride,
                                                               (uint32_t)width);
-    if (planes) {
-        const uint64_t elems = (uint64_t)padded * width;
-        split_planes_kernel<<<(unsigned)((elems / 8 + 255) / 256), 256, 0, stream>>>(
-            y, y_stride, (uint32_t)rows, padded, (uint32_t)width, planes);
-    }
     return hipGetLastError();
 }
 
@@ -2354,14 +2759,13 @@ __global__ __launch_bounds__(kThreads) void residual_norm_rows_kernel(
 template <int NV>
 __global__ __launch_bounds__(kThreads) void residual_norm_rows4_kernel(
     float *state, const float *branch, const uint16_t *wr, float off_r, const uint16_t *wn,
-    float off_n, float *norm, uint64_t norm_stride, uint32_t width, uint16_t *planes,
-    uint32_t padded, uint32_t rows) {
+    float off_n, float *norm, uint64_t norm_stride, uint32_t width, PairRows pair,
+    uint32_t rows) {
     __shared__ float red[4];
     const uint64_t row = blockIdx.x;
     const uint32_t groups = width / 4;
     if (blockIdx.x >= rows) {  // padding rows of the planes
-        for (uint32_t i = threadIdx.x; i < groups; i += kThreads)
-            write_planes4(planes, padded, blockIdx.x, 4 * i, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+        pair_zero_row(pair, blockIdx.x, width);
         return;
     }
     f32x4 b[NV], st[NV];
@@ -2408,41 +2812,38 @@ __global__ __launch_bounds__(kThreads) void residual_norm_rows4_kernel(
     for (int j = 0; j < NV; ++j) {
         const uint32_t g = threadIdx.x + kThreads * j;
         const uint32_t w[4] = {gn[j].x & 0xffffu, gn[j].x >> 16, gn[j].y & 0xffffu, gn[j].y >> 16};
-        f32x4 o;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (st[j][e] * inv2) * (bf16f(w[e]) + off_n);
-        if (g < groups) {
-            *(f32x4 *)(norm + row * norm_stride + 4 * g) = o;
-            if (planes) write_planes4(planes, padded, blockIdx.x, 4 * g, o);
-        }
+        for (int e = 0; e < 4; ++e) st[j][e] = (st[j][e] * inv2) * (bf16f(w[e]) + off_n);
+        if (!pair.planes && g < groups) *(f32x4 *)(norm + row * norm_stride + 4 * g) = st[j];
     }
+    if (pair.planes) pair_row<NV>(pair, blockIdx.x, groups, st, red);
 }
 
 hipError_t launch_residual_norm_rows(hipStream_t stream, float *state, const float *branch,
                                      const uint16_t *wr, float off_r, const uint16_t *wn,
                                      float off_n, float *norm, uint64_t norm_stride,
-                                     uint64_t width, uint64_t rows, uint16_t *planes,
-                                     uint32_t padded) {
+                                     uint64_t width, uint64_t rows, const PairRows *pair) {
     if (!rows) return hipSuccess;
-    if (planes && (padded < rows || width % (2 * kSplitBK))) return hipErrorInvalidValue;
     const uint32_t w = (uint32_t)width;
     if (width % 4 == 0 && norm_stride % 4 == 0 && !((uintptr_t)state & 15) &&
         !((uintptr_t)branch & 15) && !((uintptr_t)norm & 15) && !((uintptr_t)wr & 7) &&
         !((uintptr_t)wn & 7) && width <= 8192) {
+        if (pair && (pair->padded < rows || width % kPairK)) return hipErrorInvalidValue;
         const uint32_t n = (uint32_t)rows;
-        const unsigned grid = planes ? padded : n;
+        const unsigned grid = pair ? pair->padded : n;
+        const PairRows pr = pair ? *pair : PairRows{};
         if (width <= 2048)
             residual_norm_rows4_kernel<2><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, planes, padded, n);
+                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, n);
         else if (width <= 4096)
             residual_norm_rows4_kernel<4><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, planes, padded, n);
+                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, n);
         else
             residual_norm_rows4_kernel<8><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, planes, padded, n);
+                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, n);
         return hipGetLastError();
     }
-    if (planes) return hipErrorInvalidValue;
+    if (pair) return hipErrorInvalidValue;
     if (width <= 2048)
         residual_norm_rows_kernel<8><<<(unsigned)rows, kThreads, 0, stream>>>(
             state, branch, wr, off_r, wn, off_n, norm, norm_stride, w);
@@ -2477,45 +2878,8 @@ __global__ __launch_bounds__(kThreads) void swiglu_rows_kernel(const float *gate
     out[e] = (g / d) * u;
 }
 
-// swiglu_rows_kernel straight into the BF16 planes of the down projection's
-// matrix-core GEMM (the layout and three-term split of split_planes_kernel),
-// four columns per thread; rows past `rows` (up to `padded`) get zero planes.
-// The FP32 activation is not written: the GEMM reads the planes only.
-__global__ __launch_bounds__(kThreads) void swiglu_planes_kernel(const float *gate_up,
-                                                                 uint32_t intermediate,
-                                                                 uint32_t rows, uint32_t padded,
-                                                                 uint16_t *planes) {
-    const uint32_t quads = intermediate / 4;
-    const uint64_t e = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (e >= (uint64_t)quads * padded) return;
-    const uint32_t t = (uint32_t)(e / quads), c = (uint32_t)(e % quads) * 4;
-    f32x4 v = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    if (t < rows) {
-        const float *row = gate_up + (uint64_t)t * 2 * intermediate;
-        const f32x4 g = *(const f32x4 *)(row + c), u = *(const f32x4 *)(row + intermediate + c);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float d = plamo_exp(-g[i]) + 1.0f;
-            v[i] = (g[i] / d) * u[i];
-        }
-    }
-    write_planes4(planes, padded, t, c, v);
-}
-
 hipError_t launch_swiglu_rows(hipStream_t stream, const float *gate_up, float *out,
-                              uint64_t intermediate, uint64_t rows, uint16_t *planes,
-                              uint32_t padded) {
-    if (planes) {
-        if (intermediate % (2 * kSplitBK) || intermediate >= (1u << 30) || padded < rows ||
-            ((uintptr_t)gate_up & 15))
-            return hipErrorInvalidValue;
-        const uint64_t threads = intermediate / 4 * padded;
-        if (!threads) return hipSuccess;
-        swiglu_planes_kernel<<<(unsigned)((threads + kThreads - 1) / kThreads), kThreads, 0,
-                               stream>>>(gate_up, (uint32_t)intermediate, (uint32_t)rows, padded,
-                                         planes);
-        return hipGetLastError();
-    }
+                              uint64_t intermediate, uint64_t rows) {
     uint64_t total = intermediate * rows;
     if (!total) return hipSuccess;
     swiglu_rows_kernel<<<(unsigned)((total + kThreads - 1) / kThreads), kThreads, 0, stream>>>(
@@ -3505,14 +3869,12 @@ __global__ __launch_bounds__(kThreads) void prompt_attention_kernel(PromptAttent
 // and sum, and the factors exp(m_z - m) go to the wave's LDS slots; then the
 // sum of weights and each output column are accumulated over the splits in
 // split order, skipping splits that saw no key (maximum -inf), as a plain
-// sequential loop over the records would. With `planes`, each output value
-// is written as its three BF16 terms for the O projection's GEMM instead.
+// sequential loop over the records would.
 constexpr uint32_t kMergeSplits = 64;
 __global__ __launch_bounds__(256) void attention_merge_kernel(const float *partial,
                                                               uint32_t splits, uint64_t stride,
                                                               uint32_t dim, float *out,
-                                                              uint32_t qh, uint32_t pairs,
-                                                              uint16_t *planes, uint32_t padded) {
+                                                              uint32_t pairs) {
     __shared__ float fz_s[4][kMergeSplits], lz_s[4][kMergeSplits];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t pair = blockIdx.x * 4 + wave;  // token * qh + head
@@ -3545,11 +3907,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const float *parti
         }
         for (; z < splits; ++z)
             if (live >> z & 1) acc += p[z * stride + d] * fz[z];
-        const float o = acc / l;
-        if (planes)
-            write_planes1(planes, padded, pair / qh, pair % qh * dim + d, o);
-        else
-            out[(uint64_t)pair * dim + d] = o;
+        out[(uint64_t)pair * dim + d] = acc / l;
     }
 }
 
@@ -3743,20 +4101,7 @@ __global__ __launch_bounds__(64 * G) void prompt_attention_mfma_kernel(PromptAtt
         } else {
             float *out = a.out + (uint64_t)t * a.qh * DIM + (uint64_t)h * DIM;
 #pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                const float y = o[n][v] / l_run[v];
-                if (!a.planes) {
-                    out[16 * n + col] = y;
-                } else {
-                    // Lanes 4j .. 4j + 3 hold four adjacent columns: the
-                    // first writes them as one group of planes.
-                    const float y1 = __shfl_down(y, 1, 4), y2 = __shfl_down(y, 2, 4),
-                                y3 = __shfl_down(y, 3, 4);
-                    if (col % 4 == 0)
-                        write_planes4(a.planes, a.padded, t, h * DIM + 16 * n + col,
-                                      f32x4{y, y1, y2, y3});
-                }
-            }
+            for (int n = 0; n < NT; ++n) out[16 * n + col] = o[n][v] / l_run[v];
         }
     }
 }
@@ -3828,11 +4173,7 @@ uint64_t prompt_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t qh,
 
 hipError_t launch_prompt_attention(hipStream_t stream, const PromptAttention &a) {
     if (!a.tokens) return hipSuccess;
-    // Planes come from the matrix-core form only; the scalar form refuses
-    // them rather than leave them unwritten.
     const bool matrix = prompt_mfma_takes(a.dim, a.qh, a.kh, a.window, a.rotated);
-    if (a.planes && (!matrix || a.padded < a.tokens || (a.qh * a.dim) % (2 * kSplitBK)))
-        return hipErrorInvalidValue;
     uint32_t rows = 0, splits = 1;
     hipError_t e;
     if (matrix) {
@@ -3849,8 +4190,8 @@ hipError_t launch_prompt_attention(hipStream_t stream, const PromptAttention &a)
     if (e != hipSuccess) return e;
     if (splits > 1)
         attention_merge_kernel<<<(a.tokens * a.qh + 3) / 4, 256, 0, stream>>>(
-            a.partial, splits, (uint64_t)a.tokens * a.qh * (a.dim + 2), a.dim, a.out, a.qh,
-            a.tokens * a.qh, a.planes, a.padded);
+            a.partial, splits, (uint64_t)a.tokens * a.qh * (a.dim + 2), a.dim, a.out,
+            a.tokens * a.qh);
     return hipGetLastError();
 }
 

@@ -19,7 +19,7 @@ here for FP32 accumulation over 4096 terms.
 import numpy as np
 import pytest
 
-from parity import gate, oracle_lib, plamo_hip, say
+from parity import compare, gate, oracle_lib, plamo_hip, say
 
 pytestmark = pytest.mark.gpu
 
@@ -231,3 +231,35 @@ def test_mlp_fused_swiglu(oracle, tokens):
         be.close()
         a.close()
         s.close()
+
+
+# The fp16-pair GEMM of prompts from six tokens on: each tile (32, 64 and 128
+# tokens by 128, 256 and 512 weight rows, with and without K splits) at its
+# edges, weight rows and intermediate columns that are not whole tiles, and
+# weights whose activations span a far wider range than a norm's output.
+@pytest.mark.parametrize("hidden,inter,tokens,std", [
+    (256, 96, 6, 0.02), (256, 96, 32, 0.02), (288, 160, 33, 0.02), (512, 1056, 64, 0.02),
+    (512, 1056, 65, 1.0), (512, 1056, 128, 0.02), (288, 4128, 130, 0.02), (288, 8224, 301, 0.02),
+    (288, 8224, 700, 0.02), (256, 8192, 700, 1.0), (2048, 96, 40, 0.02),
+])
+def test_prompt_pair_gemm(hidden, inter, tokens, std):
+    say(f"pair GEMM hidden={hidden} inter={inter} tokens={tokens} std={std}")
+    syn = plamo_hip.Synthetic(hidden, 2, 4, 2, 64, inter, 200, window=1024, global_capacity=1024,
+                              pattern=2, embedding_std=1.0, weight_std=std, seed=tokens)
+    gpu, cpu = syn.instance(), syn.instance()
+    be = plamo_hip.Backend(syn)
+    try:
+        ids = [(7 * j + 3) % 200 for j in range(tokens)]
+        actual = np.zeros((tokens, hidden), np.float32)
+        expected = np.zeros((tokens, hidden), np.float32)
+        assert be.prefill(gpu, ids, actual) == 1
+        assert oracle_lib.prefill(cpu, ids, expected)
+        gate(actual, expected, "all prompt states")
+        compare(gpu, cpu)
+        info = be.info()
+        assert info.errors == 0 and info.cpu_fallbacks == 0, info.note.decode()
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
