@@ -834,7 +834,7 @@ int ensure_pair(plamo_metal *m, struct model *model) {
     for (size_t i = 0; i < places.size(); ++i) {
         const Place &q = places[i];
         *q.p = PairWeight{(uint16_t *)(m->pair_block + q.frag), (int32_t *)(m->pair_block + q.exps),
-                          (uint32_t)q.rows, (uint32_t)q.cols};
+                          (uint32_t)q.rows, (uint32_t)q.cols, (uint32_t)((q.rows + 31) / 32)};
         HIP_TRY(m, launch_pair_weights(m->stream, q.w, *q.p,
                                        q.gate_up ? m->layers[i / 4].gu_norms : nullptr,
                                        q.rows / 2));
@@ -1128,7 +1128,7 @@ int encode_decode(plamo_metal *m, struct model *model, const DecodePlan &plan, i
             pa.q = m->q;
             pa.table = rope.table;
             pa.out = m->attn;
-            pa.prefix = count;
+            pa.prefix = pa.cached = count;
             pa.tokens = 1;
             pa.qh = d.qh;
             pa.kh = d.kh;
@@ -1616,6 +1616,11 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         split_floats = std::max(split_floats,
                                 prompt_attention_scratch((uint32_t)c->count, (uint32_t)T, d.qh,
                                                          d.kh, d.dim, window, wide[i]));
+        // The last layer's attention may run for its last row alone.
+        if (i + 1 == L)
+            split_floats = std::max(split_floats,
+                                    prompt_attention_scratch((uint32_t)(c->count + T - 1), 1, d.qh,
+                                                             d.kh, d.dim, window, wide[i]));
     }
     if (split_floats && !ensure(m, m->p_attn_split, split_floats * 4)) return -1;
     if (virtual_floats && !ensure(m, m->p_virtual, virtual_floats * 4)) return -1;
@@ -1671,12 +1676,28 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                        *mpost = d.norms + 3 * h, *qn = d.norms + 4 * h, *kn = qn + d.dim;
         const RopeTable &rope = m->ropes[d.rope];
         const uint64_t qkv_w = (uint64_t)(d.qh + 2 * d.kh) * d.dim, aw = (uint64_t)d.qh * d.dim;
+        // With states == NULL only the final row feeds the logits: the last
+        // layer's queries, attention, O projection and MLP run for that row
+        // alone, as the decode step runs them (runtime/metal_model.m:761-770
+        // trims the projection and the MLP); K and V rows are formed for all.
+        const bool last_row_only = !verify && !states && i + 1 == L && T > 1;
+        const bool last_query = last_row_only && pair && aw % 32 == 0 &&
+                                prompt_attention_matrix(d.dim, d.qh, d.kh);
         if (!normed) {
             HIP_FAIL(m, launch_norm_rows(s, state, h, pre, 1.0f, norm, h, h, T, norm_pair));
             ++n;
         }
         normed = false;
-        if (pair)
+        if (last_query) {
+            Prologue pq{};
+            pq.src = state + (T - 1) * h;
+            pq.w = pre;
+            pq.offset = 1.0f;
+            HIP_FAIL(m, launch_gemm_pair(s, in, pair_rows_from(d.p_qkv, (uint32_t)aw), T, qkv + aw,
+                                         qkv_w, *ws));
+            HIP_FAIL(m, launch_gemv(s, d.qkv, aw, h, pq, qkv + (T - 1) * qkv_w, 0, 2 * m->cus));
+            ++n;
+        } else if (pair)
             HIP_FAIL(m, launch_gemm_pair(s, in, d.p_qkv, T, qkv, qkv_w, *ws));
         else
             HIP_FAIL(m, launch_gemm(s, norm, h, d.qkv, qkv_w, h, T, qkv, qkv_w, ws));
@@ -1733,17 +1754,14 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             HIP_FAIL(m, launch_rerotate(s, d.k, qp.k_virtual, rope.exact, c->count, d.kh, d.dim));
             ++n;
         }
+        qp.last_query = last_query;
         HIP_FAIL(m, launch_qkv_post(s, qp));
         ++n;
-        // With states == NULL only the final row feeds the logits; the last
-        // layer's projection and MLP run for that row alone
-        // (runtime/metal_model.m:761-770).
-        const bool last_row_only = !verify && !states && i + 1 == L && T > 1;
         PromptAttention pa{};
         pa.q = q;
         pa.table = rope.table;
         pa.out = attn;
-        pa.prefix = (uint32_t)c->count;
+        pa.prefix = pa.cached = (uint32_t)c->count;
         pa.tokens = (uint32_t)T;
         pa.partial = split_floats ? as<float>(m->p_attn_split) : nullptr;
         pa.qh = d.qh;
@@ -1766,6 +1784,12 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             pa.k_new = verify ? prop_r : d.rot + c->count * d.width;
             pa.v_new = verify ? prop_v : d.v + c->count * d.width;
             pa.window = 0;
+        }
+        if (last_query) {
+            pa.q += (T - 1) * aw;
+            pa.out += (T - 1) * aw;
+            pa.prefix += (uint32_t)(T - 1);
+            pa.tokens = 1;
         }
         HIP_FAIL(m, launch_prompt_attention(s, pa));
         ++n;
@@ -1810,23 +1834,37 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         }
         float *st = state + first * h;
         if (rows == 1 && !verify) {
-            // One prompt row: the decode GEMVs (norm and SwiGLU fused) instead of
-            // GEMM tiles. A one-candidate verify keeps the token GEMVs and the
-            // fused residual norms: C5 verify(1) 12.9 against 14.1 ms this way.
+            // One prompt row: the decode GEMVs (residual, norm and SwiGLU
+            // fused) instead of GEMM tiles. A one-candidate verify keeps the
+            // token GEMVs and the fused residual norms: C5 verify(1) 12.9
+            // against 14.1 ms this way. The state moves between `st` and
+            // state_a (a block would read what another writes otherwise); the
+            // last layer's final residual is left to the head's prologue.
             Prologue po{};
             po.src = attn + first * aw;
             HIP_FAIL(m, launch_gemv(s, d.o, h, aw, po, branch, 0, 2 * m->cus));
-            HIP_FAIL(m, launch_residual_rows(s, st, branch, post, kAttentionOffset, h, 1));
             Prologue pg{};
             pg.src = st;
             pg.w = mpre;
             pg.offset = 1.0f;
+            if (i + 1 == L) {
+                pg.branch = branch;
+                pg.rw = post;
+                pg.roffset = kAttentionOffset;
+                pg.state_out = m->state_a;
+            } else {
+                HIP_FAIL(m, launch_residual_rows(s, st, branch, post, kAttentionOffset, h, 1));
+                ++n;
+            }
             HIP_FAIL(m, launch_gemv(s, d.gu, 2 * (uint64_t)d.inter, h, pg, act, d.inter, 2 * m->cus));
             Prologue pd{};
             pd.src = act;
             HIP_FAIL(m, launch_gemv(s, d.down, h, d.inter, pd, branch, 0, 2 * m->cus));
-            HIP_FAIL(m, launch_residual_rows(s, st, branch, mpost, kMlpOffset, h, 1));
-            n += 5;
+            if (i + 1 < L) {
+                HIP_FAIL(m, launch_residual_rows(s, st, branch, mpost, kMlpOffset, h, 1));
+                ++n;
+            }
+            n += 3;
         } else {
             if (pair) {
                 // rows == T: `in` is sized for them. The attention rows become
@@ -1895,16 +1933,24 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         HIP_FAIL(m, hipMemcpyAsync(m->status_host, &m->params_dev->error, 4, hipMemcpyDeviceToHost, s));
         n += 3;
     } else {
+        const bool one_row = T == 1 || !states;  // the last layer ran as a decode step
         const float *last = state + (T - 1) * h;
         Prologue ph{};
-        ph.src = last;
+        ph.src = one_row ? m->state_a : last;
         ph.w = m->final_norm;
         ph.offset = 1.0f;
+        if (one_row) {
+            ph.branch = branch;
+            ph.rw = m->layers[L - 1].norms + 3 * h;
+            ph.roffset = kMlpOffset;
+            ph.state_out = m->outbox + V;
+        }
         ph.norm_out = m->outbox + V + h;
         ph.status = &m->params_dev->error;
         ph.status_out = m->status_dev;
         HIP_FAIL(m, launch_gemv(s, m->head, V, h, ph, m->outbox, 0, 2 * m->cus));
-        HIP_FAIL(m, hipMemcpyAsync(m->outbox + V, last, h * 4, hipMemcpyDeviceToDevice, s));
+        if (!one_row)
+            HIP_FAIL(m, hipMemcpyAsync(m->outbox + V, last, h * 4, hipMemcpyDeviceToDevice, s));
         HIP_FAIL(m, hipMemcpyAsync(m->outbox_host, m->outbox, (V + 2 * h) * 4,
                                   hipMemcpyDeviceToHost, s));
         ++n;
@@ -1921,7 +1967,8 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         return 1;
     }
     // Host mirror: prompt states, final state / normalized / logits, new KV rows.
-    if (states && hipMemcpy(states, state, T * h * 4, hipMemcpyDeviceToHost) != hipSuccess) {
+    const float *final_states = T == 1 ? m->outbox + V : state;
+    if (states && hipMemcpy(states, final_states, T * h * 4, hipMemcpyDeviceToHost) != hipSuccess) {
         problem(m, "cannot copy prompt states");
         return fail(m);
     }

@@ -100,12 +100,15 @@ hipError_t launch_gemm(hipStream_t, const float *x, uint64_t x_stride, const uin
                        uint64_t y_stride, const GemmWorkspace *ws);
 
 // A projection's weights as scaled fp16 fragments for launch_gemm_pair, and
-// each row's exponent (value = fragment * 2^-exps[row]); rows padded to 32.
+// each row's exponent (value = fragment * 2^-exps[row]); rows padded to 32,
+// `groups` groups of 32 rows per 32-column stage of the layout.
 struct PairWeight {
     uint16_t *frag;
     int32_t *exps;
-    uint32_t rows, cols;
+    uint32_t rows, cols, groups;
 };
+// The rows from `first` (a multiple of 32) on.
+PairWeight pair_rows_from(const PairWeight &w, uint32_t first);
 // Rows of X as scaled pairs of fp16 terms: [cols / 32][hi, lo][padded][32],
 // value = (hi + lo) * 2^-exps[row]. With act_exps (and norms, the largest
 // 2-norms of the gate and of the up rows as float bits), a norm also writes
@@ -177,6 +180,8 @@ struct QkvPost {
     int rows_from_count;
     int rotate_k;            // 0: leave k_rot alone (sliding overflow)
     float *stage;            // optional [3][width] copy of the last row (decode mirror)
+    int last_query;          // nonzero: only the last row's query heads
+    uint32_t head0, token0;  // first head and row of a launch (set by the launcher)
     // Optional: Q is rotated at its virtual row (count + t, past the window's
     // capacity too) by this table instead, and the keys, rotated likewise, go
     // to k_virtual[(count + t) * width].
@@ -239,8 +244,9 @@ bool attention_o_supported(uint32_t dim, uint32_t group, uint64_t cols);
 constexpr uint32_t kDecodeShortRows = 256;
 uint32_t decode_attention_splits(uint64_t rows);
 
-// General causal attention for `tokens` query rows. Key j of query t is the
-// virtual row j of [cache rows 0..prefix) ++ [new rows 0..tokens). With
+// General causal attention for `tokens` query rows, the first at virtual row
+// `prefix`. Key j of query t is the virtual row j of [cache rows 0..cached) ++
+// [new rows 0..). With
 // window > 0 query t sees only the last `window` virtual rows ending at its
 // own row; its keys are raw and rotated on the fly at their window-local
 // position, or `rotated` (keys and Q at their virtual rows) where
@@ -251,7 +257,7 @@ struct PromptAttention {
     const float *k_new, *v_new;      // rotated (or raw when window) new rows
     const float *table;
     float *out;              // [tokens, qh*dim]
-    uint32_t prefix, tokens, qh, kh, dim, window;
+    uint32_t prefix, tokens, cached, qh, kh, dim, window;
     int rotated;
     // Optional scratch for key splits (prompt_attention_scratch floats): few
     // query tiles then spread their keys over several blocks and a merge.

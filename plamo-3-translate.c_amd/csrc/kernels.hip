@@ -2249,9 +2249,18 @@ bool pair_supported(uint64_t rows, uint64_t cols) {
 uint64_t pair_frag_elems(uint64_t rows, uint64_t cols) { return (rows + 31) / 32 * 32 * cols; }
 uint64_t pair_exp_count(uint64_t rows) { return (rows + 31) / 32 * 32; }
 
+PairWeight pair_rows_from(const PairWeight &w, uint32_t first) {
+    PairWeight r = w;
+    r.frag += (uint64_t)first / 32 * 1024;
+    r.exps += first;
+    r.rows -= first;
+    return r;
+}
+
 hipError_t launch_pair_weights(hipStream_t stream, const uint16_t *w, const PairWeight &p,
                                uint32_t *norms, uint64_t half) {
-    if (!pair_supported(p.rows, p.cols) || ((uintptr_t)w & 15)) return hipErrorInvalidValue;
+    if (!pair_supported(p.rows, p.cols) || ((uintptr_t)w & 15) || p.groups != (p.rows + 31) / 32)
+        return hipErrorInvalidValue;
     pair_weights_kernel<<<(p.rows + 31) / 32, kThreads, 0, stream>>>(w, p.rows, p.cols, p.frag,
                                                                      p.exps, norms, (uint32_t)half);
     return hipGetLastError();
@@ -2309,6 +2318,7 @@ __global__ __launch_bounds__(64 * GM * GN, OCC) void gemm_pair_kernel(GemmPair g
     const uint32_t m0 = bm * BM;
     const uint32_t nst = g.w.cols / kPairK / g.splits, s0 = bz * nst;
     const uint32_t groups = (g.w.rows + 31) / 32, half = g.swiglu / 32;
+    const uint32_t stage_groups = g.w.groups;
     // Weight row group of tile j of wave column c.
     auto row_group = [&](uint32_t c, uint32_t j) -> uint32_t {
         if (g.swiglu)
@@ -2327,9 +2337,9 @@ __global__ __launch_bounds__(64 * GM * GN, OCC) void gemm_pair_kernel(GemmPair g
             advance[i] = 4 * kPairK * g.padded;
         } else {
             const uint32_t f = L - AI;
-            src[i] = (const char *)(g.w.frag + ((uint64_t)s0 * groups + row_group(f / 2 / WN, f / 2 % WN)) * 1024 +
+            src[i] = (const char *)(g.w.frag + ((uint64_t)s0 * stage_groups + row_group(f / 2 / WN, f / 2 % WN)) * 1024 +
                                     (f & 1) * 512 + lane * 8);
-            advance[i] = groups * 2048;
+            advance[i] = stage_groups * 2048;
         }
     }
     // Loads past the last stage repeat it into buffers no later step reads.
@@ -2891,7 +2901,7 @@ hipError_t launch_swiglu_rows(hipStream_t stream, const float *gate_up, float *o
 // src/qkv.s:36-67 (offset-1 head RMSNorm), src/cache.s:8 (append raw K, V),
 // src/cache_rope.s:44-75 + tests/rope_reference.s:14-30 (rotate).
 __global__ __launch_bounds__(64) void qkv_post_kernel(QkvPost a) {
-    const uint32_t h = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
+    const uint32_t h = a.head0 + blockIdx.x, t = a.token0 + blockIdx.y, lane = threadIdx.x;
     const uint32_t dim = a.dim, half = dim / 2, width = a.kh * dim;
     const uint32_t stride = (a.qh + 2 * a.kh) * dim;
     const float *x = a.qkv + (uint64_t)t * stride + (uint64_t)h * dim;
@@ -2962,6 +2972,15 @@ __global__ __launch_bounds__(64) void qkv_post_kernel(QkvPost a) {
 
 hipError_t launch_qkv_post(hipStream_t stream, const QkvPost &a) {
     if (!a.tokens) return hipSuccess;
+    if (a.last_query) {
+        QkvPost q = a;
+        q.token0 = a.tokens - 1;
+        qkv_post_kernel<<<dim3(a.qh, 1), 64, 0, stream>>>(q);
+        q.token0 = 0;
+        q.head0 = a.qh;
+        qkv_post_kernel<<<dim3(a.kh, a.tokens), 64, 0, stream>>>(q);
+        return hipGetLastError();
+    }
     qkv_post_kernel<<<dim3(a.qh + a.kh, a.tokens), 64, 0, stream>>>(a);
     return hipGetLastError();
 }
@@ -3752,10 +3771,10 @@ __global__ __launch_bounds__(kThreads) void prompt_attention_kernel(PromptAttent
                 const uint32_t i = min(base + j * kThreads, kKT * dim - 1);
                 const uint32_t r = min(i / dim, nk - 1), d = i % dim;
                 const uint32_t vrow = k0 + r;
-                const float *kp = vrow < a.prefix ? a.k_cache + (uint64_t)vrow * width
-                                                  : a.k_new + (uint64_t)(vrow - a.prefix) * width;
-                const float *vp = vrow < a.prefix ? a.v_cache + (uint64_t)vrow * width
-                                                  : a.v_new + (uint64_t)(vrow - a.prefix) * width;
+                const float *kp = vrow < a.cached ? a.k_cache + (uint64_t)vrow * width
+                                                  : a.k_new + (uint64_t)(vrow - a.cached) * width;
+                const float *vp = vrow < a.cached ? a.v_cache + (uint64_t)vrow * width
+                                                  : a.v_new + (uint64_t)(vrow - a.cached) * width;
                 kv8[j] = kp[(uint64_t)kvh * dim + d];
                 vv8[j] = vp[(uint64_t)kvh * dim + d];
             }
@@ -4015,10 +4034,10 @@ __global__ __launch_bounds__(64 * G) void prompt_attention_mfma_kernel(PromptAtt
                 const uint32_t i = threadIdx.x + (base + j) * kStride;
                 const uint32_t r = i / (DIM / 4), c = (i % (DIM / 4)) * 4;
                 const uint32_t vrow = k0 + (r < nk ? r : nk - 1);
-                const float *kp = vrow < a.prefix ? a.k_cache + (uint64_t)vrow * width
-                                                  : a.k_new + (uint64_t)(vrow - a.prefix) * width;
-                const float *vp = vrow < a.prefix ? a.v_cache + (uint64_t)vrow * width
-                                                  : a.v_new + (uint64_t)(vrow - a.prefix) * width;
+                const float *kp = vrow < a.cached ? a.k_cache + (uint64_t)vrow * width
+                                                  : a.k_new + (uint64_t)(vrow - a.cached) * width;
+                const float *vp = vrow < a.cached ? a.v_cache + (uint64_t)vrow * width
+                                                  : a.v_new + (uint64_t)(vrow - a.cached) * width;
                 if (i < kPieces) {
                     kv[j] = *(const f32x4 *)(kp + (uint64_t)kvh * DIM + c);
                     vv[j] = *(const f32x4 *)(vp + (uint64_t)kvh * DIM + c);
