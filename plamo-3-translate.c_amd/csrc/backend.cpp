@@ -178,7 +178,11 @@ struct plamo_metal {
     const CopyRow *upload_view = nullptr;  // its device view
     uint64_t verification_tokens = 0, verification_index = 0;
 
-    Buffer lin_in, lin_out, mlp_state, mlp_norm, mlp_gu, mlp_act, mlp_branch, mlp_norms;
+    Buffer lin_in, lin_out, mlp_state, mlp_norm, mlp_gu, mlp_act, mlp_branch;
+    // Pinned staging of the host rows of plamo_metal_linear / plamo_metal_mlp
+    // (at most kStageBytes) and its device view.
+    char *stage_host = nullptr, *stage_view = nullptr;
+    uint64_t stage_bytes = 0;
     GemmWorkspace gemm{};  // split-K partial tiles and arrival counters
     // Fragments of every layer's projections for the prompt GEMM, one block
     // laid out once per model, and the exponents of its input and activation
@@ -1402,6 +1406,7 @@ void plamo_metal_close(struct plamo_metal *m) {
     for (void *p : m->allocations) (void)hipFree(p);
     m->allocations.clear();
     if (m->outbox_host) (void)hipHostFree(m->outbox_host);
+    if (m->stage_host) (void)hipHostFree(m->stage_host);
     if (m->ids_host) (void)hipHostFree(m->ids_host);
     if (m->v_host) (void)hipHostFree(m->v_host);
     if (m->v_next_host) (void)hipHostFree(m->v_next_host);
@@ -2155,6 +2160,33 @@ int plamo_hip_rewind(struct plamo_metal *m, struct model *model, uint64_t steps)
     return 1;
 }
 
+// Host rows of the granular entry points cross the bus through pinned memory
+// and copy kernels on the stream, up to this size of rows in and out (the
+// staging memory grows to it on demand). The runtime's copies of pageable
+// memory cost 10-15 us each at the smallest (3072 x 2048, one row: 50 -> 27 us
+// a call; an MLP branch of 37 rows of 2560: 186 -> 153), and its strided ones
+// far more (20160 x 8064, 266 rows: 4960 -> 871).
+constexpr uint64_t kStageBytes = 32ull << 20;
+
+static uint64_t stage_round(uint64_t bytes) { return (bytes + 255) / 256 * 256; }
+
+static bool ensure_stage(plamo_metal *m, uint64_t bytes) {
+    if (bytes > kStageBytes) return false;
+    if (bytes <= m->stage_bytes) return true;
+    if (m->stage_host) (void)hipHostFree(m->stage_host);
+    m->stage_host = nullptr;
+    m->stage_bytes = 0;
+    uint64_t size = 64 << 10;
+    while (size < bytes) size *= 2;
+    if (hipHostMalloc((void **)&m->stage_host, size, hipHostMallocDefault) != hipSuccess ||
+        !(m->stage_view = (char *)device_view(m->stage_host))) {
+        (void)hipGetLastError();
+        return false;
+    }
+    m->stage_bytes = size;
+    return true;
+}
+
 int plamo_metal_linear(struct plamo_metal *m, const struct plamo_matmul *mm) {
     if (!mm || !mm->rows || !mm->columns || !mm->tokens || mm->input_stride < mm->columns ||
         mm->output_stride < mm->rows)
@@ -2164,30 +2196,50 @@ int plamo_metal_linear(struct plamo_metal *m, const struct plamo_matmul *mm) {
     if (!w) return 0;
     uint64_t T = mm->tokens, K = mm->columns, N = mm->rows;
     Buffer &in = m->lin_in, &out = m->lin_out;
-    if (!ensure(m, in, T * K * 4) || !ensure(m, out, T * N * 4)) return 0;
+    const uint64_t in_bytes = stage_round(T * K * 4), out_bytes = stage_round(T * N * 4);
+    if (!ensure(m, in, in_bytes) || !ensure(m, out, out_bytes)) return 0;
     if (configure_gemv(K) != hipSuccess) {
         (void)hipGetLastError();
         return 0;
     }
-    int ok = hipMemcpy2DAsync(in.ptr, K * 4, mm->input, mm->input_stride * 4, K * 4, T,
+    const bool staged = ensure_stage(m, in_bytes + out_bytes);
+    float *stage_in = (float *)m->stage_host, *stage_out = (float *)(m->stage_host + in_bytes);
+    int ok;
+    if (staged) {
+        for (uint64_t t = 0; t < T; ++t)
+            memcpy(stage_in + t * K, mm->input + t * mm->input_stride, K * 4);
+        ok = launch_copy_block(m->stream, m->stage_view, in.ptr, in_bytes) == hipSuccess;
+    } else {
+        ok = hipMemcpy2DAsync(in.ptr, K * 4, mm->input, mm->input_stride * 4, K * 4, T,
                               hipMemcpyHostToDevice, m->stream) == hipSuccess;
+    }
     begin_timing(m);
     if (ok && T == 1) {
+        // One row's results go straight to the staging memory, as a decode
+        // step's logits go to the host array.
         Prologue p{};
         p.src = as<float>(in);
-        ok = launch_gemv(m->stream, w, N, K, p, as<float>(out), 0, 2 * m->cus) == hipSuccess;
+        float *y = staged ? (float *)(m->stage_view + in_bytes) : as<float>(out);
+        ok = launch_gemv(m->stream, w, N, K, p, y, 0, 2 * m->cus) == hipSuccess;
     } else if (ok) {
         const GemmWorkspace *ws = gemm_workspace(m, T, K);
         ok = ws && launch_gemm(m->stream, as<float>(in), K, w, N, K, T, as<float>(out), N, ws) ==
                        hipSuccess;
+        if (ok && staged)
+            ok = launch_copy_block(m->stream, out.ptr, m->stage_view + in_bytes, out_bytes) ==
+                 hipSuccess;
     }
-    ok = ok && hipMemcpy2DAsync(mm->output, mm->output_stride * 4, out.ptr, N * 4, N * 4, T,
-                                hipMemcpyDeviceToHost, m->stream) == hipSuccess;
+    if (!staged)
+        ok = ok && hipMemcpy2DAsync(mm->output, mm->output_stride * 4, out.ptr, N * 4, N * 4, T,
+                                    hipMemcpyDeviceToHost, m->stream) == hipSuccess;
     ok = ok && end_timing(m);
     if (!ok) {
         (void)hipGetLastError();
         return problem(m, "projection failed");
     }
+    if (staged)
+        for (uint64_t t = 0; t < T; ++t)
+            memcpy(mm->output + t * mm->output_stride, stage_out + t * N, N * 4);
     ++m->info.dispatches;
     return 1;
 }
@@ -2306,28 +2358,40 @@ int plamo_metal_mlp(struct plamo_metal *m, const struct mlp *mlp, float *states,
         (void)hipGetLastError();
         return 0;
     }
-    Buffer &st = m->mlp_state, &nrm = m->mlp_norm, &g = m->mlp_gu, &a = m->mlp_act,
-           &b = m->mlp_branch, &norms = m->mlp_norms;
+    // mlp_state: the two norms, then the rows.
+    Buffer &in = m->mlp_state, &nrm = m->mlp_norm, &g = m->mlp_gu, &a = m->mlp_act,
+           &b = m->mlp_branch;
+    const uint64_t norm_bytes = stage_round(2 * h * 2), row_bytes = stage_round(T * h * 4);
     const GemmWorkspace *ws = gemm_workspace(m, T, std::max(h, I));
-    bool ok = ws && ensure(m, st, T * h * 4) && ensure(m, nrm, T * h * 4) &&
-              ensure(m, g, T * 2 * I * 4) && ensure(m, a, T * I * 4) && ensure(m, b, T * h * 4) &&
-              ensure(m, norms, 2 * h * 2);
+    bool ok = ws && ensure(m, in, norm_bytes + row_bytes) && ensure(m, nrm, T * h * 4) &&
+              ensure(m, g, T * 2 * I * 4) && ensure(m, a, T * I * 4) && ensure(m, b, T * h * 4);
     hipStream_t s = m->stream;
-    ok = ok && hipMemcpyAsync(norms.ptr, mlp->pre, h * 2, hipMemcpyHostToDevice, s) == hipSuccess &&
-         hipMemcpyAsync(as<uint16_t>(norms) + h, mlp->post, h * 2, hipMemcpyHostToDevice, s) ==
-             hipSuccess &&
-         hipMemcpyAsync(st.ptr, states, T * h * 4, hipMemcpyHostToDevice, s) == hipSuccess;
+    uint16_t *norms = as<uint16_t>(in);
+    float *st = (float *)(as<char>(in) + norm_bytes);
+    const bool staged = ok && ensure_stage(m, norm_bytes + row_bytes);
+    if (staged) {
+        memcpy(m->stage_host, mlp->pre, h * 2);
+        memcpy(m->stage_host + h * 2, mlp->post, h * 2);
+        memcpy(m->stage_host + norm_bytes, states, T * h * 4);
+        ok = launch_copy_block(s, m->stage_view, in.ptr, norm_bytes + row_bytes) == hipSuccess;
+    } else {
+        ok = ok && hipMemcpyAsync(norms, mlp->pre, h * 2, hipMemcpyHostToDevice, s) == hipSuccess &&
+             hipMemcpyAsync(norms + h, mlp->post, h * 2, hipMemcpyHostToDevice, s) == hipSuccess &&
+             hipMemcpyAsync(st, states, T * h * 4, hipMemcpyHostToDevice, s) == hipSuccess;
+    }
     if (ok) begin_timing(m);
-    ok = ok && launch_norm_rows(s, as<float>(st), h, as<uint16_t>(norms), 1.0f, as<float>(nrm), h, h, T) == hipSuccess &&
+    ok = ok && launch_norm_rows(s, st, h, norms, 1.0f, as<float>(nrm), h, h, T) == hipSuccess &&
          launch_gemm_swiglu(s, as<float>(nrm), h, gu, I, h, T, as<float>(a), as<float>(g), ws) == hipSuccess &&
          launch_gemm(s, as<float>(a), I, down, h, I, T, as<float>(b), h, ws) == hipSuccess &&
-         launch_residual_rows(s, as<float>(st), as<float>(b), as<uint16_t>(norms) + h, kMlpOffset, h, T) == hipSuccess &&
-         hipMemcpyAsync(states, st.ptr, T * h * 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
+         launch_residual_rows(s, st, as<float>(b), norms + h, kMlpOffset, h, T) == hipSuccess &&
+         (staged ? launch_copy_block(s, st, m->stage_view + norm_bytes, row_bytes)
+                 : hipMemcpyAsync(states, st, T * h * 4, hipMemcpyDeviceToHost, s)) == hipSuccess &&
          end_timing(m);
     if (!ok) {
         (void)hipGetLastError();
         return problem(m, "MLP failed");
     }
+    if (staged) memcpy(states, m->stage_host + norm_bytes, T * h * 4);
     m->info.dispatches += 5;
     ++m->info.fused_mlps;
     return 1;

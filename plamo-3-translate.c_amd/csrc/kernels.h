@@ -286,6 +286,9 @@ struct CopyRow {
     uint64_t floats;
 };
 hipError_t launch_copy_rows(hipStream_t, const CopyRow *table, uint32_t entries);
+// A copy by a kernel, for pinned host memory on either side: 16-byte-aligned
+// addresses and sizes.
+hipError_t launch_copy_block(hipStream_t, const void *src, void *dst, uint64_t bytes);
 // p[0, words) = value (a kernel, so that it is also safe inside captured graphs).
 hipError_t launch_fill(hipStream_t, uint32_t *p, uint64_t words, uint32_t value);
 // Raises the dynamic LDS limit of the GEMV variants to hold `cols` floats.

@@ -1982,7 +1982,10 @@ uint64_t gemm_plane_elems(uint64_t tokens, uint64_t cols) {
 // 125.7 -> 101.4 us, O 76.1 -> 64.4, gate/up 433.6 -> 399.9, down 227.6 ->
 // 213.1), and down at 116 (76.3 -> 75.2, K 16384).
 static bool gemm_split_wide(uint64_t rows, uint64_t cols, uint64_t tokens) {
-    return tokens > 128 || cols >= 8192 || (rows + 255) / 256 >= 64;
+    const uint64_t tiles = (rows + 255) / 256, mt = (tokens + kSplitBM - 1) / kSplitBM;
+    // A deep K splits in at most eight: too few wide tiles leave CUs idle
+    // (37 tokens of 2560 x 10240: 80 blocks; 128-row tiles take an MLP branch of those rows from 153 to 141 us).
+    return tokens > 128 || tiles >= 64 || (cols >= 8192 && tiles * mt * 8 >= 160);
 }
 // Three K stages in registers ahead of the LDS stages (2 and 4 measured within
 // 1-4 % of it, either way, with three LDS buffers).
@@ -4296,6 +4299,25 @@ __global__ __launch_bounds__(kThreads) void copy_rows_kernel(const CopyRow *tabl
 hipError_t launch_copy_rows(hipStream_t stream, const CopyRow *table, uint32_t entries) {
     if (!entries) return hipSuccess;
     copy_rows_kernel<<<dim3(8, entries), kThreads, 0, stream>>>(table);
+    return hipGetLastError();
+}
+
+// One contiguous block, 16 bytes per thread: host rows staged in pinned memory
+// to the device and back. Bound by the bus (about 50 GB/s) and one round trip
+// over it; 64 blocks keep 256 KB in flight.
+__global__ __launch_bounds__(kThreads) void copy_block_kernel(const u32x4 *src, u32x4 *dst,
+                                                              uint64_t n) {
+    for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
+         i += (uint64_t)gridDim.x * kThreads)
+        dst[i] = src[i];
+}
+
+hipError_t launch_copy_block(hipStream_t stream, const void *src, void *dst, uint64_t bytes) {
+    if (!bytes) return hipSuccess;
+    if (bytes % 16 || ((uintptr_t)src & 15) || ((uintptr_t)dst & 15)) return hipErrorInvalidValue;
+    const uint64_t n = bytes / 16, blocks = std::min<uint64_t>((n + kThreads - 1) / kThreads, 64);
+    copy_block_kernel<<<(unsigned)blocks, kThreads, 0, stream>>>((const u32x4 *)src, (u32x4 *)dst,
+                                                                 n);
     return hipGetLastError();
 }
 

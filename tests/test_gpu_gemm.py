@@ -16,6 +16,8 @@ third term would leave a relative error near 1e-5, far above the 3e-6 allowed
 here for FP32 accumulation over 4096 terms.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -263,3 +265,36 @@ def test_prompt_pair_gemm(hidden, inter, tokens, std):
         gpu.close()
         cpu.close()
         syn.close()
+
+
+# Rows of plamo_metal_linear cross the bus through pinned staging memory up to
+# 32 MiB in and out and as the runtime's copies past it: strided rows, widths
+# that are not whole 16 bytes, and a call past the limit between two below it.
+@pytest.mark.parametrize("pad", [0, 5])
+def test_linear_host_rows(pad):
+    rng = np.random.default_rng(3)
+    be = plamo_hip.Backend()
+    resident = []  # a freed array's address must not come back
+    try:
+        for tokens, cols, rows in ((1, 70, 33), (3, 70, 33), (2100, 64, 4097), (1, 2048, 501),
+                                   (40, 328, 130)):
+            say(f"linear rows tokens={tokens} cols={cols} rows={rows} pad={pad}")
+            w = (rng.standard_normal((rows, cols)).astype(np.float32).view(np.uint32) >> 16)
+            w = w.astype(np.uint16)
+            resident.append(w)
+            x = rng.standard_normal((tokens, cols + pad), dtype=np.float32)
+            y = np.full((tokens, rows + pad), 7.0, np.float32)
+            assert be.preload(w.ctypes.data, w.nbytes) == 1
+            mm = plamo_hip.Matmul(w.ctypes.data_as(plamo_hip.u16p),
+                                  x.ctypes.data_as(plamo_hip.f32p),
+                                  y.ctypes.data_as(plamo_hip.f32p), rows, cols, tokens,
+                                  cols + pad, rows + pad)
+            assert be.lib.plamo_metal_linear(be.handle, ctypes.byref(mm)) == 1
+            wide = (w.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+            ref = x[:, :cols].astype(np.float64) @ wide.T
+            # FP32 sums of `cols` products: the rounding of each addition.
+            bound = 2.0 ** -24 * cols * (np.abs(x[:, :cols]) @ np.abs(wide).T)
+            assert np.all(np.abs(y[:, :rows] - ref) <= bound)
+            assert np.all(y[:, rows:] == 7.0)
+    finally:
+        be.close()
