@@ -974,6 +974,9 @@ bool device_failed(plamo_metal *m) {
 // ---------------------------------------------------------------- decode
 struct DecodePlan {
     std::vector<char> stale, shift;
+    // The rotated rows of windows that move cross to the (pinned) host arrays
+    // on copy_stream while later layers compute.
+    bool mirror = false;
     bool special = false;
     bool direct = false;  // host arrays written in place by the step itself
     // Nonzero: every layer's rows stay below this count for the step, and the
@@ -1023,6 +1026,7 @@ int encode_decode(plamo_metal *m, struct model *model, const DecodePlan &plan, i
     ++n;
     float *cur = m->state_a, *nxt = m->state_b;
     const int blocks = 2 * m->cus;
+    std::vector<uint64_t> moved;  // windows whose rotated rows are final, not yet mirrored
     for (uint64_t i = 0; i < L; ++i) {
         Layer &d = m->layers[i];
         const uint16_t *pre = d.norms, *post = d.norms + h, *mpre = d.norms + 2 * h,
@@ -1157,6 +1161,19 @@ int encode_decode(plamo_metal *m, struct model *model, const DecodePlan &plan, i
                                                as<float>(m->p_window), d.capacity, 1, d.capacity,
                                                d.kh, d.dim));
                 n += 2;
+            }
+        }
+        if (shift && plan.mirror) {
+            moved.push_back(i);
+            if (moved.size() == 4 || i + 4 >= L) {
+                HIP_TRY(m, hipEventRecord(m->layer_events[i], s));
+                HIP_TRY(m, hipStreamWaitEvent(m->copy_stream, m->layer_events[i], 0));
+                for (uint64_t j : moved)
+                    HIP_TRY(m, hipMemcpyAsync(model->layers[j]->mixer->rotation->out,
+                                              m->layers[j].rot,
+                                              m->layers[j].capacity * m->layers[j].width * 4,
+                                              hipMemcpyDeviceToHost, m->copy_stream));
+                moved.clear();
             }
         }
         if (!fused_o) {
@@ -1489,6 +1506,7 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
     m->params_host->step = m->step_tag;
     *m->status_host = 0;
     plan.direct = m->host_direct && !plan.special;
+    plan.mirror = m->host_direct;
     bool short_ctx = true;
     for (uint64_t i = 0; i < L && short_ctx; ++i)
         short_ctx = model->layers[i]->mixer->cache->count + 1 <= kDecodeShortRows;
@@ -1526,9 +1544,41 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
             return fail(m);
         }
     }
-    if (!end_timing(m)) return fail(m);
+    // The host arrays of full windows move on by one row while the GPU works
+    // (two C3 windows of 2049 rows: 16.8 MB, as long as the step itself). The
+    // rows that drop out are kept: a step that fails leaves them as they were.
+    std::vector<float> dropped;
+    for (uint64_t i = 0; i < L; ++i) {
+        if (!plan.shift[i]) continue;
+        const struct cache *c = model->layers[i]->mixer->cache;
+        for (float *rows : {c->k, c->v}) {
+            dropped.insert(dropped.end(), rows, rows + c->width);
+            memmove(rows, rows + c->width, (c->capacity - 1) * c->width * 4);
+        }
+    }
+    auto step_failed = [&]() {
+        const float *first = dropped.data();
+        for (uint64_t i = 0; i < L; ++i) {
+            if (!plan.shift[i]) continue;
+            struct mixer *mx = model->layers[i]->mixer;
+            const struct cache *c = mx->cache;
+            // The mirrored rotations may be the new ones: stale, to be rebuilt.
+            mx->rotation->processed_count = mx->rotation->scale_bits = 0;
+            for (float *rows : {c->k, c->v}) {
+                memmove(rows + c->width, rows, (c->capacity - 1) * c->width * 4);
+                memcpy(rows, first, c->width * 4);
+                first += c->width;
+            }
+        }
+        return fail(m);
+    };
+    if (!end_timing(m)) return step_failed();
     m->info.dispatches += dispatches;
-    if (device_failed(m)) return fail(m);
+    if (device_failed(m)) return step_failed();
+    if (plan.mirror && !dropped.empty() && hipStreamSynchronize(m->copy_stream) != hipSuccess) {
+        problem(m, "cannot mirror rotated keys");
+        return step_failed();
+    }
     // Host mirror (runtime/metal_model.m:491-500); a direct step has written
     // logits, state, normalized and the new rows in place already.
     const float *out = m->outbox_host;
@@ -1545,17 +1595,15 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
         struct rotation *r = mx->rotation;
         const float *st = stage + i * 3 * m->max_width;
         uint64_t row = c->count;
-        if (plan.shift[i]) {
-            memmove(c->k, c->k + c->width, (c->capacity - 1) * c->width * 4);
-            memmove(c->v, c->v + c->width, (c->capacity - 1) * c->width * 4);
-            row = c->capacity - 1;
-        }
+        if (plan.shift[i]) row = c->capacity - 1;
         if (!plan.direct) {
             memcpy(c->k + row * c->width, st, c->width * 4);
             memcpy(c->v + row * c->width, st + c->width, c->width * 4);
         }
         uint64_t count = row + 1;
-        if (plan.shift[i] || plan.stale[i]) {
+        if (plan.shift[i] && plan.mirror) {
+            // on the host already
+        } else if (plan.shift[i] || plan.stale[i]) {
             if (hipMemcpy(r->out, d.rot, count * c->width * 4, hipMemcpyDeviceToHost) != hipSuccess) {
                 problem(m, "cannot mirror rotated keys");
                 return fail(m);
