@@ -165,7 +165,7 @@ struct plamo_metal {
     // Prompt / candidate workspace (grown on demand).
     uint64_t prompt_rows = 0;
     Buffer p_state, p_norm, p_qkv, p_q, p_attn, p_branch, p_gu, p_act, p_side_k, p_side_v,
-        p_ids, p_window, p_logits, p_attn_split, p_virtual;
+        p_ids, p_window, p_logits, p_attn_split, p_virtual, p_kv_pairs;
     uint32_t *ids_host = nullptr;
     // Candidate results kept for commit.
     float *v_state = nullptr, *v_norm = nullptr, *v_logits = nullptr, *v_prop = nullptr;
@@ -1656,7 +1656,9 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     // wide[i]: the rows overflow a sliding window and the matrix-core
     // attention takes the layer, over keys rotated at their virtual rows.
     std::vector<char> overflow(L, 0), wide(L, 0);
-    uint64_t split_floats = 0, virtual_floats = 0;
+    // paired[i]: the layer's attention runs on fp16 pairs and writes O's input.
+    std::vector<char> paired(L, 0);
+    uint64_t split_floats = 0, virtual_floats = 0, pair_bytes = 0;
     for (uint64_t i = 0; i < L; ++i) {
         const Layer &d = m->layers[i];
         const struct cache *c = model->layers[i]->mixer->cache;
@@ -1666,9 +1668,15 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             if (!ensure_exact_rows(m, m->ropes[d.rope], c->count + T)) return -1;
             virtual_floats = std::max(virtual_floats, (c->count + T) * d.width);
         }
-        split_floats = std::max(split_floats,
-                                prompt_attention_scratch((uint32_t)c->count, (uint32_t)T, d.qh,
-                                                         d.kh, d.dim, window, wide[i]));
+        paired[i] = pair && (!window || wide[i]) &&
+                    pair_attention_supported((uint32_t)c->count, (uint32_t)T, d.qh, d.kh, d.dim);
+        if (paired[i])
+            pair_bytes = std::max(pair_bytes, pair_attention_scratch((uint32_t)c->count,
+                                                                     (uint32_t)T, d.kh, d.dim));
+        else
+            split_floats = std::max(split_floats,
+                                    prompt_attention_scratch((uint32_t)c->count, (uint32_t)T, d.qh,
+                                                             d.kh, d.dim, window, wide[i]));
         // The last layer's attention may run for its last row alone.
         if (i + 1 == L)
             split_floats = std::max(split_floats,
@@ -1676,6 +1684,11 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                                                              d.kh, d.dim, window, wide[i]));
     }
     if (split_floats && !ensure(m, m->p_attn_split, split_floats * 4)) return -1;
+    // The V exponents of every layer's KV heads, after the scratch.
+    uint64_t heads = 0;
+    for (const Layer &d : m->layers) heads += d.kh;
+    pair_bytes = (pair_bytes + 255) / 256 * 256;
+    if (pair_bytes && !ensure(m, m->p_kv_pairs, pair_bytes + heads * 4)) return -1;
     if (virtual_floats && !ensure(m, m->p_virtual, virtual_floats * 4)) return -1;
     for (uint64_t i = 0; i < L; ++i) {
         Layer &d = m->layers[i];
@@ -1700,6 +1713,11 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     HIP_FAIL(m, launch_embed(s, m->embedding, as<uint32_t>(m->p_ids), nullptr, (uint32_t)T,
                             (uint32_t)h, state));
     ++n;
+    int32_t *v_exp = (int32_t *)(as<char>(m->p_kv_pairs) + pair_bytes);
+    if (pair_bytes) {
+        HIP_FAIL(m, launch_fill(s, (uint32_t *)v_exp, heads, (uint32_t)kPairNoExp));
+        ++n;
+    }
     // A residual followed by a norm of the same rows runs as one launch; then
     // `normed` says the next layer's input norm is already in `norm`.
     const bool fuse_rows = h <= 8192;
@@ -1844,8 +1862,13 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             pa.prefix += (uint32_t)(T - 1);
             pa.tokens = 1;
         }
-        HIP_FAIL(m, launch_prompt_attention(s, pa));
-        ++n;
+        const bool on_pairs = paired[i] && !last_query;
+        if (on_pairs)
+            HIP_FAIL(m, launch_pair_attention(s, pa, m->p_kv_pairs.ptr, v_exp, in));
+        else
+            HIP_FAIL(m, launch_prompt_attention(s, pa));
+        v_exp += d.kh;
+        n += on_pairs ? 2 : 1;
         if (overflow[i] && !verify) {
             HIP_FAIL(m, launch_window_store(s, d.k, d.v, d.rot, as<float>(m->p_side_k),
                                            as<float>(m->p_side_v), d.width, rope.table,
@@ -1920,10 +1943,9 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             n += 3;
         } else {
             if (pair) {
-                // rows == T: `in` is sized for them. The attention rows become
-                // planes in a launch of their own (their scale is not known
-                // while the heads are computed); the rows' activation goes
-                // past the input planes, which gate/up's blocks still read.
+                // rows == T: `in` is sized for them. Attention rows in FP32
+                // become planes in a launch of their own; the rows' activation
+                // goes past the input planes, which gate/up's blocks still read.
                 PairRows act{};
                 act.planes = ws->planes + 2 * (uint64_t)in.padded * h;
                 act.exps = m->pair_exps + kMaxPrompt + 128;
@@ -1931,7 +1953,8 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                 PairRows gu_in = in;
                 gu_in.norms = d.gu_norms;
                 gu_in.act_exps = act.exps;
-                HIP_FAIL(m, launch_norm_rows(s, attn, aw, nullptr, 0.0f, attn, aw, aw, T, &in));
+                if (!on_pairs)
+                    HIP_FAIL(m, launch_norm_rows(s, attn, aw, nullptr, 0.0f, attn, aw, aw, T, &in));
                 HIP_FAIL(m, launch_gemm_pair(s, in, d.p_o, T, branch, h, *ws));
                 HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, post, kAttentionOffset, mpre,
                                                      1.0f, norm, h, h, T, &gu_in));

@@ -270,6 +270,17 @@ bool prompt_attention_matrix(uint32_t dim, uint32_t qh, uint32_t kh);
 uint64_t prompt_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t qh, uint32_t kh,
                                   uint32_t dim, uint32_t window, int rotated);
 
+// The same attention on the fp16 matrix cores for prompts of more than 32
+// tokens, written as the O projection's input planes. scratch:
+// pair_attention_scratch bytes (256-byte aligned); v_exp: kh words set to
+// kPairNoExp. With a window the keys are rotated at their virtual rows.
+constexpr int32_t kPairNoExp = 126;
+bool pair_attention_supported(uint32_t prefix, uint32_t tokens, uint32_t qh, uint32_t kh,
+                              uint32_t dim);
+uint64_t pair_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t kh, uint32_t dim);
+hipError_t launch_pair_attention(hipStream_t, const PromptAttention &, void *scratch,
+                                 int32_t *v_exp, const PairRows &out);
+
 // Rotates cache rows [0, rows) of raw K into rotated K at their row position.
 hipError_t launch_rerotate(hipStream_t, const float *k_raw, float *k_rot, const float *table,
                            uint64_t rows, uint32_t kh, uint32_t dim);

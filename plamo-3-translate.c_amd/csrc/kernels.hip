@@ -4217,6 +4217,406 @@ hipError_t launch_prompt_attention(hipStream_t stream, const PromptAttention &a)
     return hipGetLastError();
 }
 
+// ---------------------------------------------------------------- prompt attention on fp16 pairs
+// The causal (and windowed) attention of a prompt's layer, S = K Q^T and
+// O = V^T P on the fp16 matrix cores: every operand is a scaled pair of fp16
+// terms as in the fp16-pair GEMM, of whose products hi hi, hi lo and lo hi are
+// taken (lo lo is below 2^-22 of the product); sums are FP32. The FP32 matrix
+// cores do a sixteenth of the fp16 rate, so three products leave a fifth of
+// the time. Against 64-bit results of the layers the error is the same.
+//
+// pair_kv_kernel first turns the layer's visible rows, 32 keys of one KV head
+// per block, into MFMA fragments (K and V^T, hi and lo) with one power of two
+// per tile each. The attention block is four waves, each 32 queries of one
+// head of the KV head's group; the waves share the tile in LDS (double
+// buffered, loaded straight into it). S is formed transposed (keys by
+// queries), so a lane holds 16 keys of one query: the softmax needs one
+// exchange between lane halves per tile, and its values are, in place, the
+// B operand of V^T P (the keys of a fragment are permuted to match). Blocks
+// with the most keys are dispatched first; there are no key splits: the
+// output goes out once, as the O projection's input planes.
+//
+// Bound by what a wave does for a tile (48 products of 32 cycles, about 500
+// vector instructions around them) and by the causal triangle, whose longest
+// blocks end the launch. Measured per layer with pair_kv, against the FP32
+// form with its merge and the planes launch: 32/8 heads of 128 at 1900 tokens
+// 175 against 474 us, 443 tokens 40 against 60, 116 tokens 22 against 23;
+// 16/4 heads, 3500 tokens in a 2048 window, 187 against 701.
+constexpr uint32_t kPairKeys = 32;  // keys per tile
+constexpr int pair_kv_frags(int dim) { return dim / 16 * 2 * 2; }  // 1 KB fragments of K and V
+
+struct PairAttention {
+    PromptAttention a;
+    uint16_t *kv;      // [kh][tiles][K fragments | V fragments]
+    int32_t *kv_exps;  // [kh][tiles][K, V]
+    int32_t *v_exp;    // [kh]: the smallest V exponent (of the largest values)
+    uint32_t tiles;
+    PairRows out;
+};
+
+template <int DIM>
+__global__ __launch_bounds__(kThreads) void pair_kv_kernel(PairAttention p) {
+    __shared__ float red[2][4];
+    const PromptAttention &a = p.a;
+    const uint32_t tile = blockIdx.x, kvh = blockIdx.y, width = a.kh * DIM;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t total = a.prefix + a.tokens, k0 = tile * kPairKeys;
+    auto row_of = [&](const float *cache, const float *fresh, uint32_t key) {
+        const uint32_t r = min(key, total - 1);
+        return (r < a.cached ? cache + (uint64_t)r * width : fresh + (uint64_t)(r - a.cached) * width) +
+               (uint64_t)kvh * DIM;
+    };
+    // K: (key, 8 columns) per item; V: (column, 8 keys of a fragment's half).
+    constexpr int N = kPairKeys * DIM / 8 / kThreads;
+    float kx[N][8], vx[N][8];
+    float km = 0.0f, vm = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const uint32_t item = threadIdx.x + kThreads * i;
+        const uint32_t key = item / (DIM / 8), c = item % (DIM / 8) * 8;
+        const float *kr = row_of(a.k_cache, a.k_new, k0 + key) + c;
+        const f32x4 lo4 = *(const f32x4 *)kr, hi4 = *(const f32x4 *)(kr + 4);
+        const uint32_t d = item % DIM, kk = item / DIM / 2, h = item / DIM % 2;
+        const bool live = k0 + key < total;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            kx[i][e] = live ? (e < 4 ? lo4[e] : hi4[e - 4]) : 0.0f;
+            const uint32_t vk = k0 + 16 * kk + 8 * (e / 4) + 4 * h + e % 4;
+            const float v = row_of(a.v_cache, a.v_new, vk)[d];
+            vx[i][e] = vk < total ? v : 0.0f;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            km = fmaxf(km, __builtin_fabsf(kx[i][e]));
+            vm = fmaxf(vm, __builtin_fabsf(vx[i][e]));
+        }
+    }
+    km = wave_max(km);
+    vm = wave_max(vm);
+    if (lane == 0) {
+        red[0][wave] = km;
+        red[1][wave] = vm;
+    }
+    __syncthreads();
+    km = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    vm = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
+    const int ke = pair_exponent(__float_as_uint(km)), ve = pair_exponent(__float_as_uint(vm));
+    const float ks = power_of_two(ke), vs = power_of_two(ve);
+    if (threadIdx.x == 0) {
+        p.kv_exps[(kvh * p.tiles + tile) * 2] = ke;
+        p.kv_exps[(kvh * p.tiles + tile) * 2 + 1] = ve;
+        (void)__hip_atomic_fetch_min(p.v_exp + kvh, ve, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    uint16_t *frag = p.kv + (uint64_t)(kvh * p.tiles + tile) * pair_kv_frags(DIM) * 512;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const uint32_t item = threadIdx.x + kThreads * i;
+        const uint32_t key = item / (DIM / 8), cg = item % (DIM / 8);
+        const uint32_t d = item % DIM, kk = item / DIM / 2, h = item / DIM % 2;
+        f16x8 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            _Float16 x, y;
+            pair_split(kx[i][e], ks, x, y);
+            hi[e] = x;
+            lo[e] = y;
+        }
+        uint16_t *kf = frag + (cg / 2 * 2 * 64 + key + 32 * (cg % 2)) * 8;
+        *(f16x8 *)kf = hi;
+        *(f16x8 *)(kf + 512) = lo;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            _Float16 x, y;
+            pair_split(vx[i][e], vs, x, y);
+            hi[e] = x;
+            lo[e] = y;
+        }
+        uint16_t *vf = frag + (DIM / 16 * 2 + (d / 32 * 2 + kk) * 2) * 512 + (d % 32 + 32 * h) * 8;
+        *(f16x8 *)vf = hi;
+        *(f16x8 *)(vf + 512) = lo;
+    }
+}
+
+// KW groups of four waves take the key tiles in turn, their results are merged
+// at the end: with few blocks a tile's chain of products, softmax and products
+// is what the launch waits for.
+template <int DIM, int KW>
+__global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void pair_attention_kernel(PairAttention p) {
+    constexpr int KS = DIM / 16, NT = DIM / 32, FR = pair_kv_frags(DIM), PW = FR / 4;
+    extern __shared__ u32x4 lds[];  // [2][KW][FR][64]
+    const PromptAttention &a = p.a;
+    const uint32_t lane = threadIdx.x & 63, col = lane & 31, hf = lane >> 5;
+    const uint32_t waves = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wave = waves % 4, part = waves / 4;
+    const uint32_t group = a.qh / a.kh, kvh = blockIdx.x;
+    const uint32_t units = (a.tokens + 31) / 32 * group;  // (query tile, head of the group)
+    const uint32_t block = gridDim.y - 1 - blockIdx.y;
+    // Key tiles of a query tile: [lo, hi).
+    auto tile_lo = [&](uint32_t qt) -> uint32_t {
+        const uint32_t seen = a.prefix + qt * 32 + 1;
+        return a.window && seen > a.window ? (seen - a.window) / kPairKeys : 0;
+    };
+    auto tile_hi = [&](uint32_t qt) -> uint32_t {
+        return (a.prefix + min(qt * 32 + 32, a.tokens) + kPairKeys - 1) / kPairKeys;
+    };
+    const uint32_t unit = block * 4 + wave;
+    const bool busy = unit < units;
+    const uint32_t qt = min(unit, units - 1) / group, h = kvh * group + min(unit, units - 1) % group;
+    const uint32_t t0 = qt * 32, lo = tile_lo(qt), hi = tile_hi(qt);
+    const uint32_t first = tile_lo(block * 4 / group);
+    const uint32_t last = tile_hi(min(block * 4 + 3, units - 1) / group);
+    const uint32_t token = t0 + col;
+    const u32x4 *kv = (const u32x4 *)p.kv + (uint64_t)kvh * p.tiles * FR * 64 + lane;
+    const int32_t *exps = p.kv_exps + (uint64_t)kvh * p.tiles * 2;
+    // The KW tiles from `tile` on, each by its group (past the last: that again).
+    auto load = [&](uint32_t tile, uint32_t buf) -> int {
+        const uint32_t t = min(tile + part, last - 1);
+#pragma unroll
+        for (int i = 0; i < PW; ++i)
+            __builtin_amdgcn_global_load_lds(
+                (const void *)(kv + ((uint64_t)t * FR + wave + 4 * i) * 64),
+                (__attribute__((address_space(3))) void *)(lds + ((buf * KW + part) * FR + wave + 4 * i) * 64),
+                16, 0, 0);
+        // The tile's K exponent in even lanes, V's in odd ones.
+        return exps[t * 2 + (lane & 1)];
+    };
+    int te = load(first, 0);
+    const int v_exp = p.v_exp[kvh];
+    // Q as the B operand of each 16-column step, scaled per query.
+    f16x8 qhi[KS], qlo[KS];
+    int qe;
+    {
+        const float *qrow = a.q + (uint64_t)min(token, a.tokens - 1) * a.qh * DIM + (uint64_t)h * DIM;
+        float mx = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const f32x4 x = *(const f32x4 *)(qrow + 16 * s + 8 * hf);
+            const f32x4 y = *(const f32x4 *)(qrow + 16 * s + 8 * hf + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                mx = fmaxf(mx, fmaxf(__builtin_fabsf(x[e]), __builtin_fabsf(y[e])));
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        qe = pair_exponent(__float_as_uint(mx));
+        const float scale = power_of_two(qe);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const f32x4 x = *(const f32x4 *)(qrow + 16 * s + 8 * hf);
+            const f32x4 y = *(const f32x4 *)(qrow + 16 * s + 8 * hf + 4);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                _Float16 u, v;
+                pair_split(e < 4 ? x[e] : y[e - 4], scale, u, v);
+                qhi[s][e] = u;
+                qlo[s][e] = v;
+            }
+        }
+    }
+    // Scores in base 2: s * log2(e) / sqrt(d).
+    const float base = 1.4426950408889634f / __builtin_sqrtf((float)DIM);
+    const float ninf = -__builtin_inff();
+    f32x16 o[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[n][v] = 0.0f;
+    float m_run = ninf, l_run = 0.0f;
+    loads_landed<0>();
+    for (uint32_t t = first, buf = 0; t < last; t += KW, buf ^= 1) {
+        const int ke = __builtin_amdgcn_readlane(te, 0), ve = __builtin_amdgcn_readlane(te, 1);
+        if (t + KW < last) te = load(t + KW, buf ^ 1);
+        const uint32_t tile = t + part;
+        if (busy && tile >= lo && tile < hi) {
+            const u32x4 *kf = lds + (buf * KW + part) * FR * 64 + lane, *vf = kf + KS * 2 * 64;
+            f32x16 sh, sl, sm;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sh[v] = sl[v] = sm[v] = 0.0f;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const f16x8 ah = __builtin_bit_cast(f16x8, kf[s * 2 * 64]);
+                const f16x8 al = __builtin_bit_cast(f16x8, kf[(s * 2 + 1) * 64]);
+                sh = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, qhi[s], sh, 0, 0, 0);
+                sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, qlo[s], sl, 0, 0, 0);
+                sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, qhi[s], sm, 0, 0, 0);
+            }
+            // Lane: query `col`; value v: key 8 (v / 4) + 4 hf + v % 4.
+            const uint32_t seen = a.prefix + token + 1, key0 = tile * kPairKeys + 4 * hf;
+            const uint32_t from = a.window && seen > a.window ? seen - a.window : 0;
+            const float scale = __builtin_ldexpf(base, -(ke + qe));
+            float mx = ninf;
+            const bool whole = tile * kPairKeys + kPairKeys <= a.prefix + t0 + 1 &&
+                               (!a.window || a.prefix + t0 + 32 <= a.window + tile * kPairKeys);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const uint32_t key = key0 + 8 * (v / 4) + v % 4;
+                float x = (sh[v] + (sl[v] + sm[v])) * scale;
+                if (!whole) x = key < seen && key >= from ? x : ninf;
+                sh[v] = x;
+                mx = fmaxf(mx, x);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float m_new = fmaxf(m_run, mx);
+            if (__builtin_amdgcn_ballot_w64(m_new != m_run)) {
+                // A query that has seen no key keeps zeros.
+                const float c = m_new == ninf ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+                l_run *= c;
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) o[n][v] *= c;
+                m_run = m_new;
+            }
+            const float mm = m_run == ninf ? 0.0f : m_run;
+            // P scaled to 2^14 and to this tile's V exponent.
+            const float ps = power_of_two(max(14 + v_exp - ve, -126));
+            f16x8 phi[2], plo[2];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float pv = __builtin_amdgcn_exp2f(sh[v] - mm);
+                l_run += pv;
+                _Float16 u, w;
+                pair_split(pv, ps, u, w);
+                phi[v / 8][v % 8] = u;
+                plo[v / 8][v % 8] = w;
+            }
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                f16x8 ah[NT], al[NT];
+#pragma unroll
+                for (int n = 0; n < NT; ++n) {
+                    ah[n] = __builtin_bit_cast(f16x8, vf[(n * 2 + kk) * 2 * 64]);
+                    al[n] = __builtin_bit_cast(f16x8, vf[((n * 2 + kk) * 2 + 1) * 64]);
+                }
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    o[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[n], phi[kk], o[n], 0, 0, 0);
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    o[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[n], plo[kk], o[n], 0, 0, 0);
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    o[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[n], phi[kk], o[n], 0, 0, 0);
+            }
+        }
+        loads_landed<0>();
+    }
+    float l = l_run + __shfl_xor(l_run, 32, 64);
+    if constexpr (KW == 2) {
+        // The second group's sums through LDS (every load has landed and every
+        // tile is done): [wave][16 NT + 2][64].
+        float *x = (float *)lds + wave * (16 * NT + 2) * 64 + lane;
+        if (part) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) x[(16 * n + v) * 64] = o[n][v];
+            x[16 * NT * 64] = m_run;
+            x[(16 * NT + 1) * 64] = l;
+        }
+        __syncthreads();
+        if (part) return;
+        const float m1 = x[16 * NT * 64], m = fmaxf(m_run, m1);
+        const float c0 = m_run == ninf ? 0.0f : __builtin_amdgcn_exp2f(m_run - m);
+        const float c1 = m1 == ninf ? 0.0f : __builtin_amdgcn_exp2f(m1 - m);
+        l = l * c0 + x[(16 * NT + 1) * 64] * c1;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[n][v] = o[n][v] * c0 + x[(16 * n + v) * 64] * c1;
+    }
+    if (!busy || token >= a.tokens) return;
+    // An output is a mean of V rows: below 2^(15 - v_exp) for every head, so
+    // the smallest V exponent of the KV heads scales the row for the O GEMM.
+    int re = v_exp;
+    for (uint32_t k = 0; k < a.kh; ++k) re = min(re, p.v_exp[k]);
+    if (h == 0 && hf == 0) p.out.exps[token] = re;
+    const float rs = power_of_two(re), inv = power_of_two(-14);
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            f16x4 ph, pl;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float y = __builtin_ldexpf(o[n][v + e] * inv, -v_exp) / l;
+                _Float16 u, w;
+                pair_split(y, rs, u, w);
+                ph[e] = u;
+                pl[e] = w;
+            }
+            const uint64_t at = pair_at(p.out.padded, token, h * DIM + 32 * n + 2 * v + 4 * hf);
+            *(u32x2 *)(p.out.planes + at) = __builtin_bit_cast(u32x2, ph);
+            *(u32x2 *)(p.out.planes + at + (uint64_t)p.out.padded * kPairK) =
+                __builtin_bit_cast(u32x2, pl);
+        }
+}
+
+template <int DIM>
+static hipError_t pair_attention_variant(hipStream_t stream, const PairAttention &p, dim3 grid,
+                                         bool two) {
+    constexpr size_t lds = 2 * (size_t)pair_kv_frags(DIM) * 1024;
+    if (!two) {
+        pair_attention_kernel<DIM, 1><<<grid, 256, lds, stream>>>(p);
+        return hipGetLastError();
+    }
+    static bool attr = false;
+    if (!attr) {
+        hipError_t e = hipFuncSetAttribute((const void *)pair_attention_kernel<DIM, 2>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)(2 * lds));
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    pair_attention_kernel<DIM, 2><<<grid, 512, 2 * lds, stream>>>(p);
+    return hipGetLastError();
+}
+
+static uint32_t pair_kv_tiles(uint32_t prefix, uint32_t tokens) {
+    return (prefix + tokens + kPairKeys - 1) / kPairKeys;
+}
+
+// From 33 tokens, unless a long cached prefix outweighs them: one block walks
+// its queries' keys alone, where the FP32 form spreads them over splits.
+bool pair_attention_supported(uint32_t prefix, uint32_t tokens, uint32_t qh, uint32_t kh,
+                              uint32_t dim) {
+    return tokens > 32 && prefix <= 4 * tokens && kh && qh % kh == 0 && (dim == 64 || dim == 128) &&
+           (qh * dim) % kPairK == 0 && kh <= 65535;
+}
+
+uint64_t pair_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t kh, uint32_t dim) {
+    const uint64_t tiles = (uint64_t)kh * pair_kv_tiles(prefix, tokens);
+    return tiles * pair_kv_frags((int)dim) * 1024 + tiles * 8;
+}
+
+hipError_t launch_pair_attention(hipStream_t stream, const PromptAttention &a, void *scratch,
+                                 int32_t *v_exp, const PairRows &out) {
+    if (!pair_attention_supported(a.prefix, a.tokens, a.qh, a.kh, a.dim) || out.padded < a.tokens ||
+        (a.window && !a.rotated))
+        return hipErrorInvalidValue;
+    PairAttention p{};
+    p.a = a;
+    p.tiles = pair_kv_tiles(a.prefix, a.tokens);
+    p.kv = (uint16_t *)scratch;
+    p.kv_exps = (int32_t *)((char *)scratch +
+                            (uint64_t)a.kh * p.tiles * pair_kv_frags((int)a.dim) * 1024);
+    p.v_exp = v_exp;
+    p.out = out;
+    const uint32_t units = (a.tokens + 31) / 32 * (a.qh / a.kh);
+    const dim3 prep(p.tiles, a.kh), grid(a.kh, (units + 3) / 4);
+    if (grid.y > 65535) return hipErrorInvalidValue;
+    if (a.dim == 64)
+        pair_kv_kernel<64><<<prep, kThreads, 0, stream>>>(p);
+    else
+        pair_kv_kernel<128><<<prep, kThreads, 0, stream>>>(p);
+    // Two groups of waves while one block per CU holds every block: 443 tokens
+    // (112 blocks) 34 us against 39 with one. Past that a second block fills
+    // the CU as well: 3500 windowed tokens (440 blocks) 175 us with one group,
+    // 197 with two.
+    const bool two = (uint64_t)grid.x * grid.y <= 256;
+    return a.dim == 64 ? pair_attention_variant<64>(stream, p, grid, two)
+                       : pair_attention_variant<128>(stream, p, grid, two);
+}
+
 // ---------------------------------------------------------------- rotation maintenance
 __global__ __launch_bounds__(kThreads) void rerotate_kernel(const float *k_raw, float *k_rot,
                                                             const float *table, uint64_t rows,

@@ -324,6 +324,40 @@ def test_eager_decode_matches_graph(monkeypatch):
         assert np.array_equal(x, y)
 
 
+# The fp16-pair prompt attention without a window: groups whose (query tile,
+# head) units leave waves of a block idle, prompts of one tile and a row, of
+# whole tiles, a prefix of four prompts (its limit) and one past it, and grids
+# of more than one block per CU (one group of waves per block instead of two).
+@pytest.mark.parametrize("qh,kh,dim,prefix,tokens", [
+    (6, 3, 128, 0, 33), (6, 1, 64, 0, 65), (4, 4, 64, 160, 40), (4, 4, 64, 161, 40),
+    (3, 3, 64, 5, 129), (16, 1, 128, 7, 96), (32, 32, 64, 0, 1030), (16, 4, 128, 3, 2050),
+])
+def test_prompt_pair_attention(qh, kh, dim, prefix, tokens):
+    say(f"pair attention {qh}/{kh}x{dim} prefix={prefix} tokens={tokens}")
+    syn = plamo_hip.Synthetic(256, 2, qh, kh, dim, 96, 300, window=2304, global_capacity=2304,
+                              pattern=2, embedding_std=1.0, seed=77)
+    gpu, cpu = syn.instance(), syn.instance()
+    be = plamo_hip.Backend(syn)
+    try:
+        ids = [(j * 13 + 5) % 300 for j in range(prefix + tokens)]
+        for part in (ids[:prefix], ids[prefix:]):
+            if not part:
+                continue
+            actual = np.zeros((len(part), 256), np.float32)
+            expected = np.zeros((len(part), 256), np.float32)
+            assert be.prefill(gpu, part, actual) == 1
+            assert oracle_lib.prefill(cpu, part, expected)
+            gate(actual, expected, "all prompt states")
+            compare(gpu, cpu)
+        info = be.info()
+        assert info.errors == 0 and info.cpu_fallbacks == 0, info.note.decode()
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
+
+
 # Prompts, decode steps and candidates past a sliding window at the head dims
 # and groups of the matrix-core prompt attention and the fused decode
 # attention: windows of less and more than a key tile (32) and an attention
