@@ -358,6 +358,33 @@ def test_prompt_pair_attention(qh, kh, dim, prefix, tokens):
         syn.close()
 
 
+# Decode steps whose contexts take 16, 17, 32 and 33 splits, at the edges of the
+# merging block's batches (16 partials, 32 maxima).
+@pytest.mark.parametrize("rows", [1022, 1086, 2046, 2110])
+def test_decode_split_merge(rows):
+    say(f"split merge rows={rows}")
+    syn = plamo_hip.Synthetic(256, 1, 16, 4, 128, 96, 300, window=2304, global_capacity=2304,
+                              pattern=1, embedding_std=1.0, seed=31)
+    gpu, cpu = syn.instance(), syn.instance()
+    be = plamo_hip.Backend(syn)
+    try:
+        ids = [(j * 13 + 5) % 300 for j in range(rows)]
+        states = np.zeros((rows, 256), np.float32)
+        assert be.prefill(gpu, ids, states) == 1
+        assert oracle_lib.prefill(cpu, ids, states)
+        for token in (7, 11, 2, 290):
+            assert be.forward(gpu, token) == 1
+            assert oracle_lib.forward(cpu, token)
+            compare(gpu, cpu)
+        info = be.info()
+        assert info.errors == 0 and info.cpu_fallbacks == 0, info.note.decode()
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
+
+
 # Prompts, decode steps and candidates past a sliding window at the head dims
 # and groups of the matrix-core prompt attention and the fused decode
 # attention: windows of less and more than a key tile (32) and an attention
