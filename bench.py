@@ -35,10 +35,11 @@ sys.path.insert(0, str(ROOT / "plamo-3-translate.c_amd"))
 import plamo_hip  # noqa: E402
 
 HBM_PEAK_GBPS = 8000.0        # MI355X HBM3E
-FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix
-# The prompt GEMM runs exact FP32 products as three BF16 passes on the
-# 2.5 PFLOP/s BF16 matrix cores: its own ceiling is a third of that.
-SPLIT_BF16_CEILING_TFLOPS = round(2500.0 / 3, 1)
+# A prompt's FP32 values run as scaled pairs of fp16 terms on the 2.5 PFLOP/s
+# fp16 matrix cores: two products per weight (a weight is one term), three per
+# attention product (of two pairs). The ceilings are a half and a third of that.
+PAIR_GEMM_CEILING_TFLOPS = 1250.0
+PAIR_ATTENTION_CEILING_TFLOPS = round(2500.0 / 3, 1)
 PREFIX = 12                   # fixed translation-template prefix (runtime/engine.c:358-381)
 
 
@@ -95,12 +96,12 @@ def prefill_flop(cfg: dict, prefix: int, tokens: int) -> float:
 
 def prefill_roofline(cfg: dict, prefix: int, tokens: int, ttft_ms: float) -> dict:
     """The prefill against the ceilings of the instructions it runs: the
-    projections on the BF16 matrix cores with three products per FP32 input
-    (2.5 PFLOP/s / 3), attention on the FP32 matrix cores (157.3 TFLOP/s),
-    and the weights crossing HBM once (8 TB/s) as a floor."""
+    projections on the fp16 matrix cores with two products per weight
+    (2.5 PFLOP/s / 2), attention with three (2.5 PFLOP/s / 3), and the weights
+    crossing HBM once (8 TB/s) as a floor."""
     linear, attention = prefill_flop_parts(cfg, prefix, tokens)
-    mfma_ms = (linear / (SPLIT_BF16_CEILING_TFLOPS * 1e12) +
-               attention / (FP32_MFMA_PEAK_TFLOPS * 1e12)) * 1e3
+    mfma_ms = (linear / (PAIR_GEMM_CEILING_TFLOPS * 1e12) +
+               attention / (PAIR_ATTENTION_CEILING_TFLOPS * 1e12)) * 1e3
     hbm_ms = plamo_hip.weight_bytes_per_step(cfg) / (HBM_PEAK_GBPS * 1e9) * 1e3
     bound_ms = max(mfma_ms, hbm_ms)
     flop = linear + attention
@@ -109,8 +110,8 @@ def prefill_roofline(cfg: dict, prefix: int, tokens: int, ttft_ms: float) -> dic
             "mfma_bound_ms": round(mfma_ms, 3), "hbm_bound_ms": round(hbm_ms, 3),
             "bound": "mfma" if mfma_ms >= hbm_ms else "hbm",
             "frac": round(bound_ms / ttft_ms, 4),
-            "note": "frac = max(linear / 833.3 TFLOP/s (split BF16) + attention / 157.3 TFLOP/s "
-                    "(FP32 MFMA), weights / 8 TB/s) / TTFT"}
+            "note": "frac = max(linear / 1250 TFLOP/s (fp16 pairs) + attention / 833.3 TFLOP/s "
+                    "(fp16 pairs), weights / 8 TB/s) / TTFT"}
 
 
 def host_threads() -> tuple[int, int]:
