@@ -168,12 +168,12 @@ struct plamo_metal {
         p_ids, p_window, p_logits, p_attn_split, p_virtual, p_kv_pairs;
     uint32_t *ids_host = nullptr;
     // Candidate results kept for commit.
-    float *v_state = nullptr, *v_norm = nullptr, *v_logits = nullptr, *v_prop = nullptr;
+    float *v_norm = nullptr, *v_logits = nullptr, *v_prop = nullptr;
     float *v_host = nullptr;  // pinned: states | normalized | logits | proposals
     bool prop_on_host = true;  // the last verify copied its proposals into v_host
     uint32_t *v_next = nullptr, *v_next_host = nullptr;
     void *v_argmax = nullptr;  // argmax partials of the candidate logits
-    CopyRow *copy_table = nullptr, *copy_table_host = nullptr;
+    CopyRow *copy_table_host = nullptr;  // pinned, read by the commit's kernel
     CopyRow *upload_table = nullptr;  // pinned: host-to-device rows of sync_from_host
     const CopyRow *upload_view = nullptr;  // its device view
     uint64_t verification_tokens = 0, verification_index = 0;
@@ -366,10 +366,10 @@ int add_range(plamo_metal *m, const void *host, uint64_t bytes) {
 }
 
 // ---------------------------------------------------------------- model setup
-// Candidate buffers of verify/commit. All or nothing: v_state is set only
+// Candidate buffers of verify/commit. All or nothing: v_host is set only
 // when every buffer exists, so a later call never runs on a partial set.
 void free_verify(plamo_metal *m) {
-    for (float **p : {&m->v_state, &m->v_norm, &m->v_logits, &m->v_prop}) {
+    for (float **p : {&m->v_norm, &m->v_logits, &m->v_prop}) {
         dev_free(m, *p);
         *p = nullptr;
     }
@@ -377,8 +377,6 @@ void free_verify(plamo_metal *m) {
     m->v_next = nullptr;
     dev_free(m, m->v_argmax);
     m->v_argmax = nullptr;
-    dev_free(m, m->copy_table);
-    m->copy_table = nullptr;
     if (m->v_host) (void)hipHostFree(m->v_host);
     if (m->v_next_host) (void)hipHostFree(m->v_next_host);
     if (m->copy_table_host) (void)hipHostFree(m->copy_table_host);
@@ -389,15 +387,12 @@ void free_verify(plamo_metal *m) {
 
 bool alloc_verify(plamo_metal *m, uint64_t L, uint64_t h, uint64_t V) {
     const uint64_t prop = L * 3 * kMaxVerify * m->max_width;
-    float *state = dev_alloc<float>(m, kMaxVerify * h);
     m->v_norm = dev_alloc<float>(m, kMaxVerify * h);
     m->v_logits = dev_alloc<float>(m, kMaxVerify * V);
     m->v_prop = dev_alloc<float>(m, prop);
     m->v_next = dev_alloc<uint32_t>(m, kMaxVerify);
     m->v_argmax = dev_alloc<char>(m, argmax_scratch_bytes(kMaxVerify));
-    m->copy_table = dev_alloc<CopyRow>(m, 6 * kMaxLayers);  // device and host rows per layer
-    bool ok = state && m->v_norm && m->v_logits && m->v_prop && m->v_next && m->v_argmax &&
-              m->copy_table;
+    bool ok = m->v_norm && m->v_logits && m->v_prop && m->v_next && m->v_argmax;
     ok = ok && hipHostMalloc((void **)&m->v_host, (kMaxVerify * (2 * h + V) + prop) * 4,
                              hipHostMallocDefault) == hipSuccess;
     ok = ok && hipHostMalloc((void **)&m->v_next_host, kMaxVerify * 4, hipHostMallocDefault) ==
@@ -406,12 +401,10 @@ bool alloc_verify(plamo_metal *m, uint64_t L, uint64_t h, uint64_t V) {
                              hipHostMallocDefault) == hipSuccess;
     if (!ok) {
         (void)hipGetLastError();
-        dev_free(m, state);
         free_verify(m);
         problem(m, "cannot allocate verification buffers");
         return false;
     }
-    m->v_state = state;
     return true;
 }
 
@@ -1652,7 +1645,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     const GemmWorkspace *ws = gemm_workspace(
         m, T, std::max({h, m->max_attention, m->max_inter, pair ? h + m->max_inter : 0}));
     if (!ws) return -1;
-    if (verify && !m->v_state && !alloc_verify(m, L, h, V)) return -1;
+    if (verify && !m->v_host && !alloc_verify(m, L, h, V)) return -1;
     // wide[i]: the rows overflow a sliding window and the matrix-core
     // attention takes the layer, over keys rotated at their virtual rows.
     std::vector<char> overflow(L, 0), wide(L, 0);
@@ -1704,9 +1697,11 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     hipStream_t s = m->stream;
     int n = 0;
     begin_timing(m);
-    HIP_FAIL(m, hipMemcpyAsync(m->params_dev, m->params_host, sizeof(StepParams),
-                              hipMemcpyHostToDevice, s));
-    HIP_FAIL(m, hipMemcpyAsync(m->p_ids.ptr, m->ids_host, T * 4, hipMemcpyHostToDevice, s));
+    CopyBlocks in_blocks{};
+    in_blocks.add(m->params_view, m->params_dev, sizeof(StepParams) / 4);
+    in_blocks.add(device_view(m->ids_host), m->p_ids.ptr, T);
+    HIP_FAIL(m, launch_copy_blocks(s, in_blocks));
+    ++n;
     float *state = as<float>(m->p_state), *norm = as<float>(m->p_norm), *qkv = as<float>(m->p_qkv),
           *q = as<float>(m->p_q), *attn = as<float>(m->p_attn), *branch = as<float>(m->p_branch),
           *gu = as<float>(m->p_gu), *act = as<float>(m->p_act);
@@ -1992,22 +1987,21 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         if (!final_normed) HIP_FAIL(m, launch_norm_rows(s, state, h, m->final_norm, 1.0f, m->v_norm, h, h, T));
         HIP_FAIL(m, launch_gemm(s, m->v_norm, h, m->head, V, h, T, m->v_logits, V, ws));
         HIP_FAIL(m, launch_argmax_rows(s, m->v_logits, V, T, m->v_next, m->v_argmax));
-        HIP_FAIL(m, hipMemcpyAsync(m->v_state, state, T * h * 4, hipMemcpyDeviceToDevice, s));
-        HIP_FAIL(m, hipMemcpyAsync(m->v_host, m->v_state, T * h * 4, hipMemcpyDeviceToHost, s));
-        HIP_FAIL(m, hipMemcpyAsync(m->v_host + kMaxVerify * h, m->v_norm, T * h * 4,
-                                  hipMemcpyDeviceToHost, s));
-        HIP_FAIL(m, hipMemcpyAsync(m->v_host + 2 * kMaxVerify * h, m->v_logits, T * V * 4,
-                                  hipMemcpyDeviceToHost, s));
+        float *host = device_view(m->v_host);
+        CopyBlocks out{};
+        out.add(state, host, T * h);
+        out.add(m->v_norm, host + kMaxVerify * h, T * h);
+        out.add(m->v_logits, host + 2 * kMaxVerify * h, T * V);
         // The candidates' cache rows reach the host at commit, for the
         // committed candidate only: written in place by the commit's copy
         // kernel when the host arrays are device-visible, else from this copy.
         m->prop_on_host = !m->host_direct;
         if (m->prop_on_host)
-            HIP_FAIL(m, hipMemcpyAsync(m->v_host + kMaxVerify * (2 * h + V), m->v_prop,
-                                      L * 3 * T * m->max_width * 4, hipMemcpyDeviceToHost, s));
-        HIP_FAIL(m, hipMemcpyAsync(m->v_next_host, m->v_next, T * 4, hipMemcpyDeviceToHost, s));
-        HIP_FAIL(m, hipMemcpyAsync(m->status_host, &m->params_dev->error, 4, hipMemcpyDeviceToHost, s));
-        n += 3;
+            out.add(m->v_prop, host + kMaxVerify * (2 * h + V), L * 3 * T * m->max_width);
+        out.add(m->v_next, device_view(m->v_next_host), T);
+        out.add(&m->params_dev->error, m->status_dev, 1);
+        HIP_FAIL(m, launch_copy_blocks(s, out));
+        n += 4;
     } else {
         const bool one_row = T == 1 || !states;  // the last layer ran as a decode step
         const float *last = state + (T - 1) * h;
@@ -2025,11 +2019,13 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         ph.status = &m->params_dev->error;
         ph.status_out = m->status_dev;
         HIP_FAIL(m, launch_gemv(s, m->head, V, h, ph, m->outbox, 0, 2 * m->cus));
-        if (!one_row)
-            HIP_FAIL(m, hipMemcpyAsync(m->outbox + V, last, h * 4, hipMemcpyDeviceToDevice, s));
-        HIP_FAIL(m, hipMemcpyAsync(m->outbox_host, m->outbox, (V + 2 * h) * 4,
-                                  hipMemcpyDeviceToHost, s));
-        ++n;
+        float *host = device_view(m->outbox_host);
+        CopyBlocks out{};
+        out.add(m->outbox, host, V);
+        out.add(one_row ? m->outbox + V : last, host + V, h);
+        out.add(m->outbox + V + h, host + V + h, h);
+        HIP_FAIL(m, launch_copy_blocks(s, out));
+        n += 2;
     }
     if (!end_timing(m)) return fail(m);
     m->info.dispatches += n;
@@ -2132,9 +2128,8 @@ int plamo_metal_commit(struct plamo_metal *m, struct model *model, uint64_t inde
         }
     }
     if (entries) {
-        HIP_FAIL(m, hipMemcpyAsync(m->copy_table, m->copy_table_host, entries * sizeof(CopyRow),
-                                  hipMemcpyHostToDevice, m->stream));
-        HIP_FAIL(m, launch_copy_rows(m->stream, m->copy_table, entries));
+        HIP_FAIL(m, launch_copy_rows(m->stream, (const CopyRow *)device_view(m->copy_table_host),
+                                     entries));
         ++m->info.dispatches;
     }
     if (!end_timing(m)) return fail(m);

@@ -300,6 +300,21 @@ hipError_t launch_copy_rows(hipStream_t, const CopyRow *table, uint32_t entries)
 // A copy by a kernel, for pinned host memory on either side: 16-byte-aligned
 // addresses and sizes.
 hipError_t launch_copy_block(hipStream_t, const void *src, void *dst, uint64_t bytes);
+// Up to kCopyBlocks blocks of whole words, each of any alignment to a word, in
+// one launch.
+constexpr uint32_t kCopyBlocks = 6;
+struct CopyBlocks {
+    const void *src[kCopyBlocks];
+    void *dst[kCopyBlocks];
+    uint64_t words[kCopyBlocks];
+    uint32_t count;
+    void add(const void *from, void *to, uint64_t n) {
+        src[count] = from;
+        dst[count] = to;
+        words[count++] = n;
+    }
+};
+hipError_t launch_copy_blocks(hipStream_t, const CopyBlocks &blocks);
 // p[0, words) = value (a kernel, so that it is also safe inside captured graphs).
 hipError_t launch_fill(hipStream_t, uint32_t *p, uint64_t words, uint32_t value);
 // Raises the dynamic LDS limit of the GEMV variants to hold `cols` floats.

@@ -358,6 +358,36 @@ def test_prompt_pair_attention(qh, kh, dim, prefix, tokens):
         syn.close()
 
 
+# The copies of a prompt's ids in and of its results out, at vocabularies that
+# leave the host blocks at every word alignment.
+@pytest.mark.parametrize("vocab", [200, 201, 202, 203])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_result_copies(vocab, pinned):
+    say(f"result copies vocab={vocab} pinned={pinned}")
+    syn = plamo_hip.Synthetic(256, 2, 4, 2, 64, 96, vocab, window=64, global_capacity=128,
+                              pattern=2, embedding_std=1.0, seed=vocab)
+    gpu, cpu = syn.instance(pinned=pinned), syn.instance()
+    be = plamo_hip.Backend(syn)
+    try:
+        for tokens in (1, 2, 7, 19):
+            ids = [(7 * j + 3) % vocab for j in range(tokens)]
+            assert be.prefill(gpu, ids) == 1
+            assert oracle_lib.prefill(cpu, ids)
+            compare(gpu, cpu)
+        for tokens in (1, 3, 16):
+            ids = [(5 * j + 2) % vocab for j in range(tokens)]
+            assert be.verify(gpu, ids)[0] == 1
+            for i in range(min(tokens, 2)):
+                assert oracle_lib.forward(cpu, ids[i])
+                assert be.commit(gpu, i) == 1
+                compare(gpu, cpu)
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
+
+
 # Decode steps whose contexts take 16, 17, 32 and 33 splits, at the edges of the
 # merging block's batches (16 partials, 32 maxima).
 @pytest.mark.parametrize("rows", [1022, 1086, 2046, 2110])
