@@ -124,6 +124,8 @@ struct plamo_metal {
     // launch that reads cached rows waits for it (upload_pending).
     hipEvent_t upload_event = nullptr;
     bool upload_pending = false;
+    // The last sync_from_host queued copies that read the host's rows.
+    bool uploading = false;
     std::vector<Range> ranges;
     bool hooks = false;
 
@@ -865,6 +867,7 @@ constexpr uint64_t kPromptPrefixLimit = 64;
 int sync_from_host(plamo_metal *m, struct model *model, std::vector<char> &stale,
                    bool prompt_entry) {
     stale.assign(model->count, 0);
+    m->uploading = false;
     uint32_t entries = 0;
     for (uint64_t i = 0; i < model->count; ++i) {
         Layer &d = m->layers[i];
@@ -904,6 +907,7 @@ int sync_from_host(plamo_metal *m, struct model *model, std::vector<char> &stale
                 HIP_TRY(m, hipMemcpyAsync(d.rot, r->out, bytes, hipMemcpyHostToDevice, m->stream));
         }
         stale[i] = !rotated && c->count;
+        m->uploading = m->uploading || bytes;
         d.synced = false;
     }
     // The kernel reads the table on the stream; the previous call's upload has
@@ -1480,6 +1484,11 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
     if (!resolve_layers(m, model)) return 0;
     DecodePlan plan;
     if (!sync_from_host(m, model, plan.stale, false)) return -1;
+    // The step's own work is queued behind the uploads: this marks their end.
+    if (m->uploading && hipEventRecord(m->upload_event, m->stream) != hipSuccess) {
+        problem(m, "cannot mark the end of an upload");
+        return fail(m);
+    }
     plan.shift.assign(L, 0);
     for (uint64_t i = 0; i < L; ++i) {
         Layer &d = m->layers[i];
@@ -1538,9 +1547,15 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
         }
     }
     // The host arrays of full windows move on by one row while the GPU works
-    // (two C3 windows of 2049 rows: 16.8 MB, as long as the step itself). The
-    // rows that drop out are kept: a step that fails leaves them as they were.
+    // (two C3 windows of 2049 rows: 16.8 MB, as long as the step itself), once
+    // uploads of this call have read them. The rows that drop out are kept: a
+    // step that fails leaves them as they were.
     std::vector<float> dropped;
+    if (m->uploading && std::find(plan.shift.begin(), plan.shift.end(), 1) != plan.shift.end() &&
+        hipEventSynchronize(m->upload_event) != hipSuccess) {
+        problem(m, "cannot upload the host's rows");
+        return fail(m);
+    }
     for (uint64_t i = 0; i < L; ++i) {
         if (!plan.shift[i]) continue;
         const struct cache *c = model->layers[i]->mixer->cache;

@@ -487,3 +487,46 @@ def test_past_the_window(qh, kh, dim, window, prefix, tokens, pinned):
         gpu.close()
         cpu.close()
         syn.close()
+
+
+# Steps on full 2049-row windows whose rows the host has just changed (other
+# rows, stale and current rotations; a CPU step; an announced edit), with every
+# table and buffer grown by an earlier step: 17 MB cross the bus while the step
+# moves the host's rows by one.
+@pytest.mark.parametrize("pinned", [False, True])
+def test_edited_full_windows(pinned):
+    say(f"edited full windows pinned={pinned}")
+    syn = plamo_hip.Synthetic(256, 2, 16, 8, 128, 96, 300, window=2048, global_capacity=4096,
+                              pattern=0, embedding_std=1.0, seed=12)
+    gpu, cpu = syn.instance(pinned=pinned), syn.instance()
+    be = plamo_hip.Backend(syn)
+    try:
+        def step(token):
+            assert be.forward(gpu, token) == 1
+            assert oracle_lib.forward(cpu, token)
+            compare(gpu, cpu)
+
+        for seed in (1, 2):
+            say(f"fill {seed}")
+            for inst in (gpu, cpu):
+                inst.fill_kv(2049, seed)
+            step(7)
+            step(8)
+        say("CPU step")
+        assert oracle_lib.forward(gpu, 9) and oracle_lib.forward(cpu, 9)
+        step(10)
+        say("announced edit")
+        for inst in (gpu, cpu):
+            inst.kv(1, "v")[5:1500] *= 0.5
+            inst.kv(0, "k")[5:1500] *= 0.5
+            inst.rotation(0).processed_count = 0
+        be.invalidate()
+        step(11)
+        step(12)
+        info = be.info()
+        assert info.errors == 0 and info.cpu_fallbacks == 0, info.note.decode()
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
