@@ -1513,10 +1513,31 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
     for (uint64_t i = 0; i < L && short_ctx; ++i)
         short_ctx = model->layers[i]->mixer->cache->count + 1 <= kDecodeShortRows;
     plan.row_cap = short_ctx ? kDecodeShortRows : 0;
+    // A step that fails leaves the host's rows as they were: the rows its move
+    // of a full window dropped go back. The rotations of such a window may be
+    // the moved ones (the mirror is queued with the step): stale, to be rebuilt.
+    std::vector<float> dropped;
+    auto step_failed = [&]() {
+        fail(m);
+        const float *first = dropped.data();
+        for (uint64_t i = 0; i < L; ++i) {
+            if (!plan.shift[i]) continue;
+            struct mixer *mx = model->layers[i]->mixer;
+            const struct cache *c = mx->cache;
+            mx->rotation->processed_count = mx->rotation->scale_bits = 0;
+            if (dropped.empty()) continue;
+            for (float *rows : {c->k, c->v}) {
+                memmove(rows + c->width, rows, (c->capacity - 1) * c->width * 4);
+                memcpy(rows, first, c->width * 4);
+                first += c->width;
+            }
+        }
+        return -1;
+    };
     int dispatches = 0;
     begin_timing(m);
     if (plan.special || m->eager_decode) {
-        if (!encode_decode(m, model, plan, &dispatches)) return fail(m);
+        if (!encode_decode(m, model, plan, &dispatches)) return step_failed();
     } else {
         hipGraphExec_t &g = short_ctx ? m->graph_short : m->graph;
         uint64_t &g_epoch = short_ctx ? m->graph_short_epoch : m->graph_epoch;
@@ -1548,13 +1569,11 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
     }
     // The host arrays of full windows move on by one row while the GPU works
     // (two C3 windows of 2049 rows: 16.8 MB, as long as the step itself), once
-    // uploads of this call have read them. The rows that drop out are kept: a
-    // step that fails leaves them as they were.
-    std::vector<float> dropped;
+    // uploads of this call have read them.
     if (m->uploading && std::find(plan.shift.begin(), plan.shift.end(), 1) != plan.shift.end() &&
         hipEventSynchronize(m->upload_event) != hipSuccess) {
         problem(m, "cannot upload the host's rows");
-        return fail(m);
+        return step_failed();
     }
     for (uint64_t i = 0; i < L; ++i) {
         if (!plan.shift[i]) continue;
@@ -1564,22 +1583,6 @@ int plamo_metal_forward(struct plamo_metal *m, struct model *model, uint64_t tok
             memmove(rows, rows + c->width, (c->capacity - 1) * c->width * 4);
         }
     }
-    auto step_failed = [&]() {
-        const float *first = dropped.data();
-        for (uint64_t i = 0; i < L; ++i) {
-            if (!plan.shift[i]) continue;
-            struct mixer *mx = model->layers[i]->mixer;
-            const struct cache *c = mx->cache;
-            // The mirrored rotations may be the new ones: stale, to be rebuilt.
-            mx->rotation->processed_count = mx->rotation->scale_bits = 0;
-            for (float *rows : {c->k, c->v}) {
-                memmove(rows + c->width, rows, (c->capacity - 1) * c->width * 4);
-                memcpy(rows, first, c->width * 4);
-                first += c->width;
-            }
-        }
-        return fail(m);
-    };
     if (!end_timing(m)) return step_failed();
     m->info.dispatches += dispatches;
     if (device_failed(m)) return step_failed();

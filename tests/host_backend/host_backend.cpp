@@ -244,6 +244,39 @@ void edited_window(bool pinned) {
     }
 }
 
+// A launch that fails anywhere in a step on full windows: -1, the host's rows
+// as they were, and no rotations of the moved window left as current.
+void failed_launch(bool pinned) {
+    Request q(6, 20, 6, pinned);
+    q.fill(21, 10.0f);
+    check(plamo_metal_forward(q.metal, q.model, 1) == 1, "first step");
+    std::vector<std::vector<float>> before;
+    for (uint64_t i = 0; i < q.model->count; ++i)
+        for (float *rows : {q.cache(i)->k, q.cache(i)->v})
+            before.emplace_back(rows, rows + q.cache(i)->count * q.cache(i)->width);
+    int launches = 0;
+    for (bool failed = true; failed; ++launches) {
+        fail_after = launches;
+        const int result = plamo_metal_forward(q.metal, q.model, 2);
+        failed = fail_after < 0;
+        fail_after = -1;
+        check(result == (failed ? -1 : 1), "result", 0, launches);
+        if (!failed) break;
+        for (uint64_t i = 0; i < q.model->count; ++i) {
+            const struct cache *c = q.cache(i);
+            const uint64_t n = c->count * c->width * 4;
+            check(!memcmp(c->k, before[2 * i].data(), n), "host K", i, launches);
+            check(!memcmp(c->v, before[2 * i + 1].data(), n), "host V", i, launches);
+            check(q.rotation(i)->processed_count == 0 || !memcmp(q.rotation(i)->out, c->k, n),
+                  "rotations of other rows", i, launches);
+        }
+    }
+    check(launches > 24, "launches of a step", 0, launches);
+    q.same("step after failures");
+    check(plamo_metal_forward(q.metal, q.model, 3) == 1, "next step");
+    q.same("next step");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -253,6 +286,10 @@ int main(int argc, char **argv) {
         edited_window(true);
     else if (what == "edited_window_pageable")
         edited_window(false);
+    else if (what == "failed_launch")
+        failed_launch(true);
+    else if (what == "failed_launch_pageable")
+        failed_launch(false);
     else
         check(false, "unknown scenario");
     printf("ok\n");

@@ -40,6 +40,8 @@ def host_backend(tmp_path_factory):
     # A step on full windows after the host edited them: the rows it moves are
     # still being uploaded.
     "edited_window", "edited_window_pageable",
+    # Every launch of such a step failing in turn.
+    "failed_launch", "failed_launch_pageable",
 ])
 def test_host_side(host_backend, scenario):
     r = subprocess.run([str(host_backend), scenario], capture_output=True, text=True, timeout=120,
