@@ -1160,18 +1160,15 @@ int encode_decode(plamo_metal *m, struct model *model, const DecodePlan &plan, i
                 n += 2;
             }
         }
-        if (shift && plan.mirror) {
-            moved.push_back(i);
-            if (moved.size() == 4 || i + 4 >= L) {
-                HIP_TRY(m, hipEventRecord(m->layer_events[i], s));
-                HIP_TRY(m, hipStreamWaitEvent(m->copy_stream, m->layer_events[i], 0));
-                for (uint64_t j : moved)
-                    HIP_TRY(m, hipMemcpyAsync(model->layers[j]->mixer->rotation->out,
-                                              m->layers[j].rot,
-                                              m->layers[j].capacity * m->layers[j].width * 4,
-                                              hipMemcpyDeviceToHost, m->copy_stream));
-                moved.clear();
-            }
+        if (shift && plan.mirror) moved.push_back(i);
+        if (!moved.empty() && (moved.size() == 4 || i + 4 >= L)) {
+            HIP_TRY(m, hipEventRecord(m->layer_events[i], s));
+            HIP_TRY(m, hipStreamWaitEvent(m->copy_stream, m->layer_events[i], 0));
+            for (uint64_t j : moved)
+                HIP_TRY(m, hipMemcpyAsync(model->layers[j]->mixer->rotation->out, m->layers[j].rot,
+                                          m->layers[j].capacity * m->layers[j].width * 4,
+                                          hipMemcpyDeviceToHost, m->copy_stream));
+            moved.clear();
         }
         if (!fused_o) {
             Prologue po{};

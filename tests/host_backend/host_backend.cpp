@@ -277,6 +277,18 @@ void failed_launch(bool pinned) {
     q.same("next step");
 }
 
+// One layer with a small full window, at `layer` of eight whose other windows
+// are not full: its rotated rows reach the host wherever it stands.
+void lone_window(uint64_t layer) {
+    Request q(8, 100, 0, true);
+    q.cache(layer)->capacity = 20;
+    q.fill(20, 10.0f);
+    for (uint32_t token = 1; token < 4; ++token) {
+        check(plamo_metal_forward(q.metal, q.model, token) == 1, "step", layer);
+        q.same("step");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -290,6 +302,8 @@ int main(int argc, char **argv) {
         failed_launch(true);
     else if (what == "failed_launch_pageable")
         failed_launch(false);
+    else if (what == "lone_window")
+        for (uint64_t layer = 0; layer < 8; ++layer) lone_window(layer);
     else
         check(false, "unknown scenario");
     printf("ok\n");

@@ -42,6 +42,8 @@ def host_backend(tmp_path_factory):
     "edited_window", "edited_window_pageable",
     # Every launch of such a step failing in turn.
     "failed_launch", "failed_launch_pageable",
+    # A single full window among layers whose windows are not full.
+    "lone_window",
 ])
 def test_host_side(host_backend, scenario):
     r = subprocess.run([str(host_backend), scenario], capture_output=True, text=True, timeout=120,
