@@ -1665,7 +1665,9 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     // attention takes the layer, over keys rotated at their virtual rows.
     std::vector<char> overflow(L, 0), wide(L, 0);
     // paired[i]: the layer's attention runs on fp16 pairs and writes O's input.
+    // Not the last layer's where its last row alone goes on (in FP32).
     std::vector<char> paired(L, 0);
+    const bool last_row = !verify && !states && T > 1;
     uint64_t split_floats = 0, virtual_floats = 0, pair_bytes = 0;
     for (uint64_t i = 0; i < L; ++i) {
         const Layer &d = m->layers[i];
@@ -1676,7 +1678,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             if (!ensure_exact_rows(m, m->ropes[d.rope], c->count + T)) return -1;
             virtual_floats = std::max(virtual_floats, (c->count + T) * d.width);
         }
-        paired[i] = pair && (!window || wide[i]) &&
+        paired[i] = pair && (!window || wide[i]) && !(last_row && i + 1 == L) &&
                     pair_attention_supported((uint32_t)c->count, (uint32_t)T, d.qh, d.kh, d.dim);
         if (paired[i])
             pair_bytes = std::max(pair_bytes, pair_attention_scratch((uint32_t)c->count,
@@ -1686,7 +1688,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                                     prompt_attention_scratch((uint32_t)c->count, (uint32_t)T, d.qh,
                                                              d.kh, d.dim, window, wide[i]));
         // The last layer's attention may run for its last row alone.
-        if (i + 1 == L)
+        if (last_row && i + 1 == L)
             split_floats = std::max(split_floats,
                                     prompt_attention_scratch((uint32_t)(c->count + T - 1), 1, d.qh,
                                                              d.kh, d.dim, window, wide[i]));
@@ -1761,7 +1763,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         // layer's queries, attention, O projection and MLP run for that row
         // alone, as the decode step runs them (runtime/metal_model.m:761-770
         // trims the projection and the MLP); K and V rows are formed for all.
-        const bool last_row_only = !verify && !states && i + 1 == L && T > 1;
+        const bool last_row_only = last_row && i + 1 == L;
         const bool last_query = last_row_only && pair && aw % 32 == 0 &&
                                 prompt_attention_matrix(d.dim, d.qh, d.kh);
         if (!normed) {
@@ -1872,13 +1874,12 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             pa.prefix += (uint32_t)(T - 1);
             pa.tokens = 1;
         }
-        const bool on_pairs = paired[i] && !last_query;
-        if (on_pairs)
+        if (paired[i])
             HIP_FAIL(m, launch_pair_attention(s, pa, m->p_kv_pairs.ptr, v_exp, in));
         else
             HIP_FAIL(m, launch_prompt_attention(s, pa));
         v_exp += d.kh;
-        n += on_pairs ? 2 : 1;
+        n += paired[i] ? 2 : 1;
         if (overflow[i] && !verify) {
             HIP_FAIL(m, launch_window_store(s, d.k, d.v, d.rot, as<float>(m->p_side_k),
                                            as<float>(m->p_side_v), d.width, rope.table,
@@ -1963,7 +1964,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                 PairRows gu_in = in;
                 gu_in.norms = d.gu_norms;
                 gu_in.act_exps = act.exps;
-                if (!on_pairs)
+                if (!paired[i])
                     HIP_FAIL(m, launch_norm_rows(s, attn, aw, nullptr, 0.0f, attn, aw, aw, T, &in));
                 HIP_FAIL(m, launch_gemm_pair(s, in, d.p_o, T, branch, h, *ws));
                 HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, post, kAttentionOffset, mpre,

@@ -530,3 +530,35 @@ def test_edited_full_windows(pinned):
         gpu.close()
         cpu.close()
         syn.close()
+
+
+# A prompt without its states (only the last row feeds the logits) at groups
+# the fp16-pair attention takes and the FP32 matrix-core form does not, and at
+# groups both take.
+@pytest.mark.parametrize("qh,kh,dim", [(3, 1, 128), (6, 2, 64), (5, 1, 64), (14, 2, 128), (8, 2, 128),
+                                       (6, 1, 128)])
+@pytest.mark.parametrize("prefix,tokens", [(0, 33), (9, 70), (12, 300)])
+def test_prompt_last_row(qh, kh, dim, prefix, tokens):
+    say(f"last row {qh}/{kh}x{dim} prefix={prefix} tokens={tokens}")
+    syn = plamo_hip.Synthetic(256, 2, qh, kh, dim, 96, 300, window=2304, global_capacity=2304,
+                              pattern=2, embedding_std=1.0, seed=5)
+    gpu, cpu = syn.instance(), syn.instance()
+    be = plamo_hip.Backend(syn)
+    try:
+        for turn in range(2):  # the buffers then hold another prompt's rows
+            gpu.reset()
+            cpu.reset()
+            ids = [(j * 13 + 5 * turn) % 300 for j in range(prefix + tokens)]
+            for part in (ids[:prefix], ids[prefix:]):
+                if part:
+                    assert be.prefill(gpu, part) == 1
+                    assert oracle_lib.prefill(cpu, part)
+                    compare(gpu, cpu)
+                    gate(gpu.normalized().copy(), cpu.normalized().copy(), "normalized")
+        info = be.info()
+        assert info.errors == 0 and info.cpu_fallbacks == 0, info.note.decode()
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
