@@ -73,10 +73,11 @@ struct Layer {
     const uint16_t *qkv = nullptr, *o = nullptr, *gu = nullptr, *down = nullptr;
     uint16_t *norms = nullptr;  // device: pre | post | mlp_pre | mlp_post | qn | kn
     const uint16_t *pre, *post, *mlp_pre, *mlp_post, *qn, *kn;
-    // The projections as fp16 fragments (pair_ready), and the largest 2-norms
-    // of the gate and of the up rows.
+    // The projections as fp16 fragments (pair_ready), and the scales of the
+    // SwiGLU activation's columns (launch_pair_balance).
     PairWeight p_qkv{}, p_o{}, p_gu{}, p_down{};
-    uint32_t *gu_norms = nullptr;
+    int32_t *act_cols = nullptr;
+    float *act_bound = nullptr;
     uint32_t qh = 0, kh = 0, dim = 0, hidden = 0, inter = 0, width = 0;
     uint64_t capacity = 0;
     bool sliding = false;
@@ -794,20 +795,19 @@ int ensure_pair(plamo_metal *m, struct model *model) {
         PairWeight *p;
         const uint16_t *w;
         uint64_t rows, cols, frag, exps;
-        bool gate_up;
     };
     std::vector<Place> places;
-    std::vector<uint64_t> norms;
+    std::vector<uint64_t> act_cols;
     for (Layer &d : m->layers) {
         const uint64_t aw = (uint64_t)d.qh * d.dim;
         // Norm rows and attention rows become planes in one launch each, of
         // at most 8192 columns; gate and up rows pair up in groups of 32.
         if (h % kPairK || h > 8192 || aw % kPairK || aw > 8192 || d.inter % kPairK) return 1;
-        places.push_back({&d.p_qkv, d.qkv, (uint64_t)(d.qh + 2 * d.kh) * d.dim, h, 0, 0, false});
-        places.push_back({&d.p_o, d.o, h, aw, 0, 0, false});
-        places.push_back({&d.p_gu, d.gu, 2 * (uint64_t)d.inter, h, 0, 0, true});
-        places.push_back({&d.p_down, d.down, h, d.inter, 0, 0, false});
-        norms.push_back(take(8));
+        places.push_back({&d.p_qkv, d.qkv, (uint64_t)(d.qh + 2 * d.kh) * d.dim, h, 0, 0});
+        places.push_back({&d.p_o, d.o, h, aw, 0, 0});
+        places.push_back({&d.p_gu, d.gu, 2 * (uint64_t)d.inter, h, 0, 0});
+        places.push_back({&d.p_down, d.down, h, d.inter, 0, 0});
+        act_cols.push_back(take(4 + (uint64_t)d.inter * 4));
     }
     for (Place &q : places) {
         if (!pair_supported(q.rows, q.cols) || ((uintptr_t)q.w & 15)) return 1;
@@ -815,6 +815,7 @@ int ensure_pair(plamo_metal *m, struct model *model) {
         q.exps = take(pair_exp_count(q.rows) * 4);
     }
     const uint64_t exps = take(2 * (kMaxPrompt + 128) * 4);
+    const uint64_t norms = take(2 * m->max_inter * 4);  // one layer's gate | up rows at a time
     // Room for the KV caches and prompt buffers that grow later.
     size_t free_bytes = 0, total = 0;
     if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || free_bytes < bytes + total / 16 ||
@@ -826,17 +827,19 @@ int ensure_pair(plamo_metal *m, struct model *model) {
     m->allocations.push_back(m->pair_block);
     m->info.allocated_bytes += bytes;
     m->pair_exps = (int32_t *)(m->pair_block + exps);
-    for (size_t i = 0; i < m->layers.size(); ++i) {
-        m->layers[i].gu_norms = (uint32_t *)(m->pair_block + norms[i]);
-        HIP_TRY(m, launch_fill(m->stream, m->layers[i].gu_norms, 2, 0));
-    }
-    for (size_t i = 0; i < places.size(); ++i) {
-        const Place &q = places[i];
+    for (const Place &q : places)
         *q.p = PairWeight{(uint16_t *)(m->pair_block + q.frag), (int32_t *)(m->pair_block + q.exps),
                           (uint32_t)q.rows, (uint32_t)q.cols, (uint32_t)((q.rows + 31) / 32)};
-        HIP_TRY(m, launch_pair_weights(m->stream, q.w, *q.p,
-                                       q.gate_up ? m->layers[i / 4].gu_norms : nullptr,
-                                       q.rows / 2));
+    float *row_norms = (float *)(m->pair_block + norms);
+    for (size_t i = 0; i < m->layers.size(); ++i) {
+        Layer &d = m->layers[i];
+        d.act_bound = (float *)(m->pair_block + act_cols[i]);
+        d.act_cols = (int32_t *)(d.act_bound + 1);
+        HIP_TRY(m, launch_pair_weights(m->stream, d.qkv, d.p_qkv, nullptr, nullptr));
+        HIP_TRY(m, launch_pair_weights(m->stream, d.o, d.p_o, nullptr, nullptr));
+        HIP_TRY(m, launch_pair_weights(m->stream, d.gu, d.p_gu, row_norms, nullptr));
+        HIP_TRY(m, launch_pair_balance(m->stream, row_norms, d.inter, d.act_cols, d.act_bound));
+        HIP_TRY(m, launch_pair_weights(m->stream, d.down, d.p_down, nullptr, d.act_cols));
     }
     m->pair_ready = true;
     return 1;
@@ -1961,8 +1964,9 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                 act.planes = ws->planes + 2 * (uint64_t)in.padded * h;
                 act.exps = m->pair_exps + kMaxPrompt + 128;
                 act.padded = in.padded;
+                act.col_exps = d.act_cols;
                 PairRows gu_in = in;
-                gu_in.norms = d.gu_norms;
+                gu_in.act_bound = d.act_bound;
                 gu_in.act_exps = act.exps;
                 if (!paired[i])
                     HIP_FAIL(m, launch_norm_rows(s, attn, aw, nullptr, 0.0f, attn, aw, aw, T, &in));

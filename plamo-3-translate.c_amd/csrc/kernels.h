@@ -110,32 +110,39 @@ struct PairWeight {
 // The rows from `first` (a multiple of 32) on.
 PairWeight pair_rows_from(const PairWeight &w, uint32_t first);
 // Rows of X as scaled pairs of fp16 terms: [cols / 32][hi, lo][padded][32],
-// value = (hi + lo) * 2^-exps[row]. With act_exps (and norms, the largest
-// 2-norms of the gate and of the up rows as float bits), a norm also writes
-// the exponents of the rows' SwiGLU activation.
+// value = (hi + lo) * 2^-exps[row]. With act_exps (and act_bound,
+// launch_pair_balance's) a norm also writes the exponents of the rows' SwiGLU
+// activation, whose planes hold value = (hi + lo) * 2^(col_exps[column] -
+// exps[row]).
 constexpr uint32_t kPairK = 32;
 struct PairRows {
     uint16_t *planes;
     int32_t *exps;
     uint32_t padded;
-    const uint32_t *norms;
+    const float *act_bound;
     int32_t *act_exps;
+    const int32_t *col_exps;
 };
 bool pair_supported(uint64_t rows, uint64_t cols);
 uint64_t pair_frag_elems(uint64_t rows, uint64_t cols);
 uint64_t pair_exp_count(uint64_t rows);
 // Rows of the planes for `tokens` rows (the consumer's tiles are whole).
 uint32_t pair_padded(uint64_t tokens);
-// Fills p.frag and p.exps from p.rows x p.cols BF16 weights (16-byte aligned);
-// norms (optional, zero before): the largest 2-norm of the rows below `half`
-// and of the others.
-hipError_t launch_pair_weights(hipStream_t, const uint16_t *w, const PairWeight &p,
-                               uint32_t *norms, uint64_t half);
+// Fills p.frag and p.exps from p.rows x p.cols BF16 weights (16-byte aligned),
+// column c times 2^col_exps[c] (optional); norms (optional): each row's 2-norm.
+hipError_t launch_pair_weights(hipStream_t, const uint16_t *w, const PairWeight &p, float *norms,
+                               const int32_t *col_exps);
+// From the 2-norms of a gate | up projection's rows: the exponents that balance
+// the columns of its SwiGLU activation, for the activation's planes and for
+// down's fragments, and the bound the norms scale the activation by.
+hipError_t launch_pair_balance(hipStream_t, const float *norms, uint64_t intermediate,
+                               int32_t *col_exps, float *bound);
 // y[t, r] = X W^T on the fp16 matrix cores, FP32 sums.
 hipError_t launch_gemm_pair(hipStream_t, const PairRows &x, const PairWeight &w, uint64_t tokens,
                             float *y, uint64_t y_stride, const GemmWorkspace &ws);
 // silu(gate) * up of a gate | up projection into act.planes, scaled by
-// act.exps (written by the norm that formed x); w.rows / 2 a multiple of 32.
+// act.exps (written by the norm that formed x) and act.col_exps; w.rows / 2 a
+// multiple of 32.
 hipError_t launch_gemm_pair_swiglu(hipStream_t, const PairRows &x, const PairWeight &w,
                                    uint64_t tokens, const PairRows &act, const GemmWorkspace &ws);
 // Multi-row RMSNorm; with branch: state += rms(branch) * (bf16(w) + offset).

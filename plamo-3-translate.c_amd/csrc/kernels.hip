@@ -2139,11 +2139,13 @@ __device__ __forceinline__ void pair_zero_row(const PairRows &p, uint32_t row, u
 
 // One row held by a 256-thread block (thread i: elements 4 (i + 256 j) .. + 3,
 // zero past the row) into the planes. With act_exps also the exponent of the
-// row's SwiGLU activation, from |silu(g) u| <= |g| |u| and Cauchy-Schwarz:
-// the row's 2-norm squared times the largest 2-norms of the gate and the up
-// rows (norms) is an upper bound that needs no pass over the activation. It
-// exceeds the typical value by about the row's length; the pair still
-// resolves 2^-40 of it.
+// row's SwiGLU activation, from |silu(g) u| <= |g| |u| and Cauchy-Schwarz: the
+// row's 2-norm squared times `act_bound`, the largest product of a column's
+// gate and up 2-norms once the columns are balanced (pair_balance_kernel), is
+// an upper bound that needs no pass over the activation. Balanced, it exceeds
+// every column's typical value by about the row's length (2^12 or 2^13), and
+// the pair resolves 2^-40 of it; FP32 sums of gate and up leave more than that
+// unless both rows stand within 2^-15 of a right angle to the input.
 template <int NV>
 __device__ __forceinline__ void pair_row(const PairRows &p, uint32_t row, uint32_t groups,
                                          const f32x4 (&v)[NV], float *red) {
@@ -2187,33 +2189,44 @@ __device__ __forceinline__ void pair_row(const PairRows &p, uint32_t row, uint32
     if (threadIdx.x == 0) {
         p.exps[row] = ex;
         if (p.act_exps) {
-            const float bound = __uint_as_float(p.norms[0]) * __uint_as_float(p.norms[1]) * ss;
-            p.act_exps[row] = pair_exponent(__float_as_uint(bound));
+            p.act_exps[row] = pair_exponent(__float_as_uint(*p.act_bound * ss));
         }
     }
 }
 
 // Block: 32 weight rows. Rows past `rows` (the last group's padding) are zero.
-// norms[0] (rows below `half`) and norms[1]: the largest 2-norm of a row, as
-// float bits.
+// norms (optional): each row's 2-norm. col_exps (optional): column c is taken
+// times 2^col_exps[c], at most 0.
 __global__ __launch_bounds__(kThreads) void pair_weights_kernel(const uint16_t *w, uint32_t rows,
                                                                 uint32_t cols, uint16_t *frag,
-                                                                int32_t *exps, uint32_t *norms,
-                                                                uint32_t half) {
+                                                                int32_t *exps, float *norms,
+                                                                const int32_t *col_exps) {
     __shared__ float scales[32];
     const uint32_t r0 = blockIdx.x * 32, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // Columns c .. c + 7 of a row.
+    auto load = [&](uint32_t row, uint32_t c, float (&x)[8]) {
+        const u32x4 q = *(const u32x4 *)(w + (uint64_t)row * cols + c);
+        const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[2 * e] = bf16f(u[e] & 0xffffu);
+            x[2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
+        }
+        if (col_exps)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = __builtin_ldexpf(x[e], col_exps[c + e]);
+    };
     for (uint32_t r = wave; r < 32; r += 4) {
         const uint32_t row = r0 + r;
         float mx = 0.0f, ss = 0.0f;
         if (row < rows)
             for (uint32_t c = lane * 8; c < cols; c += 512) {
-                const u32x4 q = *(const u32x4 *)(w + (uint64_t)row * cols + c);
-                const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+                float x[8];
+                load(row, c, x);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float a = bf16f(u[e] & 0xffffu), b = __uint_as_float(u[e] & 0xffff0000u);
-                    mx = fmaxf(mx, fmaxf(__builtin_fabsf(a), __builtin_fabsf(b)));
-                    ss = __builtin_fmaf(a, a, __builtin_fmaf(b, b, ss));
+                for (int e = 0; e < 8; ++e) {
+                    mx = fmaxf(mx, __builtin_fabsf(x[e]));
+                    ss = __builtin_fmaf(x[e], x[e], ss);
                 }
             }
         mx = wave_max(mx);
@@ -2222,28 +2235,45 @@ __global__ __launch_bounds__(kThreads) void pair_weights_kernel(const uint16_t *
             const int ex = pair_exponent(__float_as_uint(mx));
             exps[r0 + r] = ex;
             scales[r] = power_of_two(ex);
-            if (norms && row < rows)
-                (void)__hip_atomic_fetch_max(norms + (row < half ? 0 : 1),
-                                             __float_as_uint(__builtin_sqrtf(ss)),
-                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (norms && row < rows) norms[row] = __builtin_sqrtf(ss);
         }
     }
     __syncthreads();
     const uint32_t row = r0 + (lane & 31);
     const float scale = scales[lane & 31];
     for (uint32_t f = wave; f < cols / 16; f += 4) {
-        u32x4 q = {0u, 0u, 0u, 0u};
-        if (row < rows) q = *(const u32x4 *)(w + (uint64_t)row * cols + 16 * f + 8 * (lane >> 5));
-        const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+        float x[8] = {};
+        if (row < rows) load(row, 16 * f + 8 * (lane >> 5), x);
         f16x8 o;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            o[2 * e] = (_Float16)(bf16f(u[e] & 0xffffu) * scale);
-            o[2 * e + 1] = (_Float16)(__uint_as_float(u[e] & 0xffff0000u) * scale);
-        }
+        for (int e = 0; e < 8; ++e) o[e] = (_Float16)(x[e] * scale);
         const uint64_t at = (((uint64_t)(f / 2) * gridDim.x + blockIdx.x) * 2 + f % 2) * 512;
         *(f16x8 *)(frag + at + lane * 8) = o;
     }
+}
+
+// Column i of the SwiGLU activation is at most |gate row i| |up row i| times
+// the input's squared norm, so columns may differ as much as those rows do.
+// col_exps[i], at most 0, is the power of two that its product stands below the
+// largest one: the activation is taken over 2^col_exps[i] and down's column
+// times it, and one exponent then serves a row's every column alike. *bound:
+// the largest product, rounded up to a power of two.
+__global__ __launch_bounds__(kThreads) void pair_balance_kernel(const float *norms,
+                                                                uint32_t inter, int32_t *col_exps,
+                                                                float *bound) {
+    __shared__ float red[4];
+    float mx = 0.0f;
+    for (uint32_t i = threadIdx.x; i < inter; i += kThreads)
+        mx = fmaxf(mx, norms[i] * norms[inter + i]);
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    auto exponent = [](float x) { return (int)(__float_as_uint(x) >> 23 & 255u); };
+    const int top = exponent(mx);
+    for (uint32_t i = threadIdx.x; i < inter; i += kThreads)
+        col_exps[i] = max(min(exponent(norms[i] * norms[inter + i]) - top, 0), -126);
+    if (threadIdx.x == 0) *bound = __uint_as_float((uint32_t)min(top + 1, 255) << 23);
 }
 
 bool pair_supported(uint64_t rows, uint64_t cols) {
@@ -2261,11 +2291,18 @@ PairWeight pair_rows_from(const PairWeight &w, uint32_t first) {
 }
 
 hipError_t launch_pair_weights(hipStream_t stream, const uint16_t *w, const PairWeight &p,
-                               uint32_t *norms, uint64_t half) {
+                               float *norms, const int32_t *col_exps) {
     if (!pair_supported(p.rows, p.cols) || ((uintptr_t)w & 15) || p.groups != (p.rows + 31) / 32)
         return hipErrorInvalidValue;
     pair_weights_kernel<<<(p.rows + 31) / 32, kThreads, 0, stream>>>(w, p.rows, p.cols, p.frag,
-                                                                     p.exps, norms, (uint32_t)half);
+                                                                     p.exps, norms, col_exps);
+    return hipGetLastError();
+}
+
+hipError_t launch_pair_balance(hipStream_t stream, const float *norms, uint64_t intermediate,
+                               int32_t *col_exps, float *bound) {
+    if (!intermediate || intermediate > UINT32_MAX / 2) return hipErrorInvalidValue;
+    pair_balance_kernel<<<1, kThreads, 0, stream>>>(norms, (uint32_t)intermediate, col_exps, bound);
     return hipGetLastError();
 }
 
@@ -2289,10 +2326,10 @@ struct GemmPair {
     // Nonzero (the intermediate size I, whole groups of 32): the weight rows
     // are gate | up, a wave's even tiles take gate rows and its odd tiles the
     // up rows of the same columns, and silu(gate) * up goes to `act` as planes
-    // scaled by act_exps.
+    // scaled by act_exps, each column over 2^col_exps.
     uint32_t swiglu;
     uint16_t *act;
-    const int32_t *act_exps;
+    const int32_t *act_exps, *col_exps;
 };
 
 // SUMS accumulators per tile (1, or 4: hi and lo terms and the two halves of a
@@ -2477,6 +2514,10 @@ __global__ __launch_bounds__(64 * GM * GN, OCC) void gemm_pair_kernel(GemmPair g
     int we[WN];
 #pragma unroll
     for (int j = 0; j < WN; ++j) we[j] = g.w.exps[row_group(wn, j) * 32 + (lane & 31)];
+    int ce[(WN + 1) / 2] = {};
+    if (g.swiglu)
+#pragma unroll
+        for (int j = 0; j < WN / 2; ++j) ce[j] = g.col_exps[row_group(wn, 2 * j) * 32 + (lane & 31)];
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -2485,7 +2526,7 @@ __global__ __launch_bounds__(64 * GM * GN, OCC) void gemm_pair_kernel(GemmPair g
             if (row >= g.padded) continue;
             const int xe = g.row_exps[row];
             if (WN % 2 == 0 && g.swiglu) {
-                const float scale = power_of_two(g.act_exps[row]);
+                const int ae = g.act_exps[row];
 #pragma unroll
                 for (int j = 0; j + 1 < WN; j += 2) {
                     const uint32_t c = bn * (BN / 64) + wn * (WN / 2) + j / 2;
@@ -2495,7 +2536,7 @@ __global__ __launch_bounds__(64 * GM * GN, OCC) void gemm_pair_kernel(GemmPair g
                     const float up = __builtin_ldexpf(acc[i][j + 1][v], -(xe + we[j + 1]));
                     const float d = plamo_exp(-gate) + 1.0f;
                     _Float16 hi, lo;
-                    pair_split((gate / d) * up, scale, hi, lo);
+                    pair_split(__builtin_ldexpf((gate / d) * up, ae - ce[j / 2]), 1.0f, hi, lo);
                     const uint64_t at = pair_at(g.padded, row, c * 32 + (lane & 31));
                     g.act[at] = __builtin_bit_cast(uint16_t, hi);
                     g.act[at + (uint64_t)g.padded * kPairK] = __builtin_bit_cast(uint16_t, lo);
@@ -2593,7 +2634,7 @@ hipError_t launch_gemm_pair(hipStream_t stream, const PairRows &x, const PairWei
 hipError_t launch_gemm_pair_swiglu(hipStream_t stream, const PairRows &x, const PairWeight &w,
                                    uint64_t tokens, const PairRows &act, const GemmWorkspace &ws) {
     if (!tokens || tokens > x.padded || act.padded != x.padded || !pair_supported(w.rows, w.cols) ||
-        w.rows % 64)
+        w.rows % 64 || !act.col_exps)
         return hipErrorInvalidValue;
     GemmPair g{};
     g.planes = x.planes;
@@ -2604,6 +2645,7 @@ hipError_t launch_gemm_pair_swiglu(hipStream_t stream, const PairRows &x, const 
     g.swiglu = w.rows / 2;
     g.act = act.planes;
     g.act_exps = act.exps;
+    g.col_exps = act.col_exps;
     return gemm_pair_route(stream, g, ws);
 }
 

@@ -101,8 +101,11 @@ bool pair_supported(uint64_t, uint64_t) { return true; }
 uint64_t pair_frag_elems(uint64_t rows, uint64_t cols) { return rows * cols; }
 uint64_t pair_exp_count(uint64_t rows) { return rows; }
 uint32_t pair_padded(uint64_t tokens) { return (uint32_t)tokens; }
-hipError_t launch_pair_weights(hipStream_t s, const uint16_t *, const PairWeight &, uint32_t *,
-                               uint64_t) {
+hipError_t launch_pair_weights(hipStream_t s, const uint16_t *, const PairWeight &, float *,
+                               const int32_t *) {
+    return queue(s);
+}
+hipError_t launch_pair_balance(hipStream_t s, const float *, uint64_t, int32_t *, float *) {
     return queue(s);
 }
 hipError_t launch_gemm_pair(hipStream_t s, const PairRows &, const PairWeight &, uint64_t, float *,

@@ -21,6 +21,7 @@ import ctypes
 import numpy as np
 import pytest
 
+import parity
 from parity import compare, gate, oracle_lib, plamo_hip, say
 
 pytestmark = pytest.mark.gpu
@@ -298,3 +299,53 @@ def test_linear_host_rows(pad):
             assert np.all(y[:, rows:] == 7.0)
     finally:
         be.close()
+
+
+def scale_rows(weights, rows, cols, which, exponent):
+    """Multiplies row `which` of a BF16 matrix by 2^exponent, in place."""
+    w = np.ctypeslib.as_array(weights, shape=(rows, cols))
+    w[which] = np.where(w[which] & 0x7fff, w[which] + np.uint16(exponent << 7), w[which])
+
+
+# Gate and up rows far larger than the others (at one column, at two, one of
+# them alone), whose columns down ignores or takes as much smaller: the other
+# columns of the activation keep the precision they have without them.
+@pytest.mark.parametrize("gate,up,exponent,ignored", [
+    (None, None, 0, True), (5, 5, 8, True), (5, 700, 8, True), (1023, 1023, 10, False),
+    (0, None, 10, True), (None, 31, 10, False),
+])
+@pytest.mark.parametrize("tokens", [7, 40, 140])
+def test_prompt_activation_columns(gate, up, exponent, ignored, tokens):
+    say(f"activation columns gate={gate} up={up} 2^{exponent} ignored={ignored} tokens={tokens}")
+    hidden, inter = 1024, 1024
+    syn = plamo_hip.Synthetic(hidden, 1, 4, 2, 64, inter, 200, window=1024, global_capacity=1024,
+                              pattern=1, embedding_std=1.0, seed=tokens)
+    gpu, cpu = syn.instance(), syn.instance()
+    mlp = gpu.layer(0).mlp.contents
+    down = np.ctypeslib.as_array(mlp.down, shape=(hidden, inter))
+    for row, column in ((gate, gate), (None if up is None else inter + up, up)):
+        if row is None:
+            continue
+        scale_rows(mlp.gu, 2 * inter, hidden, row, exponent)
+        if ignored:
+            down[:, column] = 0
+        else:
+            down[:, column] = np.where(down[:, column] & 0x7fff,
+                                       down[:, column] - np.uint16(exponent << 7), 0)
+    be = plamo_hip.Backend(syn)
+    try:
+        ids = [(7 * j + 3) % 200 for j in range(tokens)]
+        actual = np.zeros((tokens, hidden), np.float32)
+        expected = np.zeros((tokens, hidden), np.float32)
+        assert be.prefill(gpu, ids, actual) == 1
+        assert oracle_lib.prefill(cpu, ids, expected)
+        rel, _ = parity.gate(actual, expected, "states")
+        say(f"relative {rel:.3g}")
+        # 1024 additions in FP32, each within half an ulp (2^-25 in the mean),
+        # leave about 2^-25 sqrt(1024) of a sum: 9.5e-7 on either side.
+        assert rel <= 1.5e-6
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
