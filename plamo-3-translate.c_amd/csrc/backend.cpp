@@ -1667,10 +1667,17 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     // wide[i]: the rows overflow a sliding window and the matrix-core
     // attention takes the layer, over keys rotated at their virtual rows.
     std::vector<char> overflow(L, 0), wide(L, 0);
-    // paired[i]: the layer's attention runs on fp16 pairs and writes O's input.
-    // Not the last layer's where its last row alone goes on (in FP32).
+    // paired[i]: the layer's attention runs on fp16 pairs.
     std::vector<char> paired(L, 0);
+    // With states == NULL only the final row feeds the logits: the last layer's
+    // O projection and MLP run for that row alone, as the decode step runs them
+    // (runtime/metal_model.m:761-770 trims the projection and the MLP), and its
+    // queries and attention (last_query) where the one-row forms cover them; K
+    // and V rows are formed for all.
     const bool last_row = !verify && !states && T > 1;
+    const Layer &end = m->layers[L - 1];
+    const bool last_query = last_row && pair && ((uint64_t)end.qh * end.dim) % 32 == 0 &&
+                            prompt_attention_matrix(end.dim, end.qh, end.kh);
     uint64_t split_floats = 0, virtual_floats = 0, pair_bytes = 0;
     for (uint64_t i = 0; i < L; ++i) {
         const Layer &d = m->layers[i];
@@ -1681,7 +1688,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             if (!ensure_exact_rows(m, m->ropes[d.rope], c->count + T)) return -1;
             virtual_floats = std::max(virtual_floats, (c->count + T) * d.width);
         }
-        paired[i] = pair && (!window || wide[i]) && !(last_row && i + 1 == L) &&
+        paired[i] = pair && (!window || wide[i]) && !(last_query && i + 1 == L) &&
                     pair_attention_supported((uint32_t)c->count, (uint32_t)T, d.qh, d.kh, d.dim);
         if (paired[i])
             pair_bytes = std::max(pair_bytes, pair_attention_scratch((uint32_t)c->count,
@@ -1690,18 +1697,13 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             split_floats = std::max(split_floats,
                                     prompt_attention_scratch((uint32_t)c->count, (uint32_t)T, d.qh,
                                                              d.kh, d.dim, window, wide[i]));
-        // The last layer's attention may run for its last row alone.
-        if (last_row && i + 1 == L)
+        if (last_query && i + 1 == L)
             split_floats = std::max(split_floats,
                                     prompt_attention_scratch((uint32_t)(c->count + T - 1), 1, d.qh,
                                                              d.kh, d.dim, window, wide[i]));
     }
     if (split_floats && !ensure(m, m->p_attn_split, split_floats * 4)) return -1;
-    // The V exponents of every layer's KV heads, after the scratch.
-    uint64_t heads = 0;
-    for (const Layer &d : m->layers) heads += d.kh;
-    pair_bytes = (pair_bytes + 255) / 256 * 256;
-    if (pair_bytes && !ensure(m, m->p_kv_pairs, pair_bytes + heads * 4)) return -1;
+    if (pair_bytes && !ensure(m, m->p_kv_pairs, pair_bytes)) return -1;
     if (virtual_floats && !ensure(m, m->p_virtual, virtual_floats * 4)) return -1;
     for (uint64_t i = 0; i < L; ++i) {
         Layer &d = m->layers[i];
@@ -1728,11 +1730,6 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     HIP_FAIL(m, launch_embed(s, m->embedding, as<uint32_t>(m->p_ids), nullptr, (uint32_t)T,
                             (uint32_t)h, state));
     ++n;
-    int32_t *v_exp = (int32_t *)(as<char>(m->p_kv_pairs) + pair_bytes);
-    if (pair_bytes) {
-        HIP_FAIL(m, launch_fill(s, (uint32_t *)v_exp, heads, (uint32_t)kPairNoExp));
-        ++n;
-    }
     // A residual followed by a norm of the same rows runs as one launch; then
     // `normed` says the next layer's input norm is already in `norm`.
     const bool fuse_rows = h <= 8192;
@@ -1762,19 +1759,13 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                        *mpost = d.norms + 3 * h, *qn = d.norms + 4 * h, *kn = qn + d.dim;
         const RopeTable &rope = m->ropes[d.rope];
         const uint64_t qkv_w = (uint64_t)(d.qh + 2 * d.kh) * d.dim, aw = (uint64_t)d.qh * d.dim;
-        // With states == NULL only the final row feeds the logits: the last
-        // layer's queries, attention, O projection and MLP run for that row
-        // alone, as the decode step runs them (runtime/metal_model.m:761-770
-        // trims the projection and the MLP); K and V rows are formed for all.
-        const bool last_row_only = last_row && i + 1 == L;
-        const bool last_query = last_row_only && pair && aw % 32 == 0 &&
-                                prompt_attention_matrix(d.dim, d.qh, d.kh);
+        const bool last_row_only = last_row && i + 1 == L, last_query_only = last_query && i + 1 == L;
         if (!normed) {
             HIP_FAIL(m, launch_norm_rows(s, state, h, pre, 1.0f, norm, h, h, T, norm_pair));
             ++n;
         }
         normed = false;
-        if (last_query) {
+        if (last_query_only) {
             Prologue pq{};
             pq.src = state + (T - 1) * h;
             pq.w = pre;
@@ -1840,7 +1831,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             HIP_FAIL(m, launch_rerotate(s, d.k, qp.k_virtual, rope.exact, c->count, d.kh, d.dim));
             ++n;
         }
-        qp.last_query = last_query;
+        qp.last_query = last_query_only;
         HIP_FAIL(m, launch_qkv_post(s, qp));
         ++n;
         PromptAttention pa{};
@@ -1871,17 +1862,16 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             pa.v_new = verify ? prop_v : d.v + c->count * d.width;
             pa.window = 0;
         }
-        if (last_query) {
+        if (last_query_only) {
             pa.q += (T - 1) * aw;
             pa.out += (T - 1) * aw;
             pa.prefix += (uint32_t)(T - 1);
             pa.tokens = 1;
         }
         if (paired[i])
-            HIP_FAIL(m, launch_pair_attention(s, pa, m->p_kv_pairs.ptr, v_exp, in));
+            HIP_FAIL(m, launch_pair_attention(s, pa, m->p_kv_pairs.ptr));
         else
             HIP_FAIL(m, launch_prompt_attention(s, pa));
-        v_exp += d.kh;
         n += paired[i] ? 2 : 1;
         if (overflow[i] && !verify) {
             HIP_FAIL(m, launch_window_store(s, d.k, d.v, d.rot, as<float>(m->p_side_k),
@@ -1957,8 +1947,8 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
             n += 3;
         } else {
             if (pair) {
-                // rows == T: `in` is sized for them. Attention rows in FP32
-                // become planes in a launch of their own; the rows' activation
+                // rows == T: `in` is sized for them. Attention rows become
+                // planes in a launch of their own; the rows' activation
                 // goes past the input planes, which gate/up's blocks still read.
                 PairRows act{};
                 act.planes = ws->planes + 2 * (uint64_t)in.padded * h;
@@ -1968,8 +1958,7 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                 PairRows gu_in = in;
                 gu_in.act_bound = d.act_bound;
                 gu_in.act_exps = act.exps;
-                if (!paired[i])
-                    HIP_FAIL(m, launch_norm_rows(s, attn, aw, nullptr, 0.0f, attn, aw, aw, T, &in));
+                HIP_FAIL(m, launch_pair_rows(s, attn, aw, aw, T, in));
                 HIP_FAIL(m, launch_gemm_pair(s, in, d.p_o, T, branch, h, *ws));
                 HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, post, kAttentionOffset, mpre,
                                                      1.0f, norm, h, h, T, &gu_in));

@@ -128,6 +128,10 @@ uint64_t pair_frag_elems(uint64_t rows, uint64_t cols);
 uint64_t pair_exp_count(uint64_t rows);
 // Rows of the planes for `tokens` rows (the consumer's tiles are whole).
 uint32_t pair_padded(uint64_t tokens);
+// FP32 rows (16-byte aligned, at most 8192 wide) into the planes, rows past
+// `rows` zero.
+hipError_t launch_pair_rows(hipStream_t, const float *x, uint64_t x_stride, uint64_t width,
+                            uint64_t rows, const PairRows &pair);
 // Fills p.frag and p.exps from p.rows x p.cols BF16 weights (16-byte aligned),
 // column c times 2^col_exps[c] (optional); norms (optional): each row's 2-norm.
 hipError_t launch_pair_weights(hipStream_t, const uint16_t *w, const PairWeight &p, float *norms,
@@ -148,8 +152,7 @@ hipError_t launch_gemm_pair_swiglu(hipStream_t, const PairRows &x, const PairWei
 // Multi-row RMSNorm; with branch: state += rms(branch) * (bf16(w) + offset).
 // With pair, the normalized rows go there instead of y, `pair->padded` rows
 // (those past `rows` zero; 16-byte-aligned rows of whole 32-column stages, at
-// most 8192 wide, hipErrorInvalidValue otherwise). Without w the rows are taken
-// as they are (pair only).
+// most 8192 wide, hipErrorInvalidValue otherwise).
 hipError_t launch_norm_rows(hipStream_t, const float *x, uint64_t x_stride, const uint16_t *w,
                             float offset, float *y, uint64_t y_stride, uint64_t width,
                             uint64_t rows, const PairRows *pair = nullptr);
@@ -277,16 +280,13 @@ bool prompt_attention_matrix(uint32_t dim, uint32_t qh, uint32_t kh);
 uint64_t prompt_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t qh, uint32_t kh,
                                   uint32_t dim, uint32_t window, int rotated);
 
-// The same attention on the fp16 matrix cores for prompts of more than 32
-// tokens, written as the O projection's input planes. scratch:
-// pair_attention_scratch bytes (256-byte aligned); v_exp: kh words set to
-// kPairNoExp. With a window the keys are rotated at their virtual rows.
-constexpr int32_t kPairNoExp = 126;
+// The same attention on the fp16 matrix cores, for prompts of more than 32
+// tokens and enough query rows. scratch: pair_attention_scratch bytes (256-byte aligned). With a window
+// the keys are rotated at their virtual rows.
 bool pair_attention_supported(uint32_t prefix, uint32_t tokens, uint32_t qh, uint32_t kh,
                               uint32_t dim);
 uint64_t pair_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t kh, uint32_t dim);
-hipError_t launch_pair_attention(hipStream_t, const PromptAttention &, void *scratch,
-                                 int32_t *v_exp, const PairRows &out);
+hipError_t launch_pair_attention(hipStream_t, const PromptAttention &, void *scratch);
 
 // Rotates cache rows [0, rows) of raw K into rotated K at their row position.
 hipError_t launch_rerotate(hipStream_t, const float *k_raw, float *k_rot, const float *table,

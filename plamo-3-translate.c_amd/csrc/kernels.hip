@@ -2194,6 +2194,69 @@ __device__ __forceinline__ void pair_row(const PairRows &p, uint32_t row, uint32
     }
 }
 
+// FP32 rows into the planes, one row per wave (at most 256 NV columns, held in
+// registers): the waves of a block write neighbouring rows, whose 64-byte
+// pieces make whole cache lines.
+template <int NV>
+__global__ __launch_bounds__(kThreads) void pair_rows_kernel(const float *x, uint64_t x_stride,
+                                                             uint32_t rows, uint32_t width,
+                                                             PairRows p) {
+    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= p.padded) return;
+    const float *xr = x + (uint64_t)min(row, rows - 1) * x_stride;
+    f32x4 v[NV];
+    float mx = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const uint32_t c = 4 * (lane + 64 * j);
+        v[j] = *(const f32x4 *)(xr + min(c, width - 4));
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[j][e] = row < rows ? v[j][e] : 0.0f;
+            mx = fmaxf(mx, __builtin_fabsf(v[j][e]));
+        }
+    mx = wave_max(mx);
+    const int ex = pair_exponent(__float_as_uint(mx));
+    const float scale = power_of_two(ex);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const uint32_t c = 4 * (lane + 64 * j);
+        if (c >= width) continue;
+        f16x4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            _Float16 h, l;
+            pair_split(v[j][e], scale, h, l);
+            hi[e] = h;
+            lo[e] = l;
+        }
+        const uint64_t at = pair_at(p.padded, row, c);
+        *(u32x2 *)(p.planes + at) = __builtin_bit_cast(u32x2, hi);
+        *(u32x2 *)(p.planes + at + (uint64_t)p.padded * kPairK) = __builtin_bit_cast(u32x2, lo);
+    }
+    if (lane == 0) p.exps[row] = ex;
+}
+
+hipError_t launch_pair_rows(hipStream_t stream, const float *x, uint64_t x_stride, uint64_t width,
+                            uint64_t rows, const PairRows &p) {
+    if (!rows) return hipSuccess;
+    if (!width || width % kPairK || width > 8192 || p.padded < rows || x_stride % 4 ||
+        ((uintptr_t)x & 15))
+        return hipErrorInvalidValue;
+    const unsigned grid = (p.padded + 3) / 4;
+    const uint32_t w = (uint32_t)width, n = (uint32_t)rows;
+    if (width <= 2048)
+        pair_rows_kernel<8><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+    else if (width <= 4096)
+        pair_rows_kernel<16><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+    else
+        pair_rows_kernel<32><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+    return hipGetLastError();
+}
+
 // Block: 32 weight rows. Rows past `rows` (the last group's padding) are zero.
 // norms (optional): each row's 2-norm. col_exps (optional): column c is taken
 // times 2^col_exps[c], at most 0.
@@ -2669,8 +2732,7 @@ __global__ __launch_bounds__(kThreads) void norm_rows_kernel(const float *x, uin
 // multiple of 4, at most 8192): every load goes out before the sum, where the
 // strided loop above waits on each in turn (C5 verify's first norm 15 us).
 // With pair.planes the normalized row goes there as a scaled pair of fp16 terms
-// instead of y; blocks past `rows` (up to pair.padded) write zeros. Without w
-// the row is taken as it is.
+// instead of y; blocks past `rows` (up to pair.padded) write zeros.
 template <int NV>
 __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, uint64_t x_stride,
                                                               const uint16_t *w, float offset,
@@ -2692,7 +2754,7 @@ __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, ui
         const uint32_t i = threadIdx.x + kThreads * j;
         const uint32_t c = (i < groups ? i : groups - 1) * 4;
         const f32x4 xv = *(const f32x4 *)(xr + c);
-        const u32x2 wv = w ? *(const u32x2 *)(w + c) : u32x2{0u, 0u};
+        const u32x2 wv = *(const u32x2 *)(w + c);
         v[j] = i < groups ? xv : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         g[j] = wv;
     }
@@ -2704,14 +2766,13 @@ __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, ui
             const float t = v[j][e] * v[j][e];
             ss = ss + t;
         }
-    const float inv = w ? block_inverse_from_partial(ss, width, red) : 1.0f;
+    const float inv = block_inverse_from_partial(ss, width, red);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const uint32_t i = threadIdx.x + kThreads * j;
         const uint32_t wb[4] = {g[j].x & 0xffffu, g[j].x >> 16, g[j].y & 0xffffu, g[j].y >> 16};
-        if (w)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[j][e] = (v[j][e] * inv) * (bf16f(wb[e]) + offset);
+        for (int e = 0; e < 4; ++e) v[j][e] = (v[j][e] * inv) * (bf16f(wb[e]) + offset);
         if (!pair.planes && i < groups) *(f32x4 *)(yr + 4 * i) = v[j];
     }
     if (pair.planes) pair_row<NV>(pair, blockIdx.x, groups, v, red);
@@ -2738,7 +2799,7 @@ hipError_t launch_norm_rows(hipStream_t stream, const float *x, uint64_t x_strid
                                                                 y_stride, wd, pr, n);
         return hipGetLastError();
     }
-    if (pair || !w) return hipErrorInvalidValue;
+    if (pair) return hipErrorInvalidValue;
     norm_rows_kernel<<<(unsigned)rows, kThreads, 0, stream>>>(x, x_stride, w, offset, y, y_stride,
                                                               (uint32_t)width);
     return hipGetLastError();
@@ -4296,37 +4357,47 @@ hipError_t launch_prompt_attention(hipStream_t stream, const PromptAttention &a)
 // the time. Against 64-bit results of the layers the error is the same.
 //
 // pair_kv_kernel first turns the layer's visible rows, 32 keys of one KV head
-// per block, into MFMA fragments (K and V^T, hi and lo) with one power of two
-// per tile each. The attention block is four waves, each 32 queries of one
+// per block, into MFMA fragments (K and V^T, hi and lo). K takes one power of
+// two per tile: its rows left an RMS norm, so their sizes are alike. V's rows
+// may differ by any factor, and a query must not lose bits to a row it does not
+// see. So a query's sums are in units of the largest V row among the keys it
+// has seen, rescaled when that grows, as with the running maximum: a tile whose
+// V rows stand within 2^kAlikeVExps of each other takes one power of two, in
+// any other each key has its own and the probabilities what it stands below the
+// largest. The output goes out in FP32, so that a row's own largest value
+// scales it for the O GEMM.
+// The attention block is four waves, each 32 queries of one
 // head of the KV head's group; the waves share the tile in LDS (double
 // buffered, loaded straight into it). S is formed transposed (keys by
 // queries), so a lane holds 16 keys of one query: the softmax needs one
 // exchange between lane halves per tile, and its values are, in place, the
 // B operand of V^T P (the keys of a fragment are permuted to match). Blocks
-// with the most keys are dispatched first; there are no key splits: the
-// output goes out once, as the O projection's input planes.
+// with the most keys are dispatched first; there are no key splits.
 //
 // Bound by what a wave does for a tile (48 products of 32 cycles, about 500
 // vector instructions around them) and by the causal triangle, whose longest
 // blocks end the launch. Measured per layer with pair_kv, against the FP32
-// form with its merge and the planes launch: 32/8 heads of 128 at 1900 tokens
-// 175 against 474 us, 443 tokens 40 against 60, 116 tokens 22 against 23;
-// 16/4 heads, 3500 tokens in a 2048 window, 187 against 701.
+// form with its merge: 32/8 heads of 128 at 1900 tokens 173 against 462 us, 443
+// tokens 39 against 57; 16/4 heads, 3500 tokens in a 2048 window, 183 against 676.
 constexpr uint32_t kPairKeys = 32;  // keys per tile
 constexpr int pair_kv_frags(int dim) { return dim / 16 * 2 * 2; }  // 1 KB fragments of K and V
 
+constexpr int kMostVExp = 100;   // of a row of zeros
+constexpr int kAlikeVExps = 6;   // costs a row as many of its 40 bits
+constexpr int kMixedTile = 1024;  // added to the exponent of a tile whose V rows are not alike
+
 struct PairAttention {
     PromptAttention a;
-    uint16_t *kv;      // [kh][tiles][K fragments | V fragments]
-    int32_t *kv_exps;  // [kh][tiles][K, V]
-    int32_t *v_exp;    // [kh]: the smallest V exponent (of the largest values)
+    uint16_t *kv;    // [kh][tiles][K fragments | V fragments]
+    int32_t *kv_exps;  // [kh][tiles][K, V]; V's of the largest row, + kMixedTile
+    int32_t *v_exps;   // [kh][tiles][key], of mixed tiles
     uint32_t tiles;
-    PairRows out;
 };
 
 template <int DIM>
 __global__ __launch_bounds__(kThreads) void pair_kv_kernel(PairAttention p) {
-    __shared__ float red[2][4];
+    __shared__ float red[4];
+    __shared__ int v_exp[kPairKeys];
     const PromptAttention &a = p.a;
     const uint32_t tile = blockIdx.x, kvh = blockIdx.y, width = a.kh * DIM;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -4339,44 +4410,53 @@ __global__ __launch_bounds__(kThreads) void pair_kv_kernel(PairAttention p) {
     // K: (key, 8 columns) per item; V: (column, 8 keys of a fragment's half).
     constexpr int N = kPairKeys * DIM / 8 / kThreads;
     float kx[N][8], vx[N][8];
-    float km = 0.0f, vm = 0.0f;
+    float km = 0.0f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         const uint32_t item = threadIdx.x + kThreads * i;
         const uint32_t key = item / (DIM / 8), c = item % (DIM / 8) * 8;
         const float *kr = row_of(a.k_cache, a.k_new, k0 + key) + c;
+        const float *vr = row_of(a.v_cache, a.v_new, k0 + key) + c;
         const f32x4 lo4 = *(const f32x4 *)kr, hi4 = *(const f32x4 *)(kr + 4);
+        const f32x4 vlo = *(const f32x4 *)vr, vhi = *(const f32x4 *)(vr + 4);
         const uint32_t d = item % DIM, kk = item / DIM / 2, h = item / DIM % 2;
         const bool live = k0 + key < total;
+        float vm = 0.0f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             kx[i][e] = live ? (e < 4 ? lo4[e] : hi4[e - 4]) : 0.0f;
+            km = fmaxf(km, __builtin_fabsf(kx[i][e]));
+            vm = fmaxf(vm, __builtin_fabsf(e < 4 ? vlo[e] : vhi[e - 4]));
             const uint32_t vk = k0 + 16 * kk + 8 * (e / 4) + 4 * h + e % 4;
             const float v = row_of(a.v_cache, a.v_new, vk)[d];
             vx[i][e] = vk < total ? v : 0.0f;
         }
+        // The DIM / 8 lanes of a key are neighbours.
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            km = fmaxf(km, __builtin_fabsf(kx[i][e]));
-            vm = fmaxf(vm, __builtin_fabsf(vx[i][e]));
-        }
+        for (int n = 1; n < DIM / 8; n *= 2) vm = fmaxf(vm, __shfl_xor(vm, n, 64));
+        if (c == 0) v_exp[key] = min(pair_exponent(__float_as_uint(live ? vm : 0.0f)), kMostVExp);
     }
     km = wave_max(km);
-    vm = wave_max(vm);
-    if (lane == 0) {
-        red[0][wave] = km;
-        red[1][wave] = vm;
-    }
+    if (lane == 0) red[wave] = km;
     __syncthreads();
-    km = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
-    vm = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
-    const int ke = pair_exponent(__float_as_uint(km)), ve = pair_exponent(__float_as_uint(vm));
-    const float ks = power_of_two(ke), vs = power_of_two(ve);
-    if (threadIdx.x == 0) {
-        p.kv_exps[(kvh * p.tiles + tile) * 2] = ke;
-        p.kv_exps[(kvh * p.tiles + tile) * 2 + 1] = ve;
-        (void)__hip_atomic_fetch_min(p.v_exp + kvh, ve, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    km = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const int ke = pair_exponent(__float_as_uint(km));
+    const float ks = power_of_two(ke);
+    // The V rows' exponents, from the largest row's to the smallest's (rows of
+    // zeros are alike with any).
+    int ve = kMostVExp, small = -126;
+#pragma unroll
+    for (uint32_t k = 0; k < kPairKeys; ++k) {
+        ve = min(ve, v_exp[k]);
+        small = max(small, v_exp[k] < kMostVExp ? v_exp[k] : -126);
     }
+    const bool mixed = small - ve > kAlikeVExps;
+    const uint32_t at = kvh * p.tiles + tile;
+    if (threadIdx.x == 0) {
+        p.kv_exps[2 * at] = ke;
+        p.kv_exps[2 * at + 1] = ve + (mixed ? kMixedTile : 0);
+    }
+    if (threadIdx.x < kPairKeys) p.v_exps[at * kPairKeys + threadIdx.x] = v_exp[threadIdx.x];
     uint16_t *frag = p.kv + (uint64_t)(kvh * p.tiles + tile) * pair_kv_frags(DIM) * 512;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
@@ -4397,7 +4477,8 @@ __global__ __launch_bounds__(kThreads) void pair_kv_kernel(PairAttention p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             _Float16 x, y;
-            pair_split(vx[i][e], vs, x, y);
+            const int xe = mixed ? v_exp[16 * kk + 8 * (e / 4) + 4 * h + e % 4] : ve;
+            pair_split(vx[i][e], power_of_two(xe), x, y);
             hi[e] = x;
             lo[e] = y;
         }
@@ -4438,6 +4519,7 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void pair_attention_kern
     const uint32_t token = t0 + col;
     const u32x4 *kv = (const u32x4 *)p.kv + (uint64_t)kvh * p.tiles * FR * 64 + lane;
     const int32_t *exps = p.kv_exps + (uint64_t)kvh * p.tiles * 2;
+    const int32_t *v_exps = p.v_exps + (uint64_t)kvh * p.tiles * kPairKeys + 4 * hf;
     // The KW tiles from `tile` on, each by its group (past the last: that again).
     auto load = [&](uint32_t tile, uint32_t buf) -> int {
         const uint32_t t = min(tile + part, last - 1);
@@ -4451,7 +4533,6 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void pair_attention_kern
         return exps[t * 2 + (lane & 1)];
     };
     int te = load(first, 0);
-    const int v_exp = p.v_exp[kvh];
     // Q as the B operand of each 16-column step, scaled per query.
     f16x8 qhi[KS], qlo[KS];
     int qe;
@@ -4490,10 +4571,13 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void pair_attention_kern
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[n][v] = 0.0f;
+    // The running maximum and sum, and the smallest V exponent (of the largest
+    // row) seen: o is in units of 2^-(v_run + 14).
     float m_run = ninf, l_run = 0.0f;
+    int v_run = kMostVExp;
     loads_landed<0>();
     for (uint32_t t = first, buf = 0; t < last; t += KW, buf ^= 1) {
-        const int ke = __builtin_amdgcn_readlane(te, 0), ve = __builtin_amdgcn_readlane(te, 1);
+        const int ke = __builtin_amdgcn_readlane(te, 0), tile_ve = __builtin_amdgcn_readlane(te, 1);
         if (t + KW < last) te = load(t + KW, buf ^ 1);
         const uint32_t tile = t + part;
         if (busy && tile >= lo && tile < hi) {
@@ -4526,24 +4610,51 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void pair_attention_kern
             }
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float m_new = fmaxf(m_run, mx);
-            if (__builtin_amdgcn_ballot_w64(m_new != m_run)) {
+            const bool mixed = tile_ve >= kMixedTile / 2;
+            // The smallest exponent of the keys the query sees; of the others
+            // the probabilities are zero at any scale.
+            int ve[16], v_new = mx == ninf ? v_run : min(v_run, tile_ve);
+            if (mixed) {
+                v_new = v_run;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    ve[v] = v_exps[tile * kPairKeys + 8 * (v / 4) + v % 4];
+                    v_new = sh[v] == ninf ? v_new : min(v_new, ve[v]);
+                }
+                v_new = min(v_new, __shfl_xor(v_new, 32, 64));
+            }
+            if (__builtin_amdgcn_ballot_w64(m_new != m_run || v_new != v_run)) {
                 // A query that has seen no key keeps zeros.
                 const float c = m_new == ninf ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+                const float oc = __builtin_ldexpf(c, v_new - v_run);
                 l_run *= c;
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) o[n][v] *= c;
+                    for (int v = 0; v < 16; ++v) o[n][v] *= oc;
                 m_run = m_new;
+                v_run = v_new;
             }
-            const float mm = m_run == ninf ? 0.0f : m_run;
-            // P scaled to 2^14 and to this tile's V exponent.
-            const float ps = power_of_two(max(14 + v_exp - ve, -126));
+            float mm = m_run == ninf ? 0.0f : m_run, counted = 1.0f;
+            // P scaled to 2^14, less what its key's V row stands below the
+            // largest seen: for the tile, or for each key in its score, whose
+            // weight is then counted here.
+            float ps = power_of_two(max(14 + min(v_run - tile_ve, 0), -126));
+            if (mixed) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    sh[v] -= mm;
+                    l_run += __builtin_amdgcn_exp2f(sh[v]);
+                    sh[v] += (float)min(v_run - ve[v], 0);
+                }
+                mm = counted = 0.0f;
+                ps = power_of_two(14);
+            }
             f16x8 phi[2], plo[2];
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const float pv = __builtin_amdgcn_exp2f(sh[v] - mm);
-                l_run += pv;
+                l_run = __builtin_fmaf(pv, counted, l_run);
                 _Float16 u, w;
                 pair_split(pv, ps, u, w);
                 phi[v / 8][v % 8] = u;
@@ -4573,8 +4684,8 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void pair_attention_kern
     float l = l_run + __shfl_xor(l_run, 32, 64);
     if constexpr (KW == 2) {
         // The second group's sums through LDS (every load has landed and every
-        // tile is done): [wave][16 NT + 2][64].
-        float *x = (float *)lds + wave * (16 * NT + 2) * 64 + lane;
+        // tile is done): [wave][16 NT + 3][64].
+        float *x = (float *)lds + wave * (16 * NT + 3) * 64 + lane;
         if (part) {
 #pragma unroll
             for (int n = 0; n < NT; ++n)
@@ -4582,6 +4693,7 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void pair_attention_kern
                 for (int v = 0; v < 16; ++v) x[(16 * n + v) * 64] = o[n][v];
             x[16 * NT * 64] = m_run;
             x[(16 * NT + 1) * 64] = l;
+            x[(16 * NT + 2) * 64] = __int_as_float(v_run);
         }
         __syncthreads();
         if (part) return;
@@ -4589,35 +4701,25 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void pair_attention_kern
         const float c0 = m_run == ninf ? 0.0f : __builtin_amdgcn_exp2f(m_run - m);
         const float c1 = m1 == ninf ? 0.0f : __builtin_amdgcn_exp2f(m1 - m);
         l = l * c0 + x[(16 * NT + 1) * 64] * c1;
+        const int v1 = __float_as_int(x[(16 * NT + 2) * 64]), v0 = v_run;
+        v_run = min(v0, v1);
+        const float o0 = __builtin_ldexpf(c0, v_run - v0), o1 = __builtin_ldexpf(c1, v_run - v1);
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) o[n][v] = o[n][v] * c0 + x[(16 * n + v) * 64] * c1;
+            for (int v = 0; v < 16; ++v) o[n][v] = o[n][v] * o0 + x[(16 * n + v) * 64] * o1;
     }
     if (!busy || token >= a.tokens) return;
-    // An output is a mean of V rows: below 2^(15 - v_exp) for every head, so
-    // the smallest V exponent of the KV heads scales the row for the O GEMM.
-    int re = v_exp;
-    for (uint32_t k = 0; k < a.kh; ++k) re = min(re, p.v_exp[k]);
-    if (h == 0 && hf == 0) p.out.exps[token] = re;
-    const float rs = power_of_two(re), inv = power_of_two(-14);
+    const float unit_out = power_of_two(-14 - v_run);
+    float *out = a.out + ((uint64_t)token * a.qh + h) * DIM + 4 * hf;
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int v = 0; v < 16; v += 4) {
-            f16x4 ph, pl;
+            f32x4 y;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float y = __builtin_ldexpf(o[n][v + e] * inv, -v_exp) / l;
-                _Float16 u, w;
-                pair_split(y, rs, u, w);
-                ph[e] = u;
-                pl[e] = w;
-            }
-            const uint64_t at = pair_at(p.out.padded, token, h * DIM + 32 * n + 2 * v + 4 * hf);
-            *(u32x2 *)(p.out.planes + at) = __builtin_bit_cast(u32x2, ph);
-            *(u32x2 *)(p.out.planes + at + (uint64_t)p.out.padded * kPairK) =
-                __builtin_bit_cast(u32x2, pl);
+            for (int e = 0; e < 4; ++e) y[e] = o[n][v + e] * unit_out / l;
+            *(f32x4 *)(out + 32 * n + 2 * v) = y;
         }
 }
 
@@ -4646,31 +4748,37 @@ static uint32_t pair_kv_tiles(uint32_t prefix, uint32_t tokens) {
 }
 
 // From 33 tokens, unless a long cached prefix outweighs them: one block walks
-// its queries' keys alone, where the FP32 form spreads them over splits.
+// its queries' keys alone, where the FP32 form spreads them over splits. Its two
+// launches take 18 us at the least, where the FP32 form, which covers most
+// groups, takes 15 to 17 up to some number of query rows (us per layer, this
+// form and that, heads of 128): 32/8 heads 21.4 and 17.6 at 116 tokens, 23.7 and
+// 24.6 at 160; 48/8 heads 21.3 and 21.0 at 96, 21.0 and 22.0 at 116; 16/4 heads
+// 28.7 and 24.6 at 256, 32.1 and 31.6 at 320.
+constexpr uint64_t kPairQueryRows = 5120;
 bool pair_attention_supported(uint32_t prefix, uint32_t tokens, uint32_t qh, uint32_t kh,
                               uint32_t dim) {
-    return tokens > 32 && prefix <= 4 * tokens && kh && qh % kh == 0 && (dim == 64 || dim == 128) &&
-           (qh * dim) % kPairK == 0 && kh <= 65535;
+    if (tokens <= 32 || prefix > 4 * tokens || !kh || qh % kh || (dim != 64 && dim != 128) ||
+        kh > 65535)
+        return false;
+    return (uint64_t)tokens * qh >= kPairQueryRows || !prompt_attention_matrix(dim, qh, kh);
 }
 
 uint64_t pair_attention_scratch(uint32_t prefix, uint32_t tokens, uint32_t kh, uint32_t dim) {
     const uint64_t tiles = (uint64_t)kh * pair_kv_tiles(prefix, tokens);
-    return tiles * pair_kv_frags((int)dim) * 1024 + tiles * 8;
+    return tiles * (pair_kv_frags((int)dim) * 1024 + kPairKeys * 4 + 8);
 }
 
-hipError_t launch_pair_attention(hipStream_t stream, const PromptAttention &a, void *scratch,
-                                 int32_t *v_exp, const PairRows &out) {
-    if (!pair_attention_supported(a.prefix, a.tokens, a.qh, a.kh, a.dim) || out.padded < a.tokens ||
+hipError_t launch_pair_attention(hipStream_t stream, const PromptAttention &a, void *scratch) {
+    if (!pair_attention_supported(a.prefix, a.tokens, a.qh, a.kh, a.dim) ||
         (a.window && !a.rotated))
         return hipErrorInvalidValue;
     PairAttention p{};
     p.a = a;
     p.tiles = pair_kv_tiles(a.prefix, a.tokens);
     p.kv = (uint16_t *)scratch;
-    p.kv_exps = (int32_t *)((char *)scratch +
-                            (uint64_t)a.kh * p.tiles * pair_kv_frags((int)a.dim) * 1024);
-    p.v_exp = v_exp;
-    p.out = out;
+    const uint64_t tiles = (uint64_t)a.kh * p.tiles;
+    p.v_exps = (int32_t *)((char *)scratch + tiles * pair_kv_frags((int)a.dim) * 1024);
+    p.kv_exps = p.v_exps + tiles * kPairKeys;
     const uint32_t units = (a.tokens + 31) / 32 * (a.qh / a.kh);
     const dim3 prep(p.tiles, a.kh), grid(a.kh, (units + 3) / 4);
     if (grid.y > 65535) return hipErrorInvalidValue;

@@ -105,6 +105,10 @@ hipError_t launch_pair_weights(hipStream_t s, const uint16_t *, const PairWeight
                                const int32_t *) {
     return queue(s);
 }
+hipError_t launch_pair_rows(hipStream_t s, const float *, uint64_t, uint64_t, uint64_t,
+                            const PairRows &) {
+    return queue(s);
+}
 hipError_t launch_pair_balance(hipStream_t s, const float *, uint64_t, int32_t *, float *) {
     return queue(s);
 }
@@ -144,10 +148,7 @@ uint64_t prompt_attention_scratch(uint32_t, uint32_t, uint32_t, uint32_t, uint32
 }
 bool pair_attention_supported(uint32_t, uint32_t, uint32_t, uint32_t, uint32_t) { return true; }
 uint64_t pair_attention_scratch(uint32_t, uint32_t, uint32_t, uint32_t) { return 256; }
-hipError_t launch_pair_attention(hipStream_t s, const PromptAttention &, void *, int32_t *,
-                                 const PairRows &) {
-    return queue(s);
-}
+hipError_t launch_pair_attention(hipStream_t s, const PromptAttention &, void *) { return queue(s); }
 hipError_t launch_window_store(hipStream_t s, float *, float *, float *, const float *,
                                const float *, uint64_t, const float *, float *, uint64_t, uint64_t,
                                uint64_t, uint32_t, uint32_t) {

@@ -328,9 +328,13 @@ def test_eager_decode_matches_graph(monkeypatch):
 # head) units leave waves of a block idle, prompts of one tile and a row, of
 # whole tiles, a prefix of four prompts (its limit) and one past it, and grids
 # of more than one block per CU (one group of waves per block instead of two).
+# Few query rows (tokens x heads below 5120) take the FP32 form at the groups it
+# covers: the first rows stand on its side, the others on that of the pairs.
 @pytest.mark.parametrize("qh,kh,dim,prefix,tokens", [
     (6, 3, 128, 0, 33), (6, 1, 64, 0, 65), (4, 4, 64, 160, 40), (4, 4, 64, 161, 40),
     (3, 3, 64, 5, 129), (16, 1, 128, 7, 96), (32, 32, 64, 0, 1030), (16, 4, 128, 3, 2050),
+    (5, 1, 64, 0, 33), (3, 1, 128, 0, 65), (128, 64, 64, 160, 40), (128, 64, 64, 161, 40),
+    (102, 51, 64, 0, 51), (60, 60, 64, 5, 129), (64, 4, 128, 7, 96), (102, 17, 64, 0, 64),
 ])
 def test_prompt_pair_attention(qh, kh, dim, prefix, tokens):
     say(f"pair attention {qh}/{kh}x{dim} prefix={prefix} tokens={tokens}")
@@ -424,6 +428,9 @@ def test_decode_split_merge(rows):
     (8, 2, 128, 40, 0, 100), (8, 2, 128, 40, 12, 45), (4, 4, 64, 17, 18, 33),
     (12, 2, 128, 32, 33, 2), (16, 1, 64, 300, 3, 700), (8, 4, 128, 64, 50, 17),
     (16, 2, 64, 5, 6, 300), (16, 2, 128, 70, 12, 75),
+    # On the fp16 pairs (enough query rows).
+    (64, 16, 128, 40, 0, 100), (52, 26, 64, 17, 18, 130), (36, 6, 128, 5, 6, 150),
+    (64, 4, 64, 64, 50, 97),
 ])
 @pytest.mark.parametrize("pinned", [False, True])
 def test_past_the_window(qh, kh, dim, window, prefix, tokens, pinned):
@@ -535,9 +542,9 @@ def test_edited_full_windows(pinned):
 # A prompt without its states (only the last row feeds the logits) at groups
 # the fp16-pair attention takes and the FP32 matrix-core form does not, and at
 # groups both take.
-@pytest.mark.parametrize("qh,kh,dim", [(3, 1, 128), (6, 2, 64), (5, 1, 64), (14, 2, 128), (8, 2, 128),
-                                       (6, 1, 128)])
-@pytest.mark.parametrize("prefix,tokens", [(0, 33), (9, 70), (12, 300)])
+@pytest.mark.parametrize("qh,kh,dim", [(3, 1, 128), (6, 2, 64), (5, 1, 64), (14, 2, 128),
+                                       (64, 16, 128), (60, 10, 128)])
+@pytest.mark.parametrize("prefix,tokens", [(0, 33), (9, 90), (12, 300)])
 def test_prompt_last_row(qh, kh, dim, prefix, tokens):
     say(f"last row {qh}/{kh}x{dim} prefix={prefix} tokens={tokens}")
     syn = plamo_hip.Synthetic(256, 2, qh, kh, dim, 96, 300, window=2304, global_capacity=2304,
@@ -557,6 +564,54 @@ def test_prompt_last_row(qh, kh, dim, prefix, tokens):
                     gate(gpu.normalized().copy(), cpu.normalized().copy(), "normalized")
         info = be.info()
         assert info.errors == 0 and info.cpu_fallbacks == 0, info.note.decode()
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
+
+
+# A prompt in which a run of tokens has V rows some 2^24 times the others' (their
+# embedding alone reaches a column of the V projection): the tokens before them,
+# in their key tiles and in earlier ones, are as close to the oracle as without
+# them, and those after them, which see them, agree with the oracle as well.
+# Runs of one, of part of a tile, and of whole tiles.
+@pytest.mark.parametrize("qh,kh,dim,prefix,tokens,at,run", [
+    (52, 26, 64, 0, 100, 80, 1), (24, 6, 128, 12, 300, 290, 1), (9, 3, 64, 5, 60, 59, 1),
+    (16, 16, 64, 0, 1030, 700, 1), (32, 8, 128, 12, 200, 84, 70), (42, 7, 64, 7, 130, 25, 105),
+    (16, 16, 64, 5, 1030, 707, 300), (5, 1, 128, 0, 90, 40, 20),
+])
+def test_prompt_attention_large_value_rows(qh, kh, dim, prefix, tokens, at, run):
+    say(f"large V rows {qh}/{kh}x{dim} prefix={prefix} tokens={tokens} at={at} run={run}")
+    hidden, vocab, special = 256, 300, 299
+    syn = plamo_hip.Synthetic(hidden, 2, qh, kh, dim, 96, vocab, window=2304, global_capacity=2304,
+                              pattern=2, embedding_std=1.0, seed=qh)
+    gpu, cpu = syn.instance(), syn.instance()
+    emb = np.ctypeslib.as_array(gpu.model.embedding, shape=(vocab, hidden))
+    emb[:, 0] = 0
+    emb[special] = 0
+    emb[special, 0] = 0x3f80  # 1.0
+    qkv = np.ctypeslib.as_array(gpu.layer(0).mixer.contents.qkv.contents.weight,
+                                shape=((qh + 2 * kh) * dim, hidden))
+    v = qkv[(qh + kh) * dim:]
+    v[:, 0] = np.where(v[:, 0] & 0x7fff, v[:, 0] + np.uint16(22 << 7), 0)  # 2^4 from the norm
+    be = plamo_hip.Backend(syn)
+    try:
+        ids = [(j * 13 + 5) % 290 for j in range(prefix + tokens)]
+        ids[prefix + at:prefix + at + run] = [special] * run
+        for part in (ids[:prefix], ids[prefix:]):
+            if not part:
+                continue
+            actual = np.zeros((len(part), hidden), np.float32)
+            expected = np.zeros((len(part), hidden), np.float32)
+            assert be.prefill(gpu, part, actual) == 1
+            assert oracle_lib.prefill(cpu, part, expected)
+            gate(actual, expected, "all prompt states")
+        before, _ = gate(actual[:at], expected[:at], "states before the rows")
+        say(f"before them {before:.3g}")
+        # Without them 2e-7 to 3.5e-7 (sums of up to 1030 terms in FP32).
+        assert before <= 1e-6
+        compare(gpu, cpu)
     finally:
         be.close()
         gpu.close()
