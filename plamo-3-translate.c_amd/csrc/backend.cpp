@@ -262,12 +262,15 @@ int fail(plamo_metal *m) {
             return problem(m, "%s: %s", #call, hipGetErrorString(e_));                             \
     } while (0)
 
+bool give_back_pair(plamo_metal *m);
+
 template <typename T>
 T *dev_alloc(plamo_metal *m, uint64_t count) {
     void *p = nullptr;
     uint64_t bytes = count * sizeof(T);
     if (!bytes) bytes = 16;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
+    if (hipMalloc(&p, bytes) != hipSuccess &&
+        (!give_back_pair(m) || hipMalloc(&p, bytes) != hipSuccess)) {
         (void)hipGetLastError();
         problem(m, "cannot allocate %llu bytes of HBM", (unsigned long long)bytes);
         return nullptr;
@@ -282,6 +285,19 @@ void dev_free(plamo_metal *m, void *p) {
     auto it = std::find(m->allocations.begin(), m->allocations.end(), p);
     if (it != m->allocations.end()) m->allocations.erase(it);
     (void)hipFree(p);
+}
+
+// The prompts' weight fragments are memory that only speed needs: an allocation
+// that does not fit beside them takes their place, and prompts run from the
+// BF16 weights from then on.
+bool give_back_pair(plamo_metal *m) {
+    (void)hipGetLastError();
+    if (!m->pair_block) return false;
+    (void)hipStreamSynchronize(m->stream);
+    dev_free(m, m->pair_block);
+    m->pair_block = nullptr;
+    m->pair_ready = false;
+    return true;
 }
 
 bool ensure(plamo_metal *m, Buffer &b, uint64_t bytes) {
@@ -1713,6 +1729,8 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         if (!ensure_kv_rows(m, d, rows) || !ensure_rope_rows(m, m->ropes[d.rope], rows)) return -1;
         m->params_host->count[i] = (uint32_t)c->count;
     }
+    // An allocation above has taken the fragments' memory: sized again without.
+    if (pair && !m->pair_ready) return run_prompt(m, model, ids, T, states, verify);
     m->params_host->tokens = (uint32_t)T;
     *m->status_host = 0;
     memcpy(m->ids_host, ids, T * 4);

@@ -293,6 +293,41 @@ void lone_window(uint64_t layer) {
     }
 }
 
+// Device memory that holds the weights twice, but not the rows of a longer
+// context beside both: the fragments make room, in a prompt, in a decode step
+// and for weights preloaded later.
+void fragments_make_room() {
+    for (int turn = 0; turn < 3; ++turn) {
+        host::device_limit = 96 << 20;
+        Request q(3, 400, 3, true);
+        check(plamo_metal_prepare_model(q.metal, q.model) == 1, "prepare");
+        check(q.metal->pair_ready, "fragments laid out", 0, turn);
+        std::vector<uint32_t> ids(300, 1);
+        std::vector<uint16_t> weights(1 << 20);
+        check(plamo_metal_prefill(q.metal, q.model, ids.data(), 20, nullptr) == 1, "prompt");
+        check(q.metal->pair_ready, "fragments kept", 0, turn);
+        // Not a byte more; for the step, three layers' rows doubled less half
+        // of the fragments.
+        host::device_limit = host::device_bytes;
+        if (turn == 1)
+            host::device_limit += (400 << 10) - host::device[q.metal->pair_block] / 2;
+        if (turn == 0) {
+            check(plamo_metal_prefill(q.metal, q.model, ids.data(), 24, nullptr) == 1, "longer prompt");
+        } else if (turn == 1) {
+            q.fill(256, 10.0f);
+            check(plamo_metal_forward(q.metal, q.model, 1) == 1, "step past the rows");
+        } else {
+            check(plamo_metal_preload(q.metal, weights.data(), 1 << 10) == 1, "preload");
+        }
+        check(!q.metal->pair_ready && !q.metal->pair_block, "fragments given back", 0, turn);
+        plamo_metal_info info;
+        plamo_metal_get_info(q.metal, &info);
+        check(info.errors == 0, info.note);
+        check(plamo_metal_prefill(q.metal, q.model, ids.data(), 7, nullptr) == 1, "next prompt");
+    }
+    host::device_limit = ~(size_t)0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -308,6 +343,8 @@ int main(int argc, char **argv) {
         failed_launch(false);
     else if (what == "lone_window")
         for (uint64_t layer = 0; layer < 8; ++layer) lone_window(layer);
+    else if (what == "fragments_make_room")
+        fragments_make_room();
     else
         check(false, "unknown scenario");
     printf("ok\n");

@@ -44,6 +44,8 @@ def host_backend(tmp_path_factory):
     "failed_launch", "failed_launch_pageable",
     # A single full window among layers whose windows are not full.
     "lone_window",
+    # An allocation that fits only without the prompts' weight fragments.
+    "fragments_make_room",
 ])
 def test_host_side(host_backend, scenario):
     r = subprocess.run([str(host_backend), scenario], capture_output=True, text=True, timeout=120,
