@@ -1674,10 +1674,9 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
     if (!sync_from_host(m, model, stale, !verify)) return -1;
     if (!ensure_prompt(m, model, T) || !ensure_window_scratch(m, model)) return -1;
     const bool pair = T >= kPairTokens && m->pair_ready;
-    // Planes room for the widest projection input, and for the fp16 planes of
-    // the gate/up GEMM's input and output side by side.
-    const GemmWorkspace *ws = gemm_workspace(
-        m, T, std::max({h, m->max_attention, m->max_inter, pair ? h + m->max_inter : 0}));
+    // Planes room for the widest projection input, and for the planes of the
+    // gate/up GEMM's input and output side by side.
+    const GemmWorkspace *ws = gemm_workspace(m, T, std::max(m->max_attention, h + m->max_inter));
     if (!ws) return -1;
     if (verify && !m->v_host && !alloc_verify(m, L, h, V)) return -1;
     // wide[i]: the rows overflow a sliding window and the matrix-core
@@ -1761,6 +1760,12 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         in.padded = pair_padded(T);
     }
     const PairRows *norm_pair = pair ? &in : nullptr;
+    // Without, the BF16 planes, where the split GEMM takes the rows.
+    bool splittable = !pair && h <= 8192;
+    for (const Layer &d : m->layers)
+        splittable = splittable && !(((uintptr_t)d.qkv | (uintptr_t)d.gu | (uintptr_t)d.down) & 15);
+    SplitRows split{ws->planes, splittable ? gemm_planes_rows(T, h, ws) : 0};
+    const SplitRows *norm_split = split.padded ? &split : nullptr;
     // Host-mirror copies of finished layers' cache rows not yet enqueued.
     struct MirrorRows {
         float *host;
@@ -1779,7 +1784,8 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         const uint64_t qkv_w = (uint64_t)(d.qh + 2 * d.kh) * d.dim, aw = (uint64_t)d.qh * d.dim;
         const bool last_row_only = last_row && i + 1 == L, last_query_only = last_query && i + 1 == L;
         if (!normed) {
-            HIP_FAIL(m, launch_norm_rows(s, state, h, pre, 1.0f, norm, h, h, T, norm_pair));
+            HIP_FAIL(m, launch_norm_rows(s, state, h, pre, 1.0f, norm, h, h, T, norm_pair,
+                                         norm_split));
             ++n;
         }
         normed = false;
@@ -1795,7 +1801,8 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
         } else if (pair)
             HIP_FAIL(m, launch_gemm_pair(s, in, d.p_qkv, T, qkv, qkv_w, *ws));
         else
-            HIP_FAIL(m, launch_gemm(s, norm, h, d.qkv, qkv_w, h, T, qkv, qkv_w, ws));
+            HIP_FAIL(m, launch_gemm(s, norm, h, d.qkv, qkv_w, h, T, qkv, qkv_w, ws,
+                                    norm_split != nullptr));
         ++n;
         if (m->upload_pending) {  // cached rows are read from here on
             HIP_FAIL(m, hipStreamWaitEvent(s, m->upload_event, 0));
@@ -1984,21 +1991,32 @@ int run_prompt(plamo_metal *m, struct model *model, const uint32_t *ids, uint64_
                 HIP_FAIL(m, launch_gemm_pair(s, act, d.p_down, T, branch, h, *ws));
             } else {
                 HIP_FAIL(m, launch_gemm(s, attn + first * aw, aw, d.o, h, aw, rows, branch, h, ws));
+                // rows == T here too; down reads the planes that gate/up writes
+                // past its own.
                 if (fuse_rows) {
                     HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, post, kAttentionOffset,
-                                                         mpre, 1.0f, norm, h, h, rows));
+                                                         mpre, 1.0f, norm, h, h, rows, nullptr,
+                                                         norm_split));
                 } else {
                     HIP_FAIL(m, launch_residual_rows(s, st, branch, post, kAttentionOffset, h, rows));
                     HIP_FAIL(m, launch_norm_rows(s, st, h, mpre, 1.0f, norm, h, h, rows));
                     ++n;
                 }
-                HIP_FAIL(m, launch_gemm_swiglu(s, norm, h, d.gu, d.inter, h, rows, act, gu, ws));
-                HIP_FAIL(m, launch_gemm(s, act, d.inter, d.down, h, d.inter, rows, branch, h, ws));
+                GemmWorkspace down_ws = *ws;
+                uint16_t *act_planes = norm_split ? gemm_swiglu_planes(d.inter, h, rows, ws) : nullptr;
+                if (act_planes) {
+                    down_ws.planes = act_planes;
+                    down_ws.plane_elems -= (uint64_t)(act_planes - ws->planes);
+                }
+                HIP_FAIL(m, launch_gemm_swiglu(s, norm, h, d.gu, d.inter, h, rows, act, gu, ws,
+                                              norm_split != nullptr, act_planes));
+                HIP_FAIL(m, launch_gemm(s, act, d.inter, d.down, h, d.inter, rows, branch, h, &down_ws,
+                                        act_planes != nullptr));
             }
             if (fuse_rows && i + 1 < L) {
                 HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, mpost, kMlpOffset,
                                                      m->layers[i + 1].norms, 1.0f, norm, h, h,
-                                                     rows, norm_pair));
+                                                     rows, norm_pair, norm_split));
                 normed = true;
             } else if (fuse_rows && verify) {
                 HIP_FAIL(m, launch_residual_norm_rows(s, st, branch, mpost, kMlpOffset,

@@ -85,6 +85,13 @@ struct GemmSplit {
     uint32_t *counters;
     uint16_t *planes;
     uint32_t xcd_group;  // nonzero: the M tiles of a weight tile share an XCD (see the kernel)
+    // Nonzero (the intermediate size I): the rows are a gate/up pair [2I]
+    // and each tile takes gate and up rows of the same intermediate columns;
+    // the epilogue writes silu(gate) * up as the BF16 planes `act` (rows
+    // padded to act_tp) instead of y.
+    uint32_t swiglu;
+    uint16_t *act;
+    uint32_t act_tp;
 };
 constexpr uint64_t kGemmPartialFloats = 16ull << 20;  // 64 MiB
 constexpr uint32_t kGemmCounters = 8192;
@@ -95,9 +102,20 @@ uint64_t gemm_plane_elems(uint64_t tokens, uint64_t cols);
 // the decode GEMV. Otherwise, with a workspace, more than one token and K a
 // multiple of 64: BF16 matrix cores on the exact three-term split of X; else
 // FP32 MFMA with BF16 weights widened in LDS.
+// planes_ready: the BF16 planes of X for the matrix-core path are already in
+// ws->planes (written by a norm with SplitRows of gemm_planes_rows(tokens, cols,
+// ws) rows, or by launch_gemm_swiglu), and x is not read; other paths fail.
 hipError_t launch_gemm(hipStream_t, const float *x, uint64_t x_stride, const uint16_t *w,
                        uint64_t rows, uint64_t cols, uint64_t tokens, float *y,
-                       uint64_t y_stride, const GemmWorkspace *ws);
+                       uint64_t y_stride, const GemmWorkspace *ws, bool planes_ready = false);
+// The padded rows of the BF16 planes launch_gemm's matrix-core path reads for
+// `tokens` rows of `cols` columns, or 0 when another path takes the call.
+uint32_t gemm_planes_rows(uint64_t tokens, uint64_t cols, const GemmWorkspace *ws);
+// Rows of X as those planes: [cols / 32][hi, mid, lo][padded][32], exact.
+struct SplitRows {
+    uint16_t *planes;
+    uint32_t padded;
+};
 
 // A projection's weights as scaled fp16 fragments for launch_gemm_pair, and
 // each row's exponent (value = fragment * 2^-exps[row]); rows padded to 32,
@@ -152,18 +170,21 @@ hipError_t launch_gemm_pair_swiglu(hipStream_t, const PairRows &x, const PairWei
 // Multi-row RMSNorm; with branch: state += rms(branch) * (bf16(w) + offset).
 // With pair, the normalized rows go there instead of y, `pair->padded` rows
 // (those past `rows` zero; 16-byte-aligned rows of whole 32-column stages, at
-// most 8192 wide, hipErrorInvalidValue otherwise).
+// most 8192 wide, hipErrorInvalidValue otherwise); with split likewise, for rows
+// of whole 64-column steps.
 hipError_t launch_norm_rows(hipStream_t, const float *x, uint64_t x_stride, const uint16_t *w,
                             float offset, float *y, uint64_t y_stride, uint64_t width,
-                            uint64_t rows, const PairRows *pair = nullptr);
+                            uint64_t rows, const PairRows *pair = nullptr,
+                            const SplitRows *split = nullptr);
 // launch_residual_rows followed by launch_norm_rows of the updated rows into
-// norm, in one launch (width <= 8192; hipErrorInvalidValue otherwise), pair as
-// launch_norm_rows.
+// norm, in one launch (width <= 8192; hipErrorInvalidValue otherwise), pair and
+// split as launch_norm_rows.
 hipError_t launch_residual_norm_rows(hipStream_t, float *state, const float *branch,
                                      const uint16_t *wr, float off_r, const uint16_t *wn,
                                      float off_n, float *norm, uint64_t norm_stride,
                                      uint64_t width, uint64_t rows,
-                                     const PairRows *pair = nullptr);
+                                     const PairRows *pair = nullptr,
+                                     const SplitRows *split = nullptr);
 hipError_t launch_residual_rows(hipStream_t, float *state, const float *branch,
                                 const uint16_t *w, float offset, uint64_t width, uint64_t rows);
 hipError_t launch_swiglu_rows(hipStream_t, const float *gate_up, float *out,
@@ -171,10 +192,17 @@ hipError_t launch_swiglu_rows(hipStream_t, const float *gate_up, float *out,
 // act[t, i] = silu(g) * u of the gate/up projection (rows i and
 // intermediate + i of w): the token GEMV writes act directly; other shapes
 // go through launch_gemm into gate_up ([tokens][2 * intermediate]) and
-// launch_swiglu_rows.
+// launch_swiglu_rows. With act_planes (gemm_swiglu_planes' place, not null) the
+// GEMM's epilogue writes the activation there alone, as the planes of a
+// launch_gemm with planes_ready.
 hipError_t launch_gemm_swiglu(hipStream_t, const float *x, uint64_t x_stride, const uint16_t *w,
                               uint64_t intermediate, uint64_t cols, uint64_t tokens, float *act,
-                              float *gate_up, const GemmWorkspace *ws);
+                              float *gate_up, const GemmWorkspace *ws, bool planes_ready = false,
+                              uint16_t *act_planes = nullptr);
+// Where in the workspace that is, past the input's planes; null when the shape
+// or the workspace (of cols + intermediate columns) does not allow it.
+uint16_t *gemm_swiglu_planes(uint64_t intermediate, uint64_t cols, uint64_t tokens,
+                             const GemmWorkspace *ws);
 
 // Q/K head RMSNorm + RoPE + cache append for `tokens` rows of one layer.
 struct QkvPost {

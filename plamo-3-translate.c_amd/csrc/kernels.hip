@@ -1083,6 +1083,39 @@ __device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) {
 __device__ __forceinline__ uint32_t swizzle(uint32_t r, uint32_t q) {
     return q ^ ((r ^ (r >> 2)) & 3);
 }
+// Columns c .. c + 3 of row `row` into the BF16 planes of launch_gemm's
+// matrix-core path (the layout split_planes_kernel writes: [c / 32][plane]
+// [padded row][c % 32], the exact three-term split).
+__device__ __forceinline__ void write_planes4(uint16_t *planes, uint32_t padded, uint32_t row,
+                                              uint32_t c, f32x4 v) {
+    uint32_t h[4], md[4], lo[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        h[e] = __float_as_uint(v[e]) & 0xffff0000u;
+        const float r = v[e] - __uint_as_float(h[e]);
+        md[e] = __float_as_uint(r) & 0xffff0000u;
+        lo[e] = __float_as_uint(r - __uint_as_float(md[e]));
+    }
+    const uint64_t at = ((uint64_t)(c / kSplitBK) * 3 * padded + row) * kSplitBK + c % kSplitBK;
+    const uint64_t pl = (uint64_t)padded * kSplitBK;
+    *(u32x2 *)(planes + at) = u32x2{pack_hi16(h[0], h[1]), pack_hi16(h[2], h[3])};
+    *(u32x2 *)(planes + at + pl) = u32x2{pack_hi16(md[0], md[1]), pack_hi16(md[2], md[3])};
+    *(u32x2 *)(planes + at + 2 * pl) = u32x2{pack_hi16(lo[0], lo[1]), pack_hi16(lo[2], lo[3])};
+}
+// One column's value: the same three terms as write_planes4.
+__device__ __forceinline__ void write_planes1(uint16_t *planes, uint32_t padded, uint32_t row,
+                                              uint32_t c, float v) {
+    const uint32_t h = __float_as_uint(v) & 0xffff0000u;
+    const float r = v - __uint_as_float(h);
+    const uint32_t md = __float_as_uint(r) & 0xffff0000u;
+    const uint32_t lo = __float_as_uint(r - __uint_as_float(md));
+    const uint64_t at = ((uint64_t)(c / kSplitBK) * 3 * padded + row) * kSplitBK + c % kSplitBK;
+    const uint64_t pl = (uint64_t)padded * kSplitBK;
+    planes[at] = (uint16_t)(h >> 16);
+    planes[at + pl] = (uint16_t)(md >> 16);
+    planes[at + 2 * pl] = (uint16_t)(lo >> 16);
+}
+
 __global__ __launch_bounds__(256) void split_planes_kernel(const float *x, uint64_t ldx,
                                                            uint32_t rows, uint32_t padded,
                                                            uint32_t k, uint16_t *planes) {
@@ -1156,12 +1189,21 @@ __global__ __launch_bounds__(64 * GM * GN, (WN > 2 || GM * GN > 4) ? 1 : 2) void
         asrc[i] = g.planes + ((uint64_t)p * g.tp + m0 + r) * kSplitBK + 8 * q;
         adst[i] = R * 4 + swizzle(R, q);
     }
+    // With swiglu, tile row r of wave column wn and 32-row group j takes the
+    // gate (j even) or up (j odd) row of intermediate column
+    // bn BN/2 + wn 16 WN + (j / 2) 32 + r % 32: a lane's accumulators j and
+    // j + 1 then hold the gate and up sums of one column.
     const uint16_t *wsrc[WPT];
     uint32_t wdst[WPT];
 #pragma unroll
     for (int i = 0; i < WPT; ++i) {
         const uint32_t G = threadIdx.x + NT * i, r = G / 4, q = G % 4;
-        const uint32_t row = min(n0 + r, g.n - 1);
+        uint32_t row = min(n0 + r, g.n - 1);
+        if (g.swiglu) {
+            const uint32_t j = r / 32 % WN;
+            const uint32_t col = bn * (BN / 2) + r / (32 * WN) * (16 * WN) + j / 2 * 32 + r % 32;
+            row = (j & 1) ? g.swiglu + col : col;
+        }
         wsrc[i] = g.w + (uint64_t)row * g.k + 8 * q;
         wdst[i] = AG + r * 4 + swizzle(r, q);
     }
@@ -1336,6 +1378,25 @@ __global__ __launch_bounds__(64 * GM * GN, (WN > 2 || GM * GN > 4) ? 1 : 2) void
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[i][j][v] = sum[i][j][v];
     }
+    if (g.swiglu) {
+        // silu(gate) * up (tests/activation_reference.s:99-126),
+        // written as the activation's BF16 planes; padding rows are not written.
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; j += 2) {
+                const uint32_t col = bn * (BN / 2) + wn * 16 * WN + j / 2 * 32 + (lane & 31);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const uint32_t row =
+                        m0 + wm * 32 * WM + 32 * i + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
+                    const float gate = acc[i][j][v], up = acc[i][j + 1][v];
+                    const float d = plamo_exp(-gate) + 1.0f;
+                    if (row < g.t) write_planes1(g.act, g.act_tp, row, col, (gate / d) * up);
+                }
+            }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -1351,9 +1412,10 @@ __global__ __launch_bounds__(64 * GM * GN, (WN > 2 || GM * GN > 4) ? 1 : 2) void
 }
 
 template <int WM, int WN, int GM = 2, int GN = 2, int PD = 3>
-static hipError_t gemm_split_variant(hipStream_t stream, GemmSplit g, const GemmWorkspace &ws) {
+static hipError_t gemm_split_variant(hipStream_t stream, GemmSplit g, const GemmWorkspace &ws,
+                                     bool planes_ready) {
     constexpr uint32_t BM = 32 * WM * GM, BN = 32 * WN * GN;
-    static_assert(BM == kSplitBM, "gemm_split_192 counts tiles of kSplitBM rows");
+    static_assert(BM == kSplitBM, "gemm_planes_rows pads the planes to kSplitBM rows");
     const uint32_t nt = (g.n + BN - 1) / BN, mt = (g.t + BM - 1) / BM;
     const uint32_t tiles = nt * mt, stages = g.k / kSplitBK;
     g.tp = mt * BM;
@@ -1378,8 +1440,9 @@ static hipError_t gemm_split_variant(hipStream_t stream, GemmSplit g, const Gemm
     // Grouping needs whole turns of the 8 XCDs: (weight tiles x splits) % 8 == 0.
     g.xcd_group = mt > 1 && (nt * splits) % 8 == 0;
     const uint64_t elems = (uint64_t)g.tp * g.k;
-    split_planes_kernel<<<(unsigned)((elems / 8 + 255) / 256), 256, 0, stream>>>(
-        g.x, g.ldx, g.t, g.tp, g.k, ws.planes);
+    if (!planes_ready)
+        split_planes_kernel<<<(unsigned)((elems / 8 + 255) / 256), 256, 0, stream>>>(
+            g.x, g.ldx, g.t, g.tp, g.k, ws.planes);
     const size_t lds = 3 * (size_t)(3 * BM * 4 + BN * 4) * sizeof(u32x4);
     static bool attr = false;
     if (!attr) {
@@ -1974,6 +2037,16 @@ uint64_t gemm_plane_elems(uint64_t tokens, uint64_t cols) {
     return 3 * ((tokens + 127) / 128 * 128) * cols;
 }
 
+uint32_t gemm_planes_rows(uint64_t tokens, uint64_t cols, const GemmWorkspace *ws) {
+    if (tokens <= kSkinnyTokens || tokens >= (1u << 31) || cols % (2 * kSplitBK) ||
+        cols > (1u << 30) || !ws || !ws->planes)
+        return 0;
+    const uint64_t tp = (tokens + kSplitBM - 1) / kSplitBM * kSplitBM;
+    return 3 * tp * cols <= ws->plane_elems && gemm_plane_elems(tokens, cols) <= ws->plane_elems
+               ? (uint32_t)tp
+               : 0;
+}
+
 // Wide tiles (256 weight rows per block, each wave 32 tokens x 128 rows)
 // except for short prompts' projections with few row tiles and K below 8192,
 // which take 128-row tiles (each wave 32 x 64) and get more blocks. Measured
@@ -1996,26 +2069,36 @@ static bool gemm_split_wide(uint64_t rows, uint64_t cols, uint64_t tokens) {
 // down 200.0 -> 187.5; at 116: QKV 40.6 -> 36.9, gate/up equal within the
 // spread between boxes).
 // Past 128 tokens, a projection whose 256-row tiles leave CUs idle takes
-// 192-row tiles when their count still fits one round of 256 blocks: C4 QKV at
-// 443 tokens, 7 x 24 = 168 against 7 x 32 = 224 blocks, 87.4-89.3 -> 81.7-85.7 us
+// 192-row tiles when their count still fits one round of 256 blocks (not for
+// SwiGLU, whose gate/up pairing needs an even number of 32-row groups per
+// wave): C4 QKV at 443 tokens, 7 x 24 = 168 against 7 x 32 = 224 blocks, 87.4-89.3 -> 81.7-85.7 us
 // without the split launch.
 static bool gemm_split_192(const GemmSplit &g) {
-    if (g.t <= 128 || g.n % 192) return false;
+    if (g.swiglu || g.t <= 128 || g.n % 192) return false;
     const uint64_t mt = (g.t + kSplitBM - 1) / kSplitBM;
     const uint64_t b256 = mt * ((g.n + 255) / 256), b192 = mt * (g.n / 192);
     return b256 < 256 && b192 <= 256 && b192 > b256;
 }
-static hipError_t gemm_split_route(hipStream_t stream, const GemmSplit &g,
-                                   const GemmWorkspace &ws) {
-    if (gemm_split_192(g)) return gemm_split_variant<1, 3, 2, 2, 3>(stream, g, ws);
-    return gemm_split_wide(g.n, g.k, g.t) ? gemm_split_variant<1, 4, 2, 2, 3>(stream, g, ws)
-                                          : gemm_split_variant<1, 2, 2, 2, 3>(stream, g, ws);
+static hipError_t gemm_split_route(hipStream_t stream, const GemmSplit &g, const GemmWorkspace &ws,
+                                   bool planes_ready) {
+    if (gemm_split_192(g)) return gemm_split_variant<1, 3, 2, 2, 3>(stream, g, ws, planes_ready);
+    return gemm_split_wide(g.n, g.k, g.t)
+               ? gemm_split_variant<1, 4, 2, 2, 3>(stream, g, ws, planes_ready)
+               : gemm_split_variant<1, 2, 2, 2, 3>(stream, g, ws, planes_ready);
+}
+// Rows of one tile of the route above (the swiglu pairing needs the
+// intermediate size to be whole half tiles).
+static uint32_t gemm_split_tile_rows(uint64_t rows, uint64_t cols, uint64_t tokens) {
+    return gemm_split_wide(rows, cols, tokens) ? 256 : 128;
 }
 
 hipError_t launch_gemm(hipStream_t stream, const float *x, uint64_t x_stride, const uint16_t *w,
                        uint64_t rows, uint64_t cols, uint64_t tokens, float *y,
-                       uint64_t y_stride, const GemmWorkspace *ws) {
+                       uint64_t y_stride, const GemmWorkspace *ws, bool planes_ready) {
     if (!tokens || !rows) return hipSuccess;
+    // planes_ready callers may not have written x: only the matrix-core route
+    // below may take them.
+    if (planes_ready && tokens <= kSkinnyTokens) return hipErrorInvalidValue;
     {
         hipError_t e = launch_token_gemv(stream, x, x_stride, w, rows, cols, tokens, 0, y,
                                          y_stride, ws);
@@ -2047,22 +2130,54 @@ hipError_t launch_gemm(hipStream_t stream, const float *x, uint64_t x_stride, co
         g.t = (uint32_t)tokens;
         g.y = y;
         g.ldy = y_stride;
-        return gemm_split_route(stream, g, *ws);
+        return gemm_split_route(stream, g, *ws, planes_ready);
     }
+    if (planes_ready) return hipErrorInvalidValue;
     if (tokens <= 16) return gemm_variant<16, 64>(stream, x, x_stride, w, rows, cols, tokens, y, y_stride);
     return gemm_variant<64, 64>(stream, x, x_stride, w, rows, cols, tokens, y, y_stride);
+}
+
+uint16_t *gemm_swiglu_planes(uint64_t intermediate, uint64_t cols, uint64_t tokens,
+                             const GemmWorkspace *ws) {
+    const uint64_t tp = gemm_planes_rows(tokens, cols, ws);
+    if (!tp || intermediate >= (1u << 30) || intermediate % (2 * kSplitBK) ||
+        intermediate % (gemm_split_tile_rows(2 * intermediate, cols, tokens) / 2) ||
+        3 * tp * (cols + intermediate) > ws->plane_elems)
+        return nullptr;
+    return ws->planes + 3 * tp * cols;
 }
 
 hipError_t launch_gemm_swiglu(hipStream_t stream, const float *x, uint64_t x_stride,
                               const uint16_t *w, uint64_t intermediate, uint64_t cols,
                               uint64_t tokens, float *act, float *gate_up,
-                              const GemmWorkspace *ws) {
+                              const GemmWorkspace *ws, bool planes_ready, uint16_t *act_planes) {
     if (!tokens || !intermediate) return hipSuccess;
-    hipError_t e = launch_token_gemv(stream, x, x_stride, w, 2 * intermediate, cols, tokens,
-                                     intermediate, act, intermediate, ws);
-    if (e != hipErrorNotSupported) return e;
-    e = launch_gemm(stream, x, x_stride, w, 2 * intermediate, cols, tokens, gate_up,
-                    2 * intermediate, ws);
+    if (act_planes) {
+        // The gate/up GEMM writes the activation planes from its epilogue, past
+        // the input's planes (which its running blocks still read).
+        if (act_planes != gemm_swiglu_planes(intermediate, cols, tokens, ws) ||
+            !gemm_split_supported(x, x_stride, w, cols))
+            return hipErrorInvalidValue;
+        GemmSplit g{};
+        g.x = x;
+        g.ldx = x_stride;
+        g.w = w;
+        g.n = (uint32_t)(2 * intermediate);
+        g.k = (uint32_t)cols;
+        g.t = (uint32_t)tokens;
+        g.swiglu = (uint32_t)intermediate;
+        g.act = act_planes;
+        g.act_tp = gemm_planes_rows(tokens, cols, ws);
+        return gemm_split_route(stream, g, *ws, planes_ready);
+    }
+    // The token GEMV reads x as FP32.
+    if (!planes_ready) {
+        hipError_t e = launch_token_gemv(stream, x, x_stride, w, 2 * intermediate, cols, tokens,
+                                         intermediate, act, intermediate, ws);
+        if (e != hipErrorNotSupported) return e;
+    }
+    hipError_t e = launch_gemm(stream, x, x_stride, w, 2 * intermediate, cols, tokens, gate_up,
+                               2 * intermediate, ws, planes_ready);
     if (e != hipSuccess) return e;
     return launch_swiglu_rows(stream, gate_up, act, intermediate, tokens);
 }
@@ -2728,21 +2843,30 @@ __global__ __launch_bounds__(kThreads) void norm_rows_kernel(const float *x, uin
 }
 
 
+// Padding rows of either planes.
+__device__ __forceinline__ void zero_row(const PairRows &pair, const SplitRows &split, uint32_t row,
+                                         uint32_t width) {
+    if (pair.planes) return pair_zero_row(pair, row, width);
+    for (uint32_t c = threadIdx.x * 4; c < width; c += 4 * kThreads)
+        write_planes4(split.planes, split.padded, row, c, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+}
+
 // norm_rows_kernel with the row held in registers, 16-byte accesses (width a
 // multiple of 4, at most 8192): every load goes out before the sum, where the
 // strided loop above waits on each in turn (C5 verify's first norm 15 us).
 // With pair.planes the normalized row goes there as a scaled pair of fp16 terms
-// instead of y; blocks past `rows` (up to pair.padded) write zeros.
+// instead of y, with split.planes as BF16 terms; blocks past `rows` (up to the
+// padded rows) write zeros.
 template <int NV>
 __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, uint64_t x_stride,
                                                               const uint16_t *w, float offset,
                                                               float *y, uint64_t y_stride,
                                                               uint32_t width, PairRows pair,
-                                                              uint32_t rows) {
+                                                              SplitRows split, uint32_t rows) {
     __shared__ float red[4];
     const uint32_t groups = width / 4;
     if (blockIdx.x >= rows) {
-        pair_zero_row(pair, blockIdx.x, width);
+        zero_row(pair, split, blockIdx.x, width);
         return;
     }
     const float *xr = x + blockIdx.x * x_stride;
@@ -2773,33 +2897,41 @@ __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, ui
         const uint32_t wb[4] = {g[j].x & 0xffffu, g[j].x >> 16, g[j].y & 0xffffu, g[j].y >> 16};
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[j][e] = (v[j][e] * inv) * (bf16f(wb[e]) + offset);
-        if (!pair.planes && i < groups) *(f32x4 *)(yr + 4 * i) = v[j];
+        if (i >= groups) continue;
+        if (split.planes)
+            write_planes4(split.planes, split.padded, blockIdx.x, 4 * i, v[j]);
+        else if (!pair.planes)
+            *(f32x4 *)(yr + 4 * i) = v[j];
     }
     if (pair.planes) pair_row<NV>(pair, blockIdx.x, groups, v, red);
 }
 
 hipError_t launch_norm_rows(hipStream_t stream, const float *x, uint64_t x_stride,
                             const uint16_t *w, float offset, float *y, uint64_t y_stride,
-                            uint64_t width, uint64_t rows, const PairRows *pair) {
+                            uint64_t width, uint64_t rows, const PairRows *pair,
+                            const SplitRows *split) {
     if (!rows) return hipSuccess;
     if (width % 4 == 0 && width <= 8192 && x_stride % 4 == 0 && y_stride % 4 == 0 &&
         !((uintptr_t)x & 15) && !((uintptr_t)y & 15) && !((uintptr_t)w & 7)) {
-        if (pair && (pair->padded < rows || width % kPairK)) return hipErrorInvalidValue;
+        if ((pair && (pair->padded < rows || width % kPairK)) ||
+            (split && (pair || split->padded < rows || width % (2 * kSplitBK))))
+            return hipErrorInvalidValue;
         const uint32_t wd = (uint32_t)width, n = (uint32_t)rows;
-        const unsigned grid = pair ? pair->padded : n;
+        const unsigned grid = pair ? pair->padded : split ? split->padded : n;
         const PairRows pr = pair ? *pair : PairRows{};
+        const SplitRows sr = split ? *split : SplitRows{};
         if (width <= 2048)
             norm_rows4_kernel<2><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, pr, n);
+                                                                y_stride, wd, pr, sr, n);
         else if (width <= 4096)
             norm_rows4_kernel<4><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, pr, n);
+                                                                y_stride, wd, pr, sr, n);
         else
             norm_rows4_kernel<8><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, pr, n);
+                                                                y_stride, wd, pr, sr, n);
         return hipGetLastError();
     }
-    if (pair) return hipErrorInvalidValue;
+    if (pair || split) return hipErrorInvalidValue;
     norm_rows_kernel<<<(unsigned)rows, kThreads, 0, stream>>>(x, x_stride, w, offset, y, y_stride,
                                                               (uint32_t)width);
     return hipGetLastError();
@@ -2876,12 +3008,12 @@ template <int NV>
 __global__ __launch_bounds__(kThreads) void residual_norm_rows4_kernel(
     float *state, const float *branch, const uint16_t *wr, float off_r, const uint16_t *wn,
     float off_n, float *norm, uint64_t norm_stride, uint32_t width, PairRows pair,
-    uint32_t rows) {
+    SplitRows split, uint32_t rows) {
     __shared__ float red[4];
     const uint64_t row = blockIdx.x;
     const uint32_t groups = width / 4;
     if (blockIdx.x >= rows) {  // padding rows of the planes
-        pair_zero_row(pair, blockIdx.x, width);
+        zero_row(pair, split, blockIdx.x, width);
         return;
     }
     f32x4 b[NV], st[NV];
@@ -2930,7 +3062,11 @@ __global__ __launch_bounds__(kThreads) void residual_norm_rows4_kernel(
         const uint32_t w[4] = {gn[j].x & 0xffffu, gn[j].x >> 16, gn[j].y & 0xffffu, gn[j].y >> 16};
 #pragma unroll
         for (int e = 0; e < 4; ++e) st[j][e] = (st[j][e] * inv2) * (bf16f(w[e]) + off_n);
-        if (!pair.planes && g < groups) *(f32x4 *)(norm + row * norm_stride + 4 * g) = st[j];
+        if (g >= groups) continue;
+        if (split.planes)
+            write_planes4(split.planes, split.padded, blockIdx.x, 4 * g, st[j]);
+        else if (!pair.planes)
+            *(f32x4 *)(norm + row * norm_stride + 4 * g) = st[j];
     }
     if (pair.planes) pair_row<NV>(pair, blockIdx.x, groups, st, red);
 }
@@ -2938,28 +3074,32 @@ __global__ __launch_bounds__(kThreads) void residual_norm_rows4_kernel(
 hipError_t launch_residual_norm_rows(hipStream_t stream, float *state, const float *branch,
                                      const uint16_t *wr, float off_r, const uint16_t *wn,
                                      float off_n, float *norm, uint64_t norm_stride,
-                                     uint64_t width, uint64_t rows, const PairRows *pair) {
+                                     uint64_t width, uint64_t rows, const PairRows *pair,
+                                     const SplitRows *split) {
     if (!rows) return hipSuccess;
     const uint32_t w = (uint32_t)width;
     if (width % 4 == 0 && norm_stride % 4 == 0 && !((uintptr_t)state & 15) &&
         !((uintptr_t)branch & 15) && !((uintptr_t)norm & 15) && !((uintptr_t)wr & 7) &&
         !((uintptr_t)wn & 7) && width <= 8192) {
-        if (pair && (pair->padded < rows || width % kPairK)) return hipErrorInvalidValue;
+        if ((pair && (pair->padded < rows || width % kPairK)) ||
+            (split && (pair || split->padded < rows || width % (2 * kSplitBK))))
+            return hipErrorInvalidValue;
         const uint32_t n = (uint32_t)rows;
-        const unsigned grid = pair ? pair->padded : n;
+        const unsigned grid = pair ? pair->padded : split ? split->padded : n;
         const PairRows pr = pair ? *pair : PairRows{};
+        const SplitRows sr = split ? *split : SplitRows{};
         if (width <= 2048)
             residual_norm_rows4_kernel<2><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, n);
+                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, sr, n);
         else if (width <= 4096)
             residual_norm_rows4_kernel<4><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, n);
+                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, sr, n);
         else
             residual_norm_rows4_kernel<8><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, n);
+                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, sr, n);
         return hipGetLastError();
     }
-    if (pair) return hipErrorInvalidValue;
+    if (pair || split) return hipErrorInvalidValue;
     if (width <= 2048)
         residual_norm_rows_kernel<8><<<(unsigned)rows, kThreads, 0, stream>>>(
             state, branch, wr, off_r, wn, off_n, norm, norm_stride, w);

@@ -93,9 +93,11 @@ hipError_t launch_rope_table(hipStream_t s, const float *, float, uint32_t, uint
 }
 uint64_t gemm_plane_elems(uint64_t tokens, uint64_t cols) { return 3 * tokens * cols; }
 hipError_t launch_gemm(hipStream_t s, const float *, uint64_t, const uint16_t *, uint64_t, uint64_t,
-                       uint64_t, float *, uint64_t, const GemmWorkspace *) {
+                       uint64_t, float *, uint64_t, const GemmWorkspace *, bool) {
     return queue(s);
 }
+uint32_t gemm_planes_rows(uint64_t, uint64_t, const GemmWorkspace *) { return 0; }
+uint16_t *gemm_swiglu_planes(uint64_t, uint64_t, uint64_t, const GemmWorkspace *) { return nullptr; }
 PairWeight pair_rows_from(const PairWeight &w, uint32_t) { return w; }
 bool pair_supported(uint64_t, uint64_t) { return true; }
 uint64_t pair_frag_elems(uint64_t rows, uint64_t cols) { return rows * cols; }
@@ -121,12 +123,13 @@ hipError_t launch_gemm_pair_swiglu(hipStream_t s, const PairRows &, const PairWe
     return queue(s);
 }
 hipError_t launch_norm_rows(hipStream_t s, const float *, uint64_t, const uint16_t *, float,
-                            float *, uint64_t, uint64_t, uint64_t, const PairRows *) {
+                            float *, uint64_t, uint64_t, uint64_t, const PairRows *,
+                            const SplitRows *) {
     return queue(s);
 }
 hipError_t launch_residual_norm_rows(hipStream_t s, float *, const float *, const uint16_t *, float,
                                      const uint16_t *, float, float *, uint64_t, uint64_t, uint64_t,
-                                     const PairRows *) {
+                                     const PairRows *, const SplitRows *) {
     return queue(s);
 }
 hipError_t launch_residual_rows(hipStream_t s, float *, const float *, const uint16_t *, float,
@@ -137,7 +140,8 @@ hipError_t launch_swiglu_rows(hipStream_t s, const float *, float *, uint64_t, u
     return queue(s);
 }
 hipError_t launch_gemm_swiglu(hipStream_t s, const float *, uint64_t, const uint16_t *, uint64_t,
-                              uint64_t, uint64_t, float *, float *, const GemmWorkspace *) {
+                              uint64_t, uint64_t, float *, float *, const GemmWorkspace *, bool,
+                              uint16_t *) {
     return queue(s);
 }
 hipError_t launch_qkv_post(hipStream_t s, const QkvPost &) { return queue(s); }

@@ -349,3 +349,40 @@ def test_prompt_activation_columns(gate, up, exponent, ignored, tokens):
         gpu.close()
         cpu.close()
         syn.close()
+
+
+# Prompts of models whose shapes the fp16 fragments do not cover (an attention
+# width that is not whole 32 columns), on the BF16 weights: the norms write the
+# split GEMM's planes, and gate/up writes down's where the intermediate size is
+# whole half tiles; skinny batches, whole and ragged tiles, both tile widths.
+@pytest.mark.parametrize("inter", [128, 192, 100, 8256])
+@pytest.mark.parametrize("tokens", [3, 16, 17, 64, 65, 140])
+def test_prompt_without_fragments(inter, tokens):
+    say(f"without fragments inter={inter} tokens={tokens}")
+    hidden = 256
+    syn = plamo_hip.Synthetic(hidden, 3, 3, 3, 20, inter, 200, window=1024, global_capacity=1024,
+                              pattern=2, embedding_std=1.0, seed=tokens)
+    gpu, cpu = syn.instance(), syn.instance()
+    be = plamo_hip.Backend(syn)
+    try:
+        for states in (True, False):
+            ids = [(7 * j + 3) % 200 for j in range(tokens)]
+            actual = np.zeros((tokens, hidden), np.float32) if states else None
+            expected = np.zeros((tokens, hidden), np.float32) if states else None
+            assert be.prefill(gpu, ids, actual) == 1
+            assert oracle_lib.prefill(cpu, ids, expected)
+            if states:
+                gate(actual, expected, "all prompt states")
+            compare(gpu, cpu)
+        if tokens <= 16:
+            assert be.verify(gpu, ids)[0] == 1
+            assert oracle_lib.forward(cpu, ids[0])
+            assert be.commit(gpu, 0) == 1
+            compare(gpu, cpu)
+        info = be.info()
+        assert info.errors == 0 and info.cpu_fallbacks == 0, info.note.decode()
+    finally:
+        be.close()
+        gpu.close()
+        cpu.close()
+        syn.close()
