@@ -2276,8 +2276,13 @@ int plamo_hip_rewind(struct plamo_metal *m, struct model *model, uint64_t steps)
 // staging memory grows to it on demand). The runtime's copies of pageable
 // memory cost 10-15 us each at the smallest (3072 x 2048, one row: 50 -> 27 us
 // a call; an MLP branch of 37 rows of 2560: 186 -> 153), and its strided ones
-// far more (20160 x 8064, 266 rows: 4960 -> 871).
+// far more (20160 x 8064, 266 rows: 4960 -> 871). An MLP branch's rows lie
+// together, and the runtime pipelines the copies of such a block, where staging
+// takes its copies by the host and over the bus one after the other: equal at
+// 2.4 and 3.1 MB (150 rows of 4096 592 us either way, 300 of 2560 550), behind
+// from there (300 rows of 4096 994 -> 1025 staged, 600 of 4096 1858 -> 1945).
 constexpr uint64_t kStageBytes = 32ull << 20;
+constexpr uint64_t kStageBlockBytes = 3ull << 20;
 
 static uint64_t stage_round(uint64_t bytes) { return (bytes + 255) / 256 * 256; }
 
@@ -2479,7 +2484,7 @@ int plamo_metal_mlp(struct plamo_metal *m, const struct mlp *mlp, float *states,
     hipStream_t s = m->stream;
     uint16_t *norms = as<uint16_t>(in);
     float *st = (float *)(as<char>(in) + norm_bytes);
-    const bool staged = ok && ensure_stage(m, norm_bytes + row_bytes);
+    const bool staged = ok && row_bytes <= kStageBlockBytes && ensure_stage(m, norm_bytes + row_bytes);
     if (staged) {
         memcpy(m->stage_host, mlp->pre, h * 2);
         memcpy(m->stage_host + h * 2, mlp->post, h * 2);

@@ -386,3 +386,34 @@ def test_prompt_without_fragments(inter, tokens):
         gpu.close()
         cpu.close()
         syn.close()
+
+
+# Rows of plamo_metal_mlp on both sides of the 3 MiB up to which they are
+# staged, one call after the other on one backend.
+def test_mlp_host_rows(oracle):
+    hidden, inter = 4096, 64
+    s = plamo_hip.Synthetic(hidden, 1, 4, 1, 128, inter, 40, window=4, global_capacity=64,
+                            pattern=1, seed=38)
+    a = s.instance()
+    be = plamo_hip.Backend(s)
+    try:
+        mlp = a.layer(0).mlp.contents
+        for tokens in (192, 193, 2, 400):
+            say(f"mlp rows tokens={tokens}")
+            st = np.random.default_rng(tokens).standard_normal((tokens, hidden), dtype=np.float32)
+            ref = st.copy()
+            assert be.lib.plamo_metal_mlp(be.handle, ctypes.byref(mlp),
+                                          st.ctypes.data_as(plamo_hip.f32p), tokens) == 1
+            for t in range(tokens):
+                row = ref[t].copy()
+                m2 = plamo_hip.Mlp(row.ctypes.data_as(plamo_hip.f32p), mlp.pre, mlp.post, mlp.gu,
+                                   mlp.down, mlp.normalized, mlp.branch, mlp.scratch, hidden, inter)
+                oracle.oracle_mlp_branch(ctypes.byref(m2))
+                ref[t] = row
+            gate(st, ref, f"mlp tokens={tokens}")
+        info = be.info()
+        assert info.errors == 0 and info.cpu_fallbacks == 0
+    finally:
+        be.close()
+        a.close()
+        s.close()
