@@ -3708,18 +3708,18 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_kernel(DecodeAt
 // its dot products: the O weights cross HBM while attention runs. The wait is
 // bounded; a block that gives up writes NaN rows (they surface as a failed
 // argmax) and sets *error.
-// O rows per wave of the fused kernel, and the LDS every block of it claims:
-// more than half of a CU's 160 KiB, so a CU holds one block. With the KV
+// O rows per wave of the fused kernel, and the LDS every block of it claims
+// for a short context (OM): more than half of a CU's 160 KiB, so a CU holds
+// one block. With the KV
 // rows allocated in small steps the launch (64 attention blocks at C4 below
 // 256 rows plus 128 O blocks) then fits the 256 CUs at once: every O block
 // requests its weights at the start, and no O block's 256 KB of weight loads
 // shares a CU's load path with an attention block's latency-bound loads.
-// A long context's launch of more than 256 blocks (256 attention blocks alone
-// at 2048 rows and 8 KV heads) claims what it uses, so that two blocks share a
-// CU: the O blocks are there from the start instead of after the first
-// attention blocks end. With the batched merge below, 1900 rows at C4: 29 us a
-// layer before, 19 after. Up to 256 blocks the claim stays (C4 at 600 rows 300
-// us a step of three layers with it, 302 without; C2 at 400 rows 325 and 326).
+// A long context's attention blocks take every CU by themselves (256 at 2048
+// rows and 8 KV heads), so its blocks claim what they use and two share a CU:
+// the O blocks are there from the start instead of after the first attention
+// blocks end. With the batched merge below, 1900 rows at C4: 29 us a layer
+// before, 19 after.
 // (Rows per wave, C4 ms per step: 2: 3.114, 3: 3.089, 4: 3.053, 5: 3.060,
 // 6: 3.114.)
 // 8192-wide rows (16 chunks) take 2 rows per wave: 4 would hold 256 VGPRs
@@ -3910,15 +3910,15 @@ static hipError_t decode_attention_dim(hipStream_t stream, const DecodeAttention
 
 template <int DIM, int G, int KC, int ROWS, bool OM = false>
 static hipError_t attention_o_variant(hipStream_t stream, const AttentionO &f) {
-    const uint32_t per_block = o_rows_per_wave(KC) * kAttnWaves;
-    const uint32_t oblocks = (f.rows + per_block - 1) / per_block;
-    const uint32_t blocks = f.a.kh * f.a.splits + oblocks;
-    size_t lds = decode_attention_lds(DIM, G, ROWS);
-    if (OM || blocks <= 256) lds = std::max(lds, kAttentionOLds);
+    const size_t lds = OM ? std::max(decode_attention_lds(DIM, G, ROWS), kAttentionOLds)
+                          : decode_attention_lds(DIM, G, ROWS);
     hipError_t e = hipFuncSetAttribute((const void *)attention_o_kernel<DIM, G, KC, ROWS, OM>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    attention_o_kernel<DIM, G, KC, ROWS, OM><<<blocks, kAttnThreads, lds, stream>>>(f);
+    const uint32_t per_block = o_rows_per_wave(KC) * kAttnWaves;
+    const uint32_t oblocks = (f.rows + per_block - 1) / per_block;
+    attention_o_kernel<DIM, G, KC, ROWS, OM>
+        <<<f.a.kh * f.a.splits + oblocks, kAttnThreads, lds, stream>>>(f);
     return hipGetLastError();
 }
 
