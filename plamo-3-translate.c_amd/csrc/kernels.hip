@@ -2056,9 +2056,12 @@ uint32_t gemm_planes_rows(uint64_t tokens, uint64_t cols, const GemmWorkspace *w
 // 213.1), and down at 116 (76.3 -> 75.2, K 16384).
 static bool gemm_split_wide(uint64_t rows, uint64_t cols, uint64_t tokens) {
     const uint64_t tiles = (rows + 255) / 256, mt = (tokens + kSplitBM - 1) / kSplitBM;
-    // A deep K splits in at most eight: too few wide tiles leave CUs idle
-    // (37 tokens of 2560 x 10240: 80 blocks; 128-row tiles take an MLP branch of those rows from 153 to 141 us).
-    return tokens > 128 || tiles >= 64 || (cols >= 8192 && tiles * mt * 8 >= 160);
+    // A deep K splits in at most eight: too few wide tiles leave CUs idle (us
+    // on 128-row and on 256-row tiles: 1024 rows at K 8192, 37 tokens 28.8 and
+    // 37.2, 100 tokens 36.2 and 43.3; 2560 rows at K 10240, 37 tokens 38.2 and
+    // 46.9). From 128 blocks on the wide ones catch up with depth (4096 rows at
+    // 37 tokens, K 8192 48.2 and 49.1, 10240 53.6 and 53.2, 16384 68.5 and 64.0).
+    return tokens > 128 || tiles >= 64 || (cols >= 8192 && tiles * mt * 8 >= 128);
 }
 // Three K stages in registers ahead of the LDS stages (2 and 4 measured within
 // 1-4 % of it, either way, with three LDS buffers).
