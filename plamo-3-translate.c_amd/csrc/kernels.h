@@ -234,7 +234,7 @@ hipError_t launch_qkv_post(hipStream_t, const QkvPost &);
 // rotated K (plus the mirror stage), and every block runs an online softmax
 // over its share of rows [0, count]; the last block of a KV head merges the
 // partials. Requires decode_attention_supported(dim, qh / kh), splits <= 8 and
-// count < capacity (a full sliding window takes the general path). Up to 256
+// count < capacity (a full sliding window's rows have moved on by one). Up to 256
 // rows run in one block per KV head; longer contexts use up to `splits` blocks.
 struct DecodeAttention {
     const float *qkv;        // [(qh+2kh)*dim] projection output
