@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
-"""Benchmark of the MI355X token-loop backend on BASELINE.json's headline config.
+"""Benchmark of the MI355X token-loop backend on the 8B-class headline model.
 
-Workload (configs[3], "8B-class headline"): hidden 4096, 32 layers, 32 query /
+Workload (C4, 8B class): hidden 4096, 32 layers, 32 query /
 8 KV heads of 128, MLP 16384, vocab 100000, seeded synthetic BF16 weights
 ~N(0, 0.02) (16.4 GB streamed per decode step, all resident in HBM). Each
 request restores a 12-token prefix KV from a snapshot (the engine's prompt
@@ -178,14 +178,14 @@ def cpu_baseline(inst: plamo_hip.Instance, token: int, seconds: float, cfg: dict
     """The C oracle on the host cores (rows split as runtime/parallel.c:35-48), on bounded
     samples of the same workloads: decode steps of the model continuing the
     GPU's sequence on the same host arrays at N threads and at 1 thread, the
-    C1 layer step at both, and the 128-token prompt's prefill
+    C1 layer step (one 2048-wide layer) at both, and the 128-token prompt's prefill
     (12-token prefix restored, 116 tokens) over the first layers of the model
     at N threads and over its first layer at 1 thread, scaled to every layer.
     Rows are split over threads in groups of 24 as runtime/parallel.c:35-48;
     the prefill runs its projections token-blocked as the reference's prompt
     path does (src/batch.s, src/matmul8x3.s)."""
     sys.path.insert(0, str(ROOT / "tests"))
-    import oracle_lib  # the checker's CPU path; test infrastructure, not the product
+    import oracle_lib  # the oracle: test infrastructure, not the product
 
     lib = oracle_lib.load()
     threads, nproc = host_threads()
@@ -456,7 +456,7 @@ def embed_draft(target: "plamo_hip.Instance", draft: "plamo_hip.Instance", mix: 
 
 
 def speculative(args) -> dict:
-    """the 31B-class model (C5, tied embedding/head) with
+    """The 31B-class model (C5, tied embedding/head) with
     the 0.8B-class model (C2 shape) as the in-process draft, 4 draft tokens
     per verify (a 5-token batched verify), a 455-token prompt and 128 greedy
     tokens through the engine's decode loop (runtime/engine.c:514-566,
@@ -601,7 +601,7 @@ def main() -> int:
                     help="also run device-to-device copies of MIB MiB (the known-size "
                          "kernel that scales rocprofv3 FETCH_SIZE / WRITE_SIZE)")
     ap.add_argument("--speculative", action="store_true",
-                    help="measure BASELINE configs[4] (C5 target, 0.8B-class draft) instead")
+                    help="measure the 31B class (C5 target, 0.8B-class draft) instead")
     ap.add_argument("--verify", action="store_true",
                     help="time the C5 target's batched verify alone, per candidate count")
     ap.add_argument("--verify-tokens", default="1,2,3,4,5,6,8,16")

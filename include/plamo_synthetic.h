@@ -1,4 +1,4 @@
-/* Synthetic PLaMo-3 model descriptors for the BASELINE configurations.
+/* Synthetic PLaMo-3 model descriptors for the named configurations (C1-C5).
  *
  * No reference counterpart as an API: it builds the same descriptor graph the
  * reference's generator emits for a real checkpoint (tools/model_layout.py:71-199:
@@ -36,7 +36,7 @@ struct plamo_synthetic_config {
 struct plamo_synthetic;
 struct plamo_synthetic_instance;
 
-/* Fills the BASELINE defaults (RoPE/YaRN constants of docs/config.json,
+/* Fills the defaults (RoPE/YaRN constants of docs/config.json,
  * window 2048, pattern 8, std 0.02) around the given shape. */
 void plamo_synthetic_defaults(struct plamo_synthetic_config *, uint64_t hidden, uint64_t layers,
                               uint64_t qh, uint64_t kh, uint64_t dim, uint64_t intermediate,

@@ -3,7 +3,7 @@
  * A scalar C restatement of the reference's FP32 CPU path, in the exact
  * operation order of its bit-exact specification (the tests/..._reference.s files) and
  * of the production assembly that is bit-identical to it (the src/ assembly). It is the
- * checker for the HIP backend and the CPU baseline of bench.py; nothing in the
+ * oracle for the HIP backend and the CPU baseline of bench.py; nothing in the
  * product links or calls it. Every function names the reference file:line it
  * follows in plamo_oracle.c.
  *

@@ -315,7 +315,7 @@ def hook_address(name: str) -> int:
     return c_void_p.in_dll(load(), name).value or 0
 
 
-# BASELINE.json configurations (hidden, layers, qh, kh, dim, intermediate, vocab).
+# The named configurations C1-C5 (hidden, layers, qh, kh, dim, intermediate, vocab).
 CONFIGS = {
     "c1": dict(hidden=2048, layers=1, qh=16, kh=4, dim=128, intermediate=8192, vocab=16),
     "c2": dict(hidden=2048, layers=16, qh=16, kh=4, dim=128, intermediate=8192, vocab=100000),

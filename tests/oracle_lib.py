@@ -1,6 +1,6 @@
 """Loader of the CPU oracle (oracle/build/liboracle.so) for tests and the CPU baseline.
 
-Test infrastructure only: the oracle is the checker, never the thing measured
+Test infrastructure only: the oracle is compared with, never the thing measured
 on the GPU path.
 """
 

@@ -1,6 +1,6 @@
 """Oracle parity on the flow and at the shapes the bench measures.
 
-C4 at full depth, 32 layers and the 100000-token
+C4 (8B class) at full depth, 32 layers and the 100000-token
 head, with bench.py's own seed and prompt ids: the 12-token template prefix is
 prefilled on the GPU and captured (runtime/prompt_cache.c:15-56); each
 request resets the model, restores that prefix (runtime/prompt_cache.c:
@@ -8,11 +8,11 @@ request resets the model, restores that prefix (runtime/prompt_cache.c:
 455-token prompt (the TTFT runs), then takes 8 greedy steps on the decode
 graph writing the pinned host arrays in place (the timed decode). The oracle
 prefills each whole prompt from a reset model. Greedy ids must agree except
-after a step whose oracle top-2 logit gap is below 1e-3 (BASELINE.json north
-star); state, logits and every layer's K / V / rotated K rows pass the
+after a step whose oracle top-2 logit gap is below 1e-3 (a tie, in FP32);
+state, logits and every layer's K / V / rotated K rows pass the
 reference's gate (tests/metal_decode.c:192-216).
 
-C5 with 2 of its 60 layers and the tied 100000 x 6144 head: a
+C5 (31B class) with 2 of its 60 layers and the tied 100000 x 6144 head: a
 real 455-token prefill, decode steps, then verify of 5 candidates (the
 speculative batch) committed against sequential oracle forwards, and a
 rejected suffix (tests/metal_decode.c:309-365 at this width).

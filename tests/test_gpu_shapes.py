@@ -1,21 +1,21 @@
-"""GPU parity at the BASELINE.json shapes, on the default decode path (the
+"""GPU parity at the named configurations' shapes (C1-C5), on the default decode path (the
 captured graph of the bench) and the prompt/verify paths.
 
-C1 (configs[0]): one layer, hidden 2048, 16/4 heads of 128, MLP 8192, KV
+C1: one layer, hidden 2048, 16/4 heads of 128, MLP 8192, KV
 pre-filled with 512 (then 254) rows of raw K/V ~ N(0,1) (rotations rebuilt by
 the first step on both sides); then decode steps and a prompt.
-C2 (configs[1]) in full: 16 layers, vocab 100000, a 32-token prompt and 64
+C2 in full: 16 layers, vocab 100000, a 32-token prompt and 64
 greedy steps; the greedy ids must match the oracle's except after a step whose
-oracle top-2 logit gap is below 1e-3, and every
+oracle top-2 logit gap is below 1e-3 (a tie, in FP32), and every
 step's logits pass the reference gate.
-C3 (configs[2]) shapes with 2 of its 24 layers (one local, one global YaRN
+C3 shapes with 2 of its 24 layers (one local, one global YaRN
 layer): attention width 2048 under hidden 2560, the 10240-column down
 projection; the engine's flow of a 12-token prefix restored from the prompt
 cache, then the 116- and 443-token suffixes of the 128- and 455-token prompts,
 then decode steps.
-C4 (configs[3]) shapes with 4 of its 32 layers and the full 100000-token
+C4 shapes with 4 of its 32 layers and the full 100000-token
 head: the 16K-column down projection and the fused attention at group 4.
-C5 (configs[4]) shapes with 2 of its 60 layers and the tied head: six query
+C5 shapes with 2 of its 60 layers and the tied head: six query
 heads per KV head, O and down at 6144 and 24576 columns; decode over a
 455-row prefix, then verify of 1-5 candidates (the token GEMV) and 6-16
 (the skinny GEMM) committed against sequential oracle forwards

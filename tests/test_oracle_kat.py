@@ -1,4 +1,4 @@
-"""Pins the CPU oracle (oracle/plamo_oracle.c) before it is trusted as the checker.
+"""Pins the CPU oracle (oracle/plamo_oracle.c) before anything is compared with it.
 
 Every test restates a known answer the reference itself relies on — its
 golden data (src/rope_constants.s), its known-answer C tests (tests/*.c), or a
