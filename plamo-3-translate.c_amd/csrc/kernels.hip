@@ -10,6 +10,8 @@
 // only by FP32 rounding.
 #include "kernels.h"
 
+#include <type_traits>
+
 namespace plamo {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -2312,21 +2314,27 @@ __device__ __forceinline__ void pair_row(const PairRows &p, uint32_t row, uint32
     }
 }
 
-// FP32 rows into the planes, one row per wave (at most 256 NV columns, held in
-// registers): the waves of a block write neighbouring rows, whose 64-byte
-// pieces make whole cache lines.
-template <int NV>
+// FP32 rows into the planes, W waves per row (at most 256 W NV columns, held in
+// registers). Few rows take four waves each: the launch is one trip to memory
+// and back. With one wave per row the waves of a block write neighbouring rows,
+// whose 64-byte pieces make whole cache lines. Us with four waves and with one:
+// 7 rows of 4096 3.8 and 4.6, 116 5.1 and 6.1, 155 5.9 and 6.3, 443 7.1 and 7.1,
+// 1900 11.2 and 10.5; 3500 of 2048 30.6 and 18.1.
+constexpr uint32_t kPairBlockRows = 256;
+template <int NV, int W>
 __global__ __launch_bounds__(kThreads) void pair_rows_kernel(const float *x, uint64_t x_stride,
                                                              uint32_t rows, uint32_t width,
                                                              PairRows p) {
-    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (row >= p.padded) return;
+    __shared__ float red[4];
+    const uint32_t wave = threadIdx.x >> 6, row = blockIdx.x * (4 / W) + wave / W;
+    const uint32_t lane = threadIdx.x & (64 * W - 1);
+    if (W == 1 && row >= p.padded) return;
     const float *xr = x + (uint64_t)min(row, rows - 1) * x_stride;
     f32x4 v[NV];
     float mx = 0.0f;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-        const uint32_t c = 4 * (lane + 64 * j);
+        const uint32_t c = 4 * (lane + 64 * W * j);
         v[j] = *(const f32x4 *)(xr + min(c, width - 4));
     }
 #pragma unroll
@@ -2337,11 +2345,16 @@ __global__ __launch_bounds__(kThreads) void pair_rows_kernel(const float *x, uin
             mx = fmaxf(mx, __builtin_fabsf(v[j][e]));
         }
     mx = wave_max(mx);
+    if constexpr (W == 4) {
+        if ((threadIdx.x & 63) == 0) red[wave] = mx;
+        __syncthreads();
+        mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    }
     const int ex = pair_exponent(__float_as_uint(mx));
     const float scale = power_of_two(ex);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-        const uint32_t c = 4 * (lane + 64 * j);
+        const uint32_t c = 4 * (lane + 64 * W * j);
         if (c >= width) continue;
         f16x4 hi, lo;
 #pragma unroll
@@ -2364,14 +2377,23 @@ hipError_t launch_pair_rows(hipStream_t stream, const float *x, uint64_t x_strid
     if (!width || width % kPairK || width > 8192 || p.padded < rows || x_stride % 4 ||
         ((uintptr_t)x & 15))
         return hipErrorInvalidValue;
-    const unsigned grid = (p.padded + 3) / 4;
     const uint32_t w = (uint32_t)width, n = (uint32_t)rows;
+    if (p.padded <= kPairBlockRows) {
+        if (width <= 2048)
+            pair_rows_kernel<2, 4><<<p.padded, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+        else if (width <= 4096)
+            pair_rows_kernel<4, 4><<<p.padded, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+        else
+            pair_rows_kernel<8, 4><<<p.padded, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+        return hipGetLastError();
+    }
+    const unsigned grid = (p.padded + 3) / 4;
     if (width <= 2048)
-        pair_rows_kernel<8><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+        pair_rows_kernel<8, 1><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
     else if (width <= 4096)
-        pair_rows_kernel<16><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+        pair_rows_kernel<16, 1><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
     else
-        pair_rows_kernel<32><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
+        pair_rows_kernel<32, 1><<<grid, kThreads, 0, stream>>>(x, x_stride, n, w, p);
     return hipGetLastError();
 }
 
@@ -2846,10 +2868,9 @@ __global__ __launch_bounds__(kThreads) void norm_rows_kernel(const float *x, uin
 }
 
 
-// Padding rows of either planes.
-__device__ __forceinline__ void zero_row(const PairRows &pair, const SplitRows &split, uint32_t row,
-                                         uint32_t width) {
-    if (pair.planes) return pair_zero_row(pair, row, width);
+// Padding rows of the BF16 planes.
+__device__ __forceinline__ void split_zero_row(const SplitRows &split, uint32_t row,
+                                               uint32_t width) {
     for (uint32_t c = threadIdx.x * 4; c < width; c += 4 * kThreads)
         write_planes4(split.planes, split.padded, row, c, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
 }
@@ -2857,19 +2878,23 @@ __device__ __forceinline__ void zero_row(const PairRows &pair, const SplitRows &
 // norm_rows_kernel with the row held in registers, 16-byte accesses (width a
 // multiple of 4, at most 8192): every load goes out before the sum, where the
 // strided loop above waits on each in turn (C5 verify's first norm 15 us).
-// With pair.planes the normalized row goes there as a scaled pair of fp16 terms
-// instead of y, with split.planes as BF16 terms; blocks past `rows` (up to the
+// With planes the normalized row goes there as a scaled pair of fp16 terms
+// instead of y (with SplitRows as BF16 terms); blocks past `rows` (up to the
 // padded rows) write zeros.
-template <int NV>
+template <int NV, typename Planes>
 __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, uint64_t x_stride,
                                                               const uint16_t *w, float offset,
                                                               float *y, uint64_t y_stride,
-                                                              uint32_t width, PairRows pair,
-                                                              SplitRows split, uint32_t rows) {
+                                                              uint32_t width, Planes planes,
+                                                              uint32_t rows) {
+    constexpr bool split = std::is_same_v<Planes, SplitRows>;
     __shared__ float red[4];
     const uint32_t groups = width / 4;
     if (blockIdx.x >= rows) {
-        zero_row(pair, split, blockIdx.x, width);
+        if constexpr (split)
+            split_zero_row(planes, blockIdx.x, width);
+        else
+            pair_zero_row(planes, blockIdx.x, width);
         return;
     }
     const float *xr = x + blockIdx.x * x_stride;
@@ -2901,12 +2926,13 @@ __global__ __launch_bounds__(kThreads) void norm_rows4_kernel(const float *x, ui
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[j][e] = (v[j][e] * inv) * (bf16f(wb[e]) + offset);
         if (i >= groups) continue;
-        if (split.planes)
-            write_planes4(split.planes, split.padded, blockIdx.x, 4 * i, v[j]);
-        else if (!pair.planes)
+        if constexpr (split)
+            write_planes4(planes.planes, planes.padded, blockIdx.x, 4 * i, v[j]);
+        else if (!planes.planes)
             *(f32x4 *)(yr + 4 * i) = v[j];
     }
-    if (pair.planes) pair_row<NV>(pair, blockIdx.x, groups, v, red);
+    if constexpr (!split)
+        if (planes.planes) pair_row<NV>(planes, blockIdx.x, groups, v, red);
 }
 
 hipError_t launch_norm_rows(hipStream_t stream, const float *x, uint64_t x_stride,
@@ -2921,17 +2947,22 @@ hipError_t launch_norm_rows(hipStream_t stream, const float *x, uint64_t x_strid
             return hipErrorInvalidValue;
         const uint32_t wd = (uint32_t)width, n = (uint32_t)rows;
         const unsigned grid = pair ? pair->padded : split ? split->padded : n;
-        const PairRows pr = pair ? *pair : PairRows{};
-        const SplitRows sr = split ? *split : SplitRows{};
-        if (width <= 2048)
-            norm_rows4_kernel<2><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, pr, sr, n);
-        else if (width <= 4096)
-            norm_rows4_kernel<4><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, pr, sr, n);
+        auto launch = [&](auto planes) {
+            using P = decltype(planes);
+            if (width <= 2048)
+                norm_rows4_kernel<2, P><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
+                                                                       y_stride, wd, planes, n);
+            else if (width <= 4096)
+                norm_rows4_kernel<4, P><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
+                                                                       y_stride, wd, planes, n);
+            else
+                norm_rows4_kernel<8, P><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
+                                                                       y_stride, wd, planes, n);
+        };
+        if (split)
+            launch(*split);
         else
-            norm_rows4_kernel<8><<<grid, kThreads, 0, stream>>>(x, x_stride, w, offset, y,
-                                                                y_stride, wd, pr, sr, n);
+            launch(pair ? *pair : PairRows{});
         return hipGetLastError();
     }
     if (pair || split) return hipErrorInvalidValue;
@@ -3007,16 +3038,20 @@ __global__ __launch_bounds__(kThreads) void residual_norm_rows_kernel(
 
 // residual_norm_rows_kernel with 16-byte accesses (width a multiple of 4):
 // thread i holds elements 4 (i + kThreads j) .. + 3.
-template <int NV>
+template <int NV, typename Planes>
 __global__ __launch_bounds__(kThreads) void residual_norm_rows4_kernel(
     float *state, const float *branch, const uint16_t *wr, float off_r, const uint16_t *wn,
-    float off_n, float *norm, uint64_t norm_stride, uint32_t width, PairRows pair,
-    SplitRows split, uint32_t rows) {
+    float off_n, float *norm, uint64_t norm_stride, uint32_t width, Planes planes,
+    uint32_t rows) {
+    constexpr bool split = std::is_same_v<Planes, SplitRows>;
     __shared__ float red[4];
     const uint64_t row = blockIdx.x;
     const uint32_t groups = width / 4;
     if (blockIdx.x >= rows) {  // padding rows of the planes
-        zero_row(pair, split, blockIdx.x, width);
+        if constexpr (split)
+            split_zero_row(planes, blockIdx.x, width);
+        else
+            pair_zero_row(planes, blockIdx.x, width);
         return;
     }
     f32x4 b[NV], st[NV];
@@ -3066,12 +3101,13 @@ __global__ __launch_bounds__(kThreads) void residual_norm_rows4_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) st[j][e] = (st[j][e] * inv2) * (bf16f(w[e]) + off_n);
         if (g >= groups) continue;
-        if (split.planes)
-            write_planes4(split.planes, split.padded, blockIdx.x, 4 * g, st[j]);
-        else if (!pair.planes)
+        if constexpr (split)
+            write_planes4(planes.planes, planes.padded, blockIdx.x, 4 * g, st[j]);
+        else if (!planes.planes)
             *(f32x4 *)(norm + row * norm_stride + 4 * g) = st[j];
     }
-    if (pair.planes) pair_row<NV>(pair, blockIdx.x, groups, st, red);
+    if constexpr (!split)
+        if (planes.planes) pair_row<NV>(planes, blockIdx.x, groups, st, red);
 }
 
 hipError_t launch_residual_norm_rows(hipStream_t stream, float *state, const float *branch,
@@ -3089,17 +3125,22 @@ hipError_t launch_residual_norm_rows(hipStream_t stream, float *state, const flo
             return hipErrorInvalidValue;
         const uint32_t n = (uint32_t)rows;
         const unsigned grid = pair ? pair->padded : split ? split->padded : n;
-        const PairRows pr = pair ? *pair : PairRows{};
-        const SplitRows sr = split ? *split : SplitRows{};
-        if (width <= 2048)
-            residual_norm_rows4_kernel<2><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, sr, n);
-        else if (width <= 4096)
-            residual_norm_rows4_kernel<4><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, sr, n);
+        auto launch = [&](auto planes) {
+            using P = decltype(planes);
+            if (width <= 2048)
+                residual_norm_rows4_kernel<2, P><<<grid, kThreads, 0, stream>>>(
+                    state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, planes, n);
+            else if (width <= 4096)
+                residual_norm_rows4_kernel<4, P><<<grid, kThreads, 0, stream>>>(
+                    state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, planes, n);
+            else
+                residual_norm_rows4_kernel<8, P><<<grid, kThreads, 0, stream>>>(
+                    state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, planes, n);
+        };
+        if (split)
+            launch(*split);
         else
-            residual_norm_rows4_kernel<8><<<grid, kThreads, 0, stream>>>(
-                state, branch, wr, off_r, wn, off_n, norm, norm_stride, w, pr, sr, n);
+            launch(pair ? *pair : PairRows{});
         return hipGetLastError();
     }
     if (pair || split) return hipErrorInvalidValue;
