@@ -46,9 +46,11 @@ enum plamo_metal_packing {
     PLAMO_PACK_DRAFT_Q4
 };
 /* runtime/metal.h:14-28. maps/count name the weight files: with memory AUTO or
- * RESIDENT each mapping is copied to HBM at open. reserve, available,
- * disk_cache_path, revision, packing and prefer_texture_weights are accepted
- * and ignored (they steer Apple unified-memory policies). */
+ * RESIDENT each mapping is copied to HBM at open. packing PLAMO_PACK_RAW keeps
+ * the BF16 weights alone: no fp16 fragments beside them, prompts run on the
+ * exact three-term split of their FP32 rows; its other values are all AUTO.
+ * reserve, available, disk_cache_path, revision and prefer_texture_weights are
+ * accepted and ignored (they steer Apple unified-memory policies). */
 struct plamo_metal_config {
     enum plamo_metal_memory memory;
     enum plamo_metal_precision precision;

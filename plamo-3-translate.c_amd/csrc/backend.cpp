@@ -795,11 +795,13 @@ bool resolve_layers(plamo_metal *m, struct model *model) {
 constexpr uint64_t kPairTokens = 6;
 
 // Lays out the fp16 fragments of every layer (about as much memory as the
-// projections themselves, one pass over them). Without the memory, or with
-// shapes the fragments do not cover, prompts keep the BF16 weights.
+// projections themselves, one pass over them). Without the memory, with shapes
+// the fragments do not cover, or for a caller who asked for raw weights, prompts
+// keep the BF16 weights.
 int ensure_pair(plamo_metal *m, struct model *model) {
     if (m->pair_tried) return 1;
     m->pair_tried = true;
+    if (m->config.packing == PLAMO_PACK_RAW) return 1;
     const uint64_t h = model->hidden;
     uint64_t bytes = 0;
     auto take = [&](uint64_t n) {

@@ -493,13 +493,15 @@ class Instance:
 class Backend:
     """plamo_metal_* handle (runtime/metal.h:48-88) opened over a synthetic model."""
 
-    def __init__(self, synthetic=None, memory: int = 0):
+    def __init__(self, synthetic=None, memory: int = 0, packing: int = 0):
         """synthetic: a Synthetic model or a Checkpoint (its weight mappings are
-        made resident), or None."""
+        made resident), or None. packing: enum plamo_metal_packing (1, raw: no
+        fp16 fragments for prompts)."""
         lib = load()
         self.lib = lib
         cfg = MetalConfig()
         cfg.memory = memory
+        cfg.packing = packing
         self._maps = None
         if synthetic is not None:
             maps = synthetic.mappings

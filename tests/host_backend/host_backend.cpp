@@ -177,7 +177,8 @@ struct Request {
     plamo_synthetic_instance *inst;
     struct model *model;
     plamo_metal *metal;
-    Request(uint64_t layers, uint64_t window, uint64_t pattern, bool pinned) {
+    Request(uint64_t layers, uint64_t window, uint64_t pattern, bool pinned,
+            plamo_metal_packing packing = PLAMO_PACK_AUTO) {
         plamo_synthetic_config cfg;
         char err[256] = "";
         plamo_synthetic_defaults(&cfg, 64, layers, 4, 2, 16, 96, 40);
@@ -190,6 +191,7 @@ struct Request {
         const plamo_mapping *map = syn ? plamo_synthetic_weights(syn) : nullptr;
         config.maps = map;
         config.count = 1;
+        config.packing = packing;
         metal = inst ? plamo_metal_open(&config, err, sizeof err) : nullptr;
         check(metal, err);
         model = plamo_synthetic_model(inst);
@@ -299,7 +301,7 @@ void lone_window(uint64_t layer) {
 
 // Device memory that holds the weights twice, but not the rows of a longer
 // context beside both: the fragments make room, in a prompt, in a decode step
-// and for weights preloaded later.
+// and for weights preloaded later. A caller who asks for raw weights has none.
 void fragments_make_room() {
     for (int turn = 0; turn < 3; ++turn) {
         host::device_limit = 96 << 20;
@@ -330,6 +332,11 @@ void fragments_make_room() {
         check(plamo_metal_prefill(q.metal, q.model, ids.data(), 7, nullptr) == 1, "next prompt");
     }
     host::device_limit = ~(size_t)0;
+    Request raw(3, 400, 3, true, PLAMO_PACK_RAW);
+    std::vector<uint32_t> ids(20, 1);
+    check(plamo_metal_prepare_model(raw.metal, raw.model) == 1, "prepare, raw");
+    check(plamo_metal_prefill(raw.metal, raw.model, ids.data(), 20, nullptr) == 1, "prompt, raw");
+    check(!raw.metal->pair_ready && !raw.metal->pair_block, "raw weights alone");
 }
 
 }  // namespace

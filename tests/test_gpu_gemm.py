@@ -352,18 +352,20 @@ def test_prompt_activation_columns(gate, up, exponent, ignored, tokens):
 
 
 # Prompts of models whose shapes the fp16 fragments do not cover (an attention
-# width that is not whole 32 columns), on the BF16 weights: the norms write the
+# width that is not whole 32 columns), or of callers who asked for raw weights,
+# on the BF16 weights: the norms write the
 # split GEMM's planes, and gate/up writes down's where the intermediate size is
 # whole half tiles; skinny batches, whole and ragged tiles, both tile widths.
 @pytest.mark.parametrize("inter", [128, 192, 100, 8256])
 @pytest.mark.parametrize("tokens", [3, 16, 17, 64, 65, 140])
-def test_prompt_without_fragments(inter, tokens):
-    say(f"without fragments inter={inter} tokens={tokens}")
+@pytest.mark.parametrize("dim,packing", [(20, 0), (64, 1)])
+def test_prompt_without_fragments(inter, tokens, dim, packing):
+    say(f"without fragments inter={inter} tokens={tokens} dim={dim} packing={packing}")
     hidden = 256
-    syn = plamo_hip.Synthetic(hidden, 3, 3, 3, 20, inter, 200, window=1024, global_capacity=1024,
+    syn = plamo_hip.Synthetic(hidden, 3, 3, 3, dim, inter, 200, window=1024, global_capacity=1024,
                               pattern=2, embedding_std=1.0, seed=tokens)
     gpu, cpu = syn.instance(), syn.instance()
-    be = plamo_hip.Backend(syn)
+    be = plamo_hip.Backend(syn, packing=packing)
     try:
         for states in (True, False):
             ids = [(7 * j + 3) % 200 for j in range(tokens)]

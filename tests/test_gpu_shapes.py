@@ -544,10 +544,11 @@ def test_edited_full_windows(pinned):
 # groups both take.
 @pytest.mark.parametrize("qh,kh,dim", [(3, 1, 128), (6, 2, 64), (5, 1, 64), (14, 2, 128),
                                        (64, 16, 128), (60, 10, 128)])
-@pytest.mark.parametrize("prefix,tokens", [(0, 33), (9, 90), (12, 300)])
-def test_prompt_last_row(qh, kh, dim, prefix, tokens):
-    say(f"last row {qh}/{kh}x{dim} prefix={prefix} tokens={tokens}")
-    syn = plamo_hip.Synthetic(256, 2, qh, kh, dim, 96, 300, window=2304, global_capacity=2304,
+@pytest.mark.parametrize("prefix,tokens,window", [(0, 33, 2304), (9, 90, 2304), (12, 300, 2304),
+                                                  (9, 90, 40)])
+def test_prompt_last_row(qh, kh, dim, prefix, tokens, window):
+    say(f"last row {qh}/{kh}x{dim} prefix={prefix} tokens={tokens} window={window}")
+    syn = plamo_hip.Synthetic(256, 3, qh, kh, dim, 96, 300, window=window, global_capacity=2304,
                               pattern=2, embedding_std=1.0, seed=5)
     gpu, cpu = syn.instance(), syn.instance()
     be = plamo_hip.Backend(syn)
