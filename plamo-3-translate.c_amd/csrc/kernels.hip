@@ -1386,7 +1386,7 @@ __global__ __launch_bounds__(64 * GM * GN, (WN > 2 || GM * GN > 4) ? 1 : 2) void
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
-            for (int j = 0; j < WN; j += 2) {
+            for (int j = 0; j + 1 < WN; j += 2) {
                 const uint32_t col = bn * (BN / 2) + wn * 16 * WN + j / 2 * 32 + (lane & 31);
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
@@ -4572,7 +4572,7 @@ constexpr int kMixedTile = 1024;  // added to the exponent of a tile whose V row
 
 struct PairAttention {
     PromptAttention a;
-    uint16_t *kv;    // [kh][tiles][K fragments | V fragments]
+    uint16_t *kv;      // [kh][tiles][K fragments | V fragments]
     int32_t *kv_exps;  // [kh][tiles][K, V]; V's of the largest row, + kMixedTile
     int32_t *v_exps;   // [kh][tiles][key], of mixed tiles
     uint32_t tiles;
